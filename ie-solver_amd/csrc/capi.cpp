@@ -2256,7 +2256,7 @@ int iegpu_evaluate(iegpu_ctx* c, int n_targets, const double* targets,
       c->e_alpha.upload(alpha, c->hole_dim, st);
       dalpha = c->e_alpha.p;
     }
-    c->e_partial.alloc((size_t)eval_chunks(c->n_points) * sd * n_targets);
+    c->e_partial.alloc((size_t)eval_chunks(c->n_points, sd, n_targets) * sd * n_targets);
     c->e_out.alloc((size_t)sd * n_targets);
     launch_eval(c->geom(), n_targets, c->e_tg.p, dmask, c->e_mu.p,
                 holes ? c->n_holes : 0, c->d_hole_c.p, dalpha, c->e_partial.p,

@@ -7,12 +7,13 @@
 //                   boundary, kernel.cpp:29-63 with tgt.is_boundary = false).
 // Targets outside the domain give 0 (initialization.cpp:43-49).
 //
-// Grid: (target blocks of 256) x (source chunks); each thread accumulates
-// one target over a source chunk staged in LDS, then a second kernel sums
-// the chunks in a fixed order and adds the hole terms.
+// Grid: (blocks of kTargets targets) x (source chunks); k_eval_partial
+// forms the sums of one chunk, k_eval_finish adds the chunks in a fixed
+// order with the hole terms.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 
@@ -29,61 +30,109 @@ static __device__ __align__(256) double scratch[kEvalScratchElems];
 
 namespace {
 
-constexpr int kTile = 256;
+// k_eval_partial: 8 waves share kTargets = 128 targets, two per lane; wave
+// w takes sources 64 w .. 64 w + 63 of every staged tile of kTile, and the
+// eight waves' sums are added in wave order.  FP64 issue bounds it: a
+// Laplace pair costs ten FP64 instructions and one reciprocal (v_rcp_f64
+// with one Newton step, within two ulp; a full division alone costs as much
+// again), and two targets per lane share each source's LDS reads, which
+// one per lane would make the bound (two b128 broadcasts per pair and
+// wave).  10,000 targets x 65,536 Laplace sources: 954 us with one target
+// per thread, divisions and 320 workgroups of four waves; 353 us.
+constexpr int kTargets = 128, kTile = 512;
+// Targets past this magnitude (and NaN) take the division: |r|^2 would
+// overflow, and the Newton step turns the reciprocal's 0 into NaN.
+constexpr double kFarTarget = 1e150;
 
-__global__ __launch_bounds__(kTile) void k_eval_partial(DevGeom g, int nt,
-                                                        const double* tg,
-                                                        const double* mu,
-                                                        int64_t chunk,
+// One source's contribution at the target p, added to a: xy the point; ab
+// -w mu n / (2 pi) (Laplace), (w mu / (4 pi), 0) (Neumann) or w n / pi
+// (Stokes); m the Stokes density.  FAST: reciprocal by v_rcp_f64 and a
+// Newton step, else the IEEE division.
+template <int PDE, bool FAST>
+__device__ inline void eval_pair(double2 p, double2 xy, double2 ab, double2 m, double2& a) {
+  const double r0 = p.x - xy.x, r1 = p.y - xy.y;
+  const double d2 = fma(r0, r0, r1 * r1);
+  if constexpr (PDE == kPdeLaplaceNeumann) {
+    a.x = fma(ab.x, log(d2), a.x);  // single layer w (1/2 pi) log|r| (kernel.cpp:95-102)
+  } else {
+    const double inv = FAST ? recip(d2) : 1.0 / d2;
+    const double rn = fma(r0, ab.x, r1 * ab.y);
+    if constexpr (PDE == kPdeStokes) {
+      const double pot = rn * inv * inv * fma(r0, m.x, r1 * m.y);
+      a.x = fma(pot, r0, a.x);
+      a.y = fma(pot, r1, a.y);
+    } else {
+      a.x = fma(rn, inv, a.x);
+    }
+  }
+}
+
+template <int PDE>
+__global__ __launch_bounds__(kTile) void k_eval_partial(DevGeom g, int nt, const double* tg,
+                                                        const double* mu, int64_t chunk,
                                                         double* partial) {
-  __shared__ double sx[kTile], sy[kTile], snx[kTile], sny[kTile], sw[kTile],
-      sm0[kTile], sm1[kTile];
-  const int t = blockIdx.x * kTile + threadIdx.x;
-  const int sd = g.sol_dim;
-  const double x0 = t < nt ? tg[2 * t] : 0, x1 = t < nt ? tg[2 * t + 1] : 0;
+  constexpr bool stokes = PDE == kPdeStokes;
+  constexpr int NW = kTile / 64, SD = stokes ? 2 : 1;
+  __shared__ double2 sxy[kTile], sab[kTile], sm[stokes ? kTile : 1];
+  __shared__ double red[NW][kTargets][SD];
+  const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
+  const int t0 = blockIdx.x * kTargets + lane;
   const int64_t lo = blockIdx.y * chunk;
   const int64_t hi = lo + chunk < g.n_points ? lo + chunk : g.n_points;
-  double a0 = 0, a1 = 0;
+  double2 p[2], acc[2];
+  bool far = false;
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int t = min(t0 + 64 * u, nt - 1);
+    p[u] = make_double2(tg[2 * (int64_t)t], tg[2 * (int64_t)t + 1]);
+    acc[u] = make_double2(0, 0);
+    far = far || !(fabs(p[u].x) < kFarTarget && fabs(p[u].y) < kFarTarget);
+  }
+  far = __any(far);  // the same in every wave: all hold the same targets
   for (int64_t base = lo; base < hi; base += kTile) {
-    const int64_t j = base + threadIdx.x;
+    const int64_t j = base + tid;
     if (j < hi) {
-      sx[threadIdx.x] = g.pts[2 * j];
-      sy[threadIdx.x] = g.pts[2 * j + 1];
-      snx[threadIdx.x] = g.nrm[2 * j];
-      sny[threadIdx.x] = g.nrm[2 * j + 1];
-      sw[threadIdx.x] = g.wts[j];
-      sm0[threadIdx.x] = mu[sd * j];
-      sm1[threadIdx.x] = sd == 2 ? mu[2 * j + 1] : 0.0;
+      sxy[tid] = make_double2(g.pts[2 * j], g.pts[2 * j + 1]);
+      const double n0 = g.nrm[2 * j], n1 = g.nrm[2 * j + 1], w = g.wts[j];
+      if constexpr (stokes) {
+        sab[tid] = make_double2(w * (1.0 / M_PI) * n0, w * (1.0 / M_PI) * n1);
+        sm[tid] = make_double2(mu[2 * j], mu[2 * j + 1]);
+      } else if constexpr (PDE == kPdeLaplaceNeumann) {
+        sab[tid] = make_double2(w * (0.25 / M_PI) * mu[j], 0);
+      } else {
+        const double c = -w * (0.5 / M_PI) * mu[j];
+        sab[tid] = make_double2(c * n0, c * n1);
+      }
     }
     __syncthreads();
-    const int cnt = (int)((hi - base) < kTile ? (hi - base) : kTile);
-    if (g.pde == kPdeStokes) {
-      for (int q = 0; q < cnt; q++) {
-        const double r0 = x0 - sx[q], r1 = x1 - sy[q];
-        const double d2 = r0 * r0 + r1 * r1;
-        const double pot = sw[q] * (1.0 / M_PI) * (r0 * snx[q] + r1 * sny[q]) / (d2 * d2);
-        const double proj = r0 * sm0[q] + r1 * sm1[q];
-        a0 += pot * r0 * proj;
-        a1 += pot * r1 * proj;
-      }
-    } else if (g.pde == kPdeLaplaceNeumann) {
-      // single layer w (1/2 pi) log|r| (kernel.cpp:95-102)
-      for (int q = 0; q < cnt; q++) {
-        const double r0 = x0 - sx[q], r1 = x1 - sy[q];
-        a0 += sw[q] * (1.0 / (2 * M_PI)) * log(sqrt(r0 * r0 + r1 * r1)) * sm0[q];
-      }
+    const int q0 = 64 * wv, q1 = min((int64_t)q0 + 64, hi - base);
+    if (!far) {
+#pragma unroll 4
+      for (int q = q0; q < q1; q++)
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+          eval_pair<PDE, true>(p[u], sxy[q], sab[q], sm[stokes ? q : 0], acc[u]);
     } else {
-      for (int q = 0; q < cnt; q++) {
-        const double r0 = x0 - sx[q], r1 = x1 - sy[q];
-        a0 += -sw[q] * (1.0 / (2 * M_PI)) * (r0 * snx[q] + r1 * sny[q]) /
-              (r0 * r0 + r1 * r1) * sm0[q];
-      }
+      for (int q = q0; q < q1; q++)
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+          eval_pair<PDE, false>(p[u], sxy[q], sab[q], sm[stokes ? q : 0], acc[u]);
     }
     __syncthreads();
   }
-  if (t < nt) {
-    partial[(int64_t)blockIdx.y * sd * nt + (int64_t)sd * t] = a0;
-    if (sd == 2) partial[(int64_t)blockIdx.y * sd * nt + (int64_t)sd * t + 1] = a1;
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    red[wv][lane + 64 * u][0] = acc[u].x;
+    if constexpr (stokes) red[wv][lane + 64 * u][SD - 1] = acc[u].y;
+  }
+  __syncthreads();
+  for (int i = tid; i < kTargets * SD; i += kTile) {
+    const int t = blockIdx.x * kTargets + i / SD;
+    if (t >= nt) continue;
+    double v = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) v += red[w][i / SD][i % SD];
+    partial[((int64_t)blockIdx.y * nt + t) * SD + i % SD] = v;
   }
 }
 
@@ -144,12 +193,21 @@ int eval_scratch_address(int device, double** ptr) {
 }
 
 int64_t eval_scratch_need(int64_t n_points, int sol_dim, int64_t n_targets) {
-  return (int64_t)eval_chunks(n_points) * sol_dim * n_targets;
+  return (int64_t)eval_chunks(n_points, sol_dim, n_targets) * sol_dim * n_targets;
 }
 
-int eval_chunks(int64_t n_points) {
-  int64_t c = (n_points + 8191) / 8192;
-  return (int)(c < 1 ? 1 : (c > 64 ? 64 : c));
+// At least one chunk per 8192 sources (64 at most), and more where the
+// target blocks alone leave the chip idle: enough for 1024 workgroups (four
+// per CU; a host call with 65,536 sources takes 127 us at 100 targets and
+// 124 at 1,000, against 222 and 194 with 8 chunks, 407 against 417 at
+// 10,000), while a chunk keeps a tile of sources and the partial sums stay
+// within the static scratch of the allocation-free call.
+int eval_chunks(int64_t n_points, int sol_dim, int64_t n_targets) {
+  const int64_t c = std::min<int64_t>(std::max<int64_t>((n_points + 8191) / 8192, 1), 64);
+  const int64_t blocks = std::max<int64_t>((n_targets + kTargets - 1) / kTargets, 1);
+  const int64_t fill = std::min((1024 + blocks - 1) / blocks, (n_points + kTile - 1) / kTile);
+  const int64_t room = kEvalScratchElems / (sol_dim * std::max<int64_t>(n_targets, 1));
+  return (int)std::max(c, std::min(fill, room));
 }
 
 void launch_eval(const DevGeom& g, int nt, const double* tg, const int* in_domain,
@@ -157,10 +215,15 @@ void launch_eval(const DevGeom& g, int nt, const double* tg, const int* in_domai
                  const double* alpha, double* partial, double* out,
                  hipStream_t st) {
   if (nt <= 0) return;
-  const int nc = eval_chunks(g.n_points);
+  const int nc = eval_chunks(g.n_points, g.sol_dim, nt);
   const int64_t chunk = (g.n_points + nc - 1) / nc;
-  dim3 grid((nt + kTile - 1) / kTile, nc);
-  k_eval_partial<<<grid, kTile, 0, st>>>(g, nt, tg, mu, chunk, partial);
+  const dim3 grid((nt + kTargets - 1) / kTargets, nc);
+  if (g.pde == kPdeStokes)
+    k_eval_partial<kPdeStokes><<<grid, kTile, 0, st>>>(g, nt, tg, mu, chunk, partial);
+  else if (g.pde == kPdeLaplaceNeumann)
+    k_eval_partial<kPdeLaplaceNeumann><<<grid, kTile, 0, st>>>(g, nt, tg, mu, chunk, partial);
+  else
+    k_eval_partial<kPdeLaplace><<<grid, kTile, 0, st>>>(g, nt, tg, mu, chunk, partial);
   k_eval_finish<<<(nt + 255) / 256, 256, 0, st>>>(g, nt, tg, in_domain, partial, nc,
                                                   n_holes, hole_centers, alpha, out);
 }

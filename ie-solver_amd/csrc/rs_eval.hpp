@@ -10,7 +10,7 @@
 namespace iegpu {
 
 // Number of source chunks the partial sums are split into.
-int eval_chunks(int64_t n_points);
+int eval_chunks(int64_t n_points, int sol_dim, int64_t n_targets);
 
 // The allocation-free evaluation keeps its partial sums in a static device
 // array of kEvalScratchElems doubles (4 MiB) per GPU.
@@ -24,7 +24,7 @@ int64_t eval_scratch_need(int64_t n_points, int sol_dim, int64_t n_targets);
 int eval_scratch_address(int device, double** ptr);
 
 // out (sol_dim per target) = K_domain mu + U_forward alpha; partial holds
-// eval_chunks(n_points) * sol_dim * nt doubles.
+// eval_chunks(n_points, sol_dim, nt) * sol_dim * nt doubles.
 void launch_eval(const DevGeom& g, int nt, const double* targets,
                  const int* in_domain, const double* mu, int n_holes,
                  const double* hole_centers, const double* alpha,

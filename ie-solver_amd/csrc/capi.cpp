@@ -15,6 +15,7 @@
 #include "rs_holes.hpp"
 #include "rs_eval.hpp"
 #include "rs_fmm.hpp"
+#include "rs_inv.hpp"
 #include "rs_kernels.hpp"
 #include "rs_matvec.hpp"
 #include "rs_mlp.hpp"
@@ -25,6 +26,7 @@ using namespace iegpu;
 static_assert(IEGPU_RANK_FEATURES == kFeat && IEGPU_RANK_MODEL_LEN == kMlpLen &&
                   IEGPU_RANK_PARAMS == kMlpParams,
               "rank model layout of iegpu.h");
+static_assert(kRootPiv == kInvFlags, "panel flags behind a root's pivot rows");
 static_assert(IEGPU_NUM_LAUNCH_CAPS == kNumCaps, "launch caps of iegpu.h");
 
 namespace {
@@ -214,9 +216,9 @@ struct iegpu_ctx {
   int n_holes = 0;
   int hole_dim = 0;
   std::vector<double> h_hole_c, h_hole_r;
-  DevBuf<double> d_U, d_PsiT;  // ndof x hole_dim each
-  DevBuf<double> d_mU, d_mPsiT, d_DinvC, d_gram, d_partial, d_Smat, d_tail,
-      d_ybuf, d_alpha;
+  DevBuf<double> d_U, d_PsiT;  // row-major ndof x hole_dim each
+  DevBuf<double> d_mU, d_mPsiT, d_DinvC, d_gram, d_partial, d_Smat,
+      d_Sinv, d_ybuf, d_alpha;
   DevBuf<int> d_Spiv, d_mask;
   DevBuf<double> d_hole_c;  // hole centres (2 per hole)
   // interior evaluation buffers
@@ -257,6 +259,7 @@ struct iegpu_ctx {
   int rid_margin = 0;
   DevBuf<float> d_model, d_feat, m_X, m_y, m_work;
   DevBuf<double> d_work;  // solve vector for host-pointer solves
+  DevBuf<double> d_cols;  // its column-major form with several columns
   // iterative refinement: b, x, residual / correction (ndof), border parts,
   // reduction partials
   DevBuf<double> r_b, r_x, r_r, r_a, r_ra, r_part;
@@ -429,7 +432,8 @@ int from_hip(iegpu_ctx* c, const HipError& e) {
   return fail(c, oom ? IEGPU_ERR_OOM : IEGPU_ERR_HIP, m);
 }
 
-// U / Psi^T on the boundary points: ie_solver/linear_solve.cpp:20-112.
+// U / Psi^T on the boundary points, row-major (ndof x hole_dim):
+// ie_solver/linear_solve.cpp:20-112.
 void build_border(iegpu_ctx* c, const double* centers, const double* radii,
                   std::vector<double>* U, std::vector<double>* PsiT) {
   const int np = c->n_points, h = c->n_holes;
@@ -450,12 +454,12 @@ void build_border(iegpu_ctx* c, const double* centers, const double* radii,
       const double x0 = c->h_pts[2 * i], x1 = c->h_pts[2 * i + 1];
       for (int k = 0; k < h; k++) {
         const double r0 = x0 - centers[2 * k], r1 = x1 - centers[2 * k + 1];
-        (*U)[i + nd * k] = std::log(std::sqrt(r0 * r0 + r1 * r1));
+        (*U)[i * (int64_t)h + k] = std::log(std::sqrt(r0 * r0 + r1 * r1));
       }
       for (int k = 0; k < h; k++) {
         const double r0 = x0 - centers[2 * k], r1 = x1 - centers[2 * k + 1];
         if (std::sqrt(r0 * r0 + r1 * r1) < radii[k] + 1e-8) {
-          (*PsiT)[i + nd * k] = c->h_wts[i];
+          (*PsiT)[i * (int64_t)h + k] = c->h_wts[i];
           break;
         }
       }
@@ -474,21 +478,21 @@ void build_border(iegpu_ctx* c, const double* centers, const double* radii,
       const double r0 = x0 - centers[2 * k], r1 = x1 - centers[2 * k + 1];
       const double rn = std::sqrt(r0 * r0 + r1 * r1);
       const double rn2 = rn * rn;
-      (*U)[r0i + nd * (3 * k)] = scale * (std::log(1 / rn) + (1.0 / rn2) * r0 * r0);
-      (*U)[r1i + nd * (3 * k)] = scale * ((1.0 / rn2) * r1 * r0);
-      (*U)[r0i + nd * (3 * k + 1)] = scale * ((1.0 / rn2) * r0 * r1);
-      (*U)[r1i + nd * (3 * k + 1)] = scale * (std::log(1 / rn) + (1.0 / rn2) * r1 * r1);
-      (*U)[r0i + nd * (3 * k + 2)] = r1 * (scale / rn2);
-      (*U)[r1i + nd * (3 * k + 2)] = -r0 * (scale / rn2);
+      (*U)[r0i * hd + 3 * k] = scale * (std::log(1 / rn) + (1.0 / rn2) * r0 * r0);
+      (*U)[r1i * hd + 3 * k] = scale * ((1.0 / rn2) * r1 * r0);
+      (*U)[r0i * hd + 3 * k + 1] = scale * ((1.0 / rn2) * r0 * r1);
+      (*U)[r1i * hd + 3 * k + 1] = scale * (std::log(1 / rn) + (1.0 / rn2) * r1 * r1);
+      (*U)[r0i * hd + 3 * k + 2] = r1 * (scale / rn2);
+      (*U)[r1i * hd + 3 * k + 2] = -r0 * (scale / rn2);
     }
     for (int k = 0; k < h; k++) {
       const double r0 = x0 - centers[2 * k], r1 = x1 - centers[2 * k + 1];
       if (std::sqrt(r0 * r0 + r1 * r1) < radii[k] + 1e-8) {
         const double w = c->h_wts[i];
-        (*PsiT)[r0i + nd * (3 * k)] = w;
-        (*PsiT)[r1i + nd * (3 * k + 1)] = w;
-        (*PsiT)[r0i + nd * (3 * k + 2)] = w * x1;
-        (*PsiT)[r1i + nd * (3 * k + 2)] = -w * x0;
+        (*PsiT)[r0i * hd + 3 * k] = w;
+        (*PsiT)[r1i * hd + 3 * k + 1] = w;
+        (*PsiT)[r0i * hd + 3 * k + 2] = w * x1;
+        (*PsiT)[r1i * hd + 3 * k + 2] = -w * x0;
         break;
       }
     }
@@ -552,7 +556,7 @@ void alloc_state(iegpu_ctx* c) {
   c->s_fac_top.alloc(1);
   c->s_err.alloc(4);
   const size_t nr = c->tree.n_roots;
-  c->s_root_piv.alloc(nr * (c->ncap + 64));
+  c->s_root_piv.alloc(nr * (c->ncap + kRootPiv));
   c->s_root_mat.alloc(nr * 2 * c->ncap * c->ncap * 8);  // matrix + inverse per root
   c->s_id_pool.alloc((size_t)2 * c->id_cap * c->elem());  // odd and even levels
   c->s_row_pool.alloc((size_t)c->row_cap);
@@ -580,7 +584,7 @@ void enqueue_factor(iegpu_ctx* c, double tol, const double* fb = nullptr,
   DevState s = c->dstate();
   hipStream_t st = c->stream;
   const HostTree& T = c->tree;
-  const SolveVec fv{fx, (int64_t)c->ndof(), 1};
+  const SolveVec fv{fx, 1, c->ndof(), 1};
   if (fx && fb != fx) launch_copy(fx, fb, c->ndof(), st);
   const bool split = c->overlap && !c->prof.on && c->stream2 != nullptr;
   hipStream_t st2 = split ? c->stream2 : st;
@@ -667,38 +671,32 @@ void enqueue_border_factor(iegpu_ctx* c) {
   c->prof.run(kProfBorder, 0, st, [&] {
     launch_copy(c->d_mU.p, c->d_U.p, nd * h, st);
     launch_copy(c->d_mPsiT.p, c->d_PsiT.p, nd * h, st);
-    SolveVec vu{c->d_mU.p, nd, h};
-    SolveVec vp{c->d_mPsiT.p, nd, h};
+    SolveVec vu{c->d_mU.p, h, 1, h};
+    SolveVec vp{c->d_mPsiT.p, h, 1, h};
     for (int lv = T.n_levels - 1; lv >= 1; lv--) {
       const int start = T.level_start[lv];
       const int count = T.level_start[lv + 1] - start;
-      launch_sweep_up<R>(s, start, count, vu, false, false, st);
+      launch_sweep_up<R>(s, start, count, vu, false, true, st, c->d_DinvC.p);
       launch_sweep_up<R>(s, start, count, vp, true, false, st);
-    }
-    launch_copy(c->d_DinvC.p, c->d_mU.p, nd * h, st);
-    SolveVec vd{c->d_DinvC.p, nd, h};
-    for (int lv = T.n_levels - 1; lv >= 1; lv--) {
-      const int start = T.level_start[lv];
-      const int count = T.level_start[lv + 1] - start;
-      launch_diag<R>(s, start, count, vd, st);
     }
     launch_mark_skel(s, c->d_mask.p, nd, st);
     launch_border_gram(c->d_mPsiT.p, c->d_DinvC.p, c->d_mask.p, nd, h,
                        c->d_partial.p, c->d_gram.p, st);
-    launch_border_factor<R>(s, c->d_mU.p, c->d_mPsiT.p, c->d_gram.p, nd, h,
-                            c->d_Smat.p, c->d_Spiv.p, st);
+    launch_border_factor<R>(s, c->d_mU.p, c->d_mPsiT.p, c->d_gram.p, h, c->d_Smat.p,
+                            c->d_Sinv.p, c->d_Spiv.p, st);
   });
 }
 
 // x (ndof) <- M^{-1} x in place; with holes alpha (hole_dim) is written and
 // g (hole_dim, device, may be NULL = 0) is the border right-hand side.
+// Several right-hand sides (nrhs > 1, no holes) are row-major.
 template <typename R>
 void enqueue_solve(iegpu_ctx* c, double* x, double* alpha, hipStream_t st,
                    const double* g = nullptr, int nrhs = 1) {
   DevState s = c->dstate();
   const HostTree& T = c->tree;
   const int64_t nd = c->ndof();
-  SolveVec v{x, nd, nrhs};
+  SolveVec v{x, nrhs, 1, nrhs};
   const bool holes = c->hole_dim > 0;
   for (int lv = T.n_levels - 1; lv >= 1; lv--) {
     const int start = T.level_start[lv];
@@ -711,10 +709,8 @@ void enqueue_solve(iegpu_ctx* c, double* x, double* alpha, hipStream_t st,
       launch_root_solve<R>(s, T.n_roots, v, st);
     } else {
       const int h = c->hole_dim;
-      launch_border_gemv(c->d_mPsiT.p, x, c->d_mask.p, nd, h, c->d_partial.p,
-                         c->d_tail.p, -1.0, st);
-      launch_border_solve(s, c->d_Smat.p, c->d_Spiv.p, h, x, c->d_tail.p, g,
-                          alpha, c->d_ybuf.p, st);
+      launch_border_solve(s, c->d_mPsiT.p, c->d_Sinv.p, c->d_mask.p, nd, h, x, g, alpha,
+                          c->d_partial.p, c->d_ybuf.p, st);
       launch_red_update(x, c->d_DinvC.p, c->d_mask.p, alpha, nd, h, st);
     }
   });
@@ -1189,8 +1185,7 @@ void upload_border(iegpu_ctx* c) {
     c->d_mPsiT.alloc(nd * h);
     c->d_DinvC.alloc(nd * h);
     c->d_gram.alloc((size_t)h * h);
-    c->d_partial.alloc((size_t)border_partial_blocks(nd) * h * h);
-    c->d_tail.alloc(h);
+    c->d_partial.alloc((size_t)border_partials(nd, h));
     c->d_alpha.alloc(h);
     c->d_mask.alloc(nd);
     c->d_hole_c.upload(centers, 2 * (size_t)n_holes, st);
@@ -1553,7 +1548,8 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
       if (c->hole_dim > 0) {
         const int ns_max = c->ncap + c->hole_dim;
         c->d_Smat.alloc((size_t)ns_max * ns_max);
-        c->d_Spiv.alloc(ns_max);
+        c->d_Sinv.alloc((size_t)ns_max * ns_max);
+        c->d_Spiv.alloc(ns_max + kInvFlags);
         c->d_ybuf.alloc(ns_max);
       }
       if (c->inc_run)  // new slots go past the kept ones (a failed attempt moved the top)
@@ -1690,6 +1686,10 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
     c->fac_bytes = (double)top * c->elem();
     c->kept_top = top;
     if (!c->last_incremental) c->full_top = top;
+    if (errbits & kErrWait) {
+      c->factored = false;
+      return fail(c, IEGPU_ERR_HIP, "a wait between workgroups did not end");
+    }
     if (errbits & kErrSingular) {
       c->factored = false;
       return fail(c, IEGPU_ERR_SINGULAR, "exact zero pivot in an LU factorization");
@@ -1796,15 +1796,24 @@ int iegpu_solve_nrhs(iegpu_ctx* c, int nrhs, const double* b, double* mu, double
                                hipMemcpyDeviceToHost, st));
       }
     } else {
-      // every column through each sweep kernel in one pass
+      // every column through each sweep kernel in one pass, row-major there
+      // (a DOF's columns share its cache lines)
+      double* cols = nullptr;
       c->d_work.alloc(nd * nrhs);
-      HIP_TRY(hipMemcpyAsync(c->d_work.p, b, nd * nrhs * sizeof(double), hipMemcpyHostToDevice,
-                             st));
-      if (c->precision == IEGPU_FP32) enqueue_solve<float>(c, c->d_work.p, nullptr, st, nullptr, nrhs);
-      else enqueue_solve<double>(c, c->d_work.p, nullptr, st, nullptr, nrhs);
+      double* rows = c->d_work.p;
+      if (nrhs > 1) {
+        c->d_cols.alloc(nd * nrhs);
+        cols = c->d_cols.p;
+      } else {
+        cols = rows;
+      }
+      HIP_TRY(hipMemcpyAsync(cols, b, nd * nrhs * sizeof(double), hipMemcpyHostToDevice, st));
+      if (nrhs > 1) launch_transpose(rows, cols, nd, nrhs, true, st);
+      if (c->precision == IEGPU_FP32) enqueue_solve<float>(c, rows, nullptr, st, nullptr, nrhs);
+      else enqueue_solve<double>(c, rows, nullptr, st, nullptr, nrhs);
+      if (nrhs > 1) launch_transpose(cols, rows, nd, nrhs, false, st);
       HIP_TRY(hipGetLastError());
-      HIP_TRY(hipMemcpyAsync(mu, c->d_work.p, nd * nrhs * sizeof(double), hipMemcpyDeviceToHost,
-                             st));
+      HIP_TRY(hipMemcpyAsync(mu, cols, nd * nrhs * sizeof(double), hipMemcpyDeviceToHost, st));
     }
     HIP_TRY(hipStreamSynchronize(st));
   } catch (const HipError& e) {
@@ -1828,11 +1837,11 @@ int iegpu_set_border(iegpu_ctx* c, int hole_dim, const double* U, const double* 
       return fail(c, IEGPU_ERR_INVALID, "non-finite border entry");
   try {
     HIP_TRY(hipSetDevice(c->device));
-    std::vector<double> PsiT(nd * h);
-    for (int k = 0; k < h; k++)  // Psi is h x ndof column-major
-      for (int64_t i = 0; i < nd; i++) PsiT[i + nd * k] = Psi[k + (int64_t)h * i];
-    c->d_U.upload(U, nd * h, c->stream);
-    c->d_PsiT.upload(PsiT, c->stream);
+    std::vector<double> Ur(nd * h);  // row-major; Psi (h x ndof column-major) already is
+    for (int k = 0; k < h; k++)
+      for (int64_t i = 0; i < nd; i++) Ur[k + (int64_t)h * i] = U[i + nd * k];
+    c->d_U.upload(Ur, c->stream);
+    c->d_PsiT.upload(Psi, nd * h, c->stream);
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->factored = false;
   } catch (const HipError& e) {
@@ -2155,8 +2164,8 @@ int iegpu_solve_refined(iegpu_ctx* c, const double* b, double* x, double* alpha,
       // r = b - A x  (A bordered by [U; Psi, -I] with holes)
       enqueue_matvec(c, c->r_x.p, c->r_r.p, st);
       if (h > 0)
-        launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->r_r.p,
-                            c->r_ra.p, st);
+        launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->d_partial.p,
+                            c->r_r.p, c->r_ra.p, st);
       launch_residual(c->r_b.p, c->r_r.p, nd, c->r_part.p, st);
       HIP_TRY(hipMemcpyAsync(part.data(), c->r_part.p, sizeof(double) * 2 * nres,
                              hipMemcpyDeviceToHost, st));
@@ -2215,8 +2224,8 @@ int iegpu_apply(iegpu_ctx* c, const double* x, const double* alpha, double* y,
     if (h > 0 && alpha && z) {
       c->r_a.upload(alpha, h, st);
       c->r_ra.alloc(h);
-      launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->r_r.p,
-                          c->r_ra.p, st);
+      launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->d_partial.p,
+                          c->r_r.p, c->r_ra.p, st);
       HIP_TRY(hipMemcpyAsync(z, c->r_ra.p, sizeof(double) * h, hipMemcpyDeviceToHost, st));
     }
     HIP_TRY(hipGetLastError());

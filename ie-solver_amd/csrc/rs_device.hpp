@@ -25,6 +25,7 @@ enum : int {
   kErrRowPool = 16,    // row-index pool exhausted
   kErrDecPool = 32,    // decouple operand pool exhausted
   kErrPlan = 64,       // a list whose kernels the launch plan skipped was not empty
+  kErrWait = 128,      // a bounded wait between workgroups did not end
 };
 
 // Launch plan (DevState::plan_skip, per level): the ID-stage kernels not
@@ -53,8 +54,9 @@ constexpr int kMaxChunks = 8;
 constexpr int kMaxLevels = 64;  // tree depth bound (per-level job counters)
 constexpr int kSmallBox = 64;     // decouple with every operand in LDS
 constexpr int kSmallBox1 = 44;    // smaller LDS class of that decouple
-constexpr int kRootRegMax = 192;  // root blocks inverted in registers
-constexpr int kRootBlkMax = 512;  // root blocks inverted by the blocked kernel
+constexpr int kRootRegMax = 192;  // root blocks inverted by one workgroup, in registers
+constexpr int kRootBatch = 16;    // roots from which that form is used
+constexpr int kRootPiv = kMaxBoxDofs / 16 + 16;  // ints behind a root's pivot rows (panel flags)
 
 // Per-level lists of the boxes each QRCP kernel takes, built by prefix
 // sums (k_scan) so that a kernel's workgroups map onto exactly its boxes.
@@ -187,7 +189,7 @@ struct DevState {
   int* err;            // [0] error bits, [1] / [2] / [3] decouple / ID / row
                        // pool size a level needed on overflow (1024 elements)
   void* root_mat;      // per root: 2 ncap^2 elements (matrix + inverse)
-  int* root_piv;       // per root: ncap + 64
+  int* root_piv;       // per root: ncap pivot rows, kRootPiv panel flags
   // Kept for the compressed forward apply when requested (else null): X_rr
   // of every compressed box at its factor-slot offset, and each root's
   // block (ncap^2 elements per root), as formed before their inversion.
@@ -754,7 +756,7 @@ __device__ inline R* root_block(const DevState& s, int r) {
   return reinterpret_cast<R*>(s.root_mat) + 2 * (int64_t)s.ncap * s.ncap * r;
 }
 __device__ inline int* root_pivots(const DevState& s, int r) {
-  return s.root_piv + (int64_t)(s.ncap + 64) * r;
+  return s.root_piv + (int64_t)(s.ncap + kRootPiv) * r;
 }
 
 }  // namespace iegpu

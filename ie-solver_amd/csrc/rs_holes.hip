@@ -14,6 +14,7 @@
 
 #include "rs_device.hpp"
 #include "rs_holes.hpp"
+#include "rs_inv.hpp"
 
 namespace iegpu {
 
@@ -36,200 +37,193 @@ __global__ void k_copy(double* dst, const double* src, int64_t n) {
     dst[i] = src[i];
 }
 
+// The border blocks are row-major (ndof x h): the h entries of a row are
+// one or two cache lines, read by neighbouring lanes.
+
 // partial[blk][a + h*c] = sum over redundant rows i of chunk blk of
-// P[i,a] * C[i,c]   (P, C: ndof x h, ld ndof).
-__global__ __launch_bounds__(256) void k_gram_partial(const double* P,
-                                                      const double* C,
-                                                      const int* mask,
-                                                      int64_t ndof, int h,
-                                                      int64_t chunk,
-                                                      double* partial) {
+// P[i,a] * C[i,c].  Rows are staged gram_rows(h) at a time in LDS, a thread
+// owning four of the h^2 sums per pass over the chunk (one pass up to
+// h = 32).  LDS reads bound it: 139 us at 262,144 DOFs and h = 24 (1,982 us
+// with the blocks column-major, each row's 2 h entries on 2 h lines).
+constexpr int kGramLds = 4096;  // doubles for each block's rows
+__device__ inline int gram_rows(int h) { return min(64, kGramLds / h); }
+
+__global__ __launch_bounds__(256) void k_gram_partial(const double* P, const double* C,
+                                                      const int* mask, int64_t ndof, int h,
+                                                      int64_t chunk, double* partial) {
+  __shared__ double sp[kGramLds], sc[kGramLds];
   const int64_t lo = blockIdx.x * chunk;
   const int64_t hi = lo + chunk < ndof ? lo + chunk : ndof;
-  for (int pc = threadIdx.x; pc < h * h; pc += blockDim.x) {
-    const int a = pc % h, c = pc / h;
-    double acc = 0;
-    for (int64_t i = lo; i < hi; i++)
-      if (!mask[i]) acc += P[i + ndof * a] * C[i + ndof * c];
-    partial[blockIdx.x * (int64_t)h * h + pc] = acc;
+  const int tr = gram_rows(h);
+  for (int e0 = 0; e0 < h * h; e0 += 1024) {
+    double acc[4] = {0, 0, 0, 0};
+    int ea[4], ec[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int e = min(e0 + (int)threadIdx.x + 256 * u, h * h - 1);
+      ea[u] = e % h;
+      ec[u] = e / h;
+    }
+    for (int64_t r0 = lo; r0 < hi; r0 += tr) {
+      const int rows = (int)min((int64_t)tr, hi - r0);
+      __syncthreads();
+      for (int i = threadIdx.x; i < rows * h; i += 256) {
+        sp[i] = mask[r0 + i / h] ? 0.0 : P[r0 * h + i];
+        sc[i] = C[r0 * h + i];
+      }
+      __syncthreads();
+      for (int i = 0; i < rows; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) acc[u] = fma(sp[i * h + ea[u]], sc[i * h + ec[u]], acc[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int e = e0 + threadIdx.x + 256 * u;
+      if (e < h * h) partial[blockIdx.x * (int64_t)h * h + e] = acc[u];
+    }
   }
 }
 
-// partial[blk][a] = sum over redundant rows i of P[i,a] * x[i].
-__global__ __launch_bounds__(64) void k_gemv_partial(const double* P,
-                                                     const double* x,
-                                                     const int* mask,
-                                                     int64_t ndof, int h,
-                                                     int64_t chunk,
-                                                     double* partial) {
+// partial[blk][a] = sum over the rows i of chunk blk (mask given: the
+// redundant ones) of P[i,a] * x[i]: 256 / h rows at a time, then the row
+// lanes added in order.  Reads 50 MB at 262,144 DOFs and h = 24: 22 us (656
+// us with 64 one-wave workgroups on column-major blocks).
+__global__ __launch_bounds__(256) void k_gemv_partial(const double* P, const double* x,
+                                                      const int* mask, int64_t ndof, int h,
+                                                      int64_t chunk, double* partial) {
+  __shared__ double red[256];
+  const int rl = 256 / h, a = threadIdx.x % h, rr = threadIdx.x / h;
   const int64_t lo = blockIdx.x * chunk;
   const int64_t hi = lo + chunk < ndof ? lo + chunk : ndof;
-  for (int a = threadIdx.x; a < h; a += blockDim.x) {
-    double acc = 0;
-    for (int64_t i = lo; i < hi; i++)
-      if (!mask[i]) acc += P[i + ndof * a] * x[i];
+  double acc = 0;
+  if (rr < rl)
+    for (int64_t i = lo + rr; i < hi; i += rl)
+      acc += (mask && mask[i]) ? 0.0 : P[i * h + a] * x[i];
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  if (threadIdx.x < h) {
+    for (int q = 1; q < rl; q++) acc += red[a + h * q];
     partial[blockIdx.x * (int64_t)h + a] = acc;
   }
 }
 
-// out[j] = sum_blk partial[blk][j] (fixed order: deterministic).
-__global__ void k_reduce_partials(const double* partial, int nblk, int len,
-                                  double* out, double sign) {
-  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < len;
-       j += gridDim.x * blockDim.x) {
-    double acc = 0;
-    for (int b = 0; b < nblk; b++) acc += partial[(int64_t)b * len + j];
-    out[j] = sign * acc;
-  }
-}
-
-template <typename R>
-__device__ int lu_inplace_1024(R* X, int n, int ld, int* ipiv) {
-  __shared__ int sh_p;
-  const int tid = threadIdx.x, lane = tid & 63;
-  constexpr int NT = 1024;
-  int info = 0;
-  for (int j = 0; j < n; j++) {
-    if (tid < 64) {
-      R best = -1;
-      int bi = n;
-      for (int i = j + lane; i < n; i += 64) {
-        const R v = fabs(X[i + (int64_t)ld * j]);
-        if (v > best) {
-          best = v;
-          bi = i;
-        }
-      }
-      for (int o = 32; o > 0; o >>= 1) {
-        const R ob = __shfl_xor(best, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        if (ob > best || (ob == best && oi < bi)) {
-          best = ob;
-          bi = oi;
-        }
-      }
-      if (bi >= n) bi = j;  // NaN column: no interchange
-      if (lane == 0) {
-        sh_p = bi;
-        ipiv[j] = bi;
-      }
-    }
-    __syncthreads();
-    const int p = sh_p;
-    if (p != j)
-      for (int c = tid; c < n; c += NT) {
-        const R t = X[j + (int64_t)ld * c];
-        X[j + (int64_t)ld * c] = X[p + (int64_t)ld * c];
-        X[p + (int64_t)ld * c] = t;
-      }
-    __syncthreads();
-    const R piv = X[j + (int64_t)ld * j];
-    if (piv != 0) {
-      const R inv = 1 / piv;
-      for (int i = j + 1 + tid; i < n; i += NT) X[i + (int64_t)ld * j] *= inv;
-    } else if (info == 0) {
-      info = j + 1;
-    }
-    __syncthreads();
-    const int len = n - j - 1;
-    for (int64_t idx = tid; idx < (int64_t)len * len; idx += NT) {
-      const int i = j + 1 + (int)(idx % len), c = j + 1 + (int)(idx / len);
-      X[i + (int64_t)ld * c] -= X[i + (int64_t)ld * j] * X[j + (int64_t)ld * c];
-    }
+// Sum over blocks of partial[blk][j], in every thread of a workgroup of 256
+// (fixed order: deterministic).
+__device__ inline double sum_partials(const double* partial, int nblk, int64_t len, int j,
+                                      double* red) {
+  double acc = 0;
+  for (int b = threadIdx.x; b < nblk; b += 256) acc += partial[b * len + j];
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
     __syncthreads();
   }
-  return info;
+  return red[0];
 }
 
-// Assemble S (ns + h square, ld ns + h) and factor it (one workgroup).
+// out[j] = sum_blk partial[blk][j] - sub[j] (sub may be null), j = workgroup.
+__global__ __launch_bounds__(256) void k_reduce_partials(const double* partial, int nblk, int len,
+                                                         double* out, const double* sub) {
+  __shared__ double red[256];
+  const int j = blockIdx.x;
+  const double v = sum_partials(partial, nblk, len, j, red);
+  if (threadIdx.x == 0) out[j] = v - (sub ? sub[j] : 0.0);
+}
+
+// S (ns + h square, column-major), and its inverse's panel flags cleared.
 template <typename R>
-__global__ __launch_bounds__(1024) void k_border_factor(DevState s,
-                                                        const double* mU,
-                                                        const double* mPsiT,
-                                                        const double* gram,
-                                                        int64_t ndof, int h,
-                                                        double* Smat,
-                                                        int* Spiv) {
+__global__ __launch_bounds__(256) void k_border_assemble(DevState s, const double* mU,
+                                                         const double* mPsiT, const double* gram,
+                                                         int h, double* Smat, int* flags) {
   const int ns = s.act_cnt[0];
   const int N = ns + h;
   const int* act = s.act_list;
   const R* A = reinterpret_cast<const R*>(s.root_mat);
-  for (int64_t idx = threadIdx.x; idx < (int64_t)N * N; idx += blockDim.x) {
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < kInvFlags; i += 256) flags[i] = 0;
+  for (int64_t idx = blockIdx.x * 256 + threadIdx.x; idx < (int64_t)N * N;
+       idx += gridDim.x * 256) {
     const int i = (int)(idx % N), j = (int)(idx / N);
     double v;
     if (i < ns && j < ns) v = (double)A[i + (int64_t)ns * j];
-    else if (i >= ns && j < ns) v = mPsiT[act[j] + ndof * (i - ns)];
-    else if (i < ns) v = mU[act[i] + ndof * (j - ns)];
+    else if (i >= ns && j < ns) v = mPsiT[(int64_t)act[j] * h + (i - ns)];
+    else if (i < ns) v = mU[(int64_t)act[i] * h + (j - ns)];
     else v = (i == j ? -1.0 : 0.0) - gram[(i - ns) + h * (j - ns)];
     Smat[idx] = v;
   }
-  __syncthreads();
-  const int info = lu_inplace_1024<double>(Smat, N, N, Spiv);
-  if (info != 0 && threadIdx.x == 0) atomicOr(s.err, kErrSingular);
 }
 
-// y = S^{-1} [x(skel); g + tail]; then x(skel) = y_head, alpha = y_tail.
-// g is the right-hand side of the border rows (NULL: zero, as in the
-// reference's [f; 0]).
-__global__ __launch_bounds__(64) void k_border_solve(DevState s,
-                                                     const double* Smat,
-                                                     const int* Spiv, int h,
-                                                     double* x,
-                                                     const double* tail,
-                                                     const double* g,
-                                                     double* alpha,
-                                                     double* ybuf) {
-  const int lane = threadIdx.x;
-  const int ns = s.act_cnt[0];
-  const int N = ns + h;
-  const int* act = s.act_list;
-  for (int i = lane; i < ns; i += 64) ybuf[i] = x[act[i]];
-  for (int i = lane; i < h; i += 64) ybuf[ns + i] = tail[i] + (g ? g[i] : 0.0);
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  if (lane == 0)
-    for (int i = 0; i < N; i++) {
-      const int p = Spiv[i];
-      if (p != i) {
-        const double t = ybuf[i];
-        ybuf[i] = ybuf[p];
-        ybuf[p] = t;
-      }
-    }
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  for (int l = 0; l < N; l++) {
-    const double yl = ybuf[l];
-    for (int i = l + 1 + lane; i < N; i += 64) ybuf[i] -= Smat[i + (int64_t)N * l] * yl;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+// rhs = [x(skel); g - the sum of the partial products mPsi^T(red,:) x]  (g:
+// the right-hand side of the border rows; null: zero, as in the reference's
+// [f; 0]).  Workgroups 0 .. h-1 form one border entry each, the others copy.
+__global__ __launch_bounds__(256) void k_border_rhs(DevState s, const double* x,
+                                                    const double* partial, int nblk, int h,
+                                                    const double* g, double* rhs) {
+  __shared__ double red[256];
+  const int ns = s.act_cnt[0], a = blockIdx.x;
+  if (a < h) {
+    const double v = sum_partials(partial, nblk, h, a, red);
+    if (threadIdx.x == 0) rhs[ns + a] = (g ? g[a] : 0.0) - v;
+    return;
   }
-  for (int i = N - 1; i >= 0; i--) {
-    if (lane == 0) ybuf[i] /= Smat[i + (int64_t)N * i];
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const double yi = ybuf[i];
-    for (int l = lane; l < i; l += 64) ybuf[l] -= Smat[l + (int64_t)N * i] * yi;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+  const int i = (a - h) * 256 + threadIdx.x;
+  if (i < ns) rhs[i] = x[s.act_list[i]];
+}
+
+// y = S^{-1} rhs; x(skel) = y_head, alpha = y_tail: 16 rows per workgroup,
+// a row's sum in 16 strided parts added in order (a 354-DOF S: 982 us by
+// triangular solves in one wave, 12 us).
+__global__ __launch_bounds__(256) void k_border_solve(DevState s, const double* Sinv, int h,
+                                                      const double* rhs, double* x,
+                                                      double* alpha) {
+  __shared__ double red[16][17];
+  const int ns = s.act_cnt[0], N = ns + h;
+  const int row = threadIdx.x & 15, part = threadIdx.x >> 4;
+  const int i = blockIdx.x * 16 + row;
+  double acc = 0;
+  if (i < N)
+    for (int j = part; j < N; j += 16) acc = fma(Sinv[i + (int64_t)N * j], rhs[j], acc);
+  red[part][row] = acc;
+  __syncthreads();
+  if (part == 0 && i < N) {
+    double y = 0;
+#pragma unroll
+    for (int q = 0; q < 16; q++) y += red[q][row];
+    if (i < ns) x[s.act_list[i]] = y;
+    else alpha[i - ns] = y;
   }
-  for (int i = lane; i < ns; i += 64) x[act[i]] = ybuf[i];
-  for (int i = lane; i < h; i += 64) alpha[i] = ybuf[ns + i];
 }
 
 // x(red) -= C(red,:) alpha.
-__global__ void k_red_update(double* x, const double* C, const int* mask,
-                             const double* alpha, int64_t ndof, int h) {
+__global__ void k_red_update(double* x, const double* C, const int* mask, const double* alpha,
+                             int64_t ndof, int h) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ndof;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (mask[i]) continue;
     double acc = x[i];
-    for (int c = 0; c < h; c++) acc -= C[i + ndof * c] * alpha[c];
+    for (int c = 0; c < h; c++) acc -= C[i * h + c] * alpha[c];
     x[i] = acc;
   }
 }
 
-constexpr int64_t kChunk = 4096;
+// y[i] += sum_c U[i,c] a[c].
+__global__ void k_border_apply_u(double* y, const double* U, const double* a, int64_t ndof,
+                                 int h) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ndof;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    double acc = y[i];
+    for (int c = 0; c < h; c++) acc += U[i * h + c] * a[c];
+    y[i] = acc;
+  }
+}
+
+// Rows of a partial sum: 1,024 workgroups of a product at 262,144 DOFs (256
+// rows; 64 of 4,096 rows left the chip idle), the Gram matrix's h^2 sums in
+// fewer.
+constexpr int64_t kChunk = 256;
+inline int64_t gram_chunk(int h) { return h <= 48 ? 1024 : 4096; }
+inline int blocks_of(int64_t n, int64_t chunk) { return (int)((n + chunk - 1) / chunk); }
 
 }  // namespace
 
@@ -266,53 +260,65 @@ void launch_gather_rows(void* dst, const void* src, const int* map, int n_rows, 
                                         row_words);
 }
 
-int64_t border_partial_blocks(int64_t ndof) { return (ndof + kChunk - 1) / kChunk; }
+int64_t border_partials(int64_t ndof, int h) {
+  return std::max((int64_t)blocks_of(ndof, kChunk) * h,
+                  (int64_t)blocks_of(ndof, gram_chunk(h)) * h * h);
+}
 
 void launch_border_gram(const double* P, const double* C, const int* mask,
                         int64_t ndof, int h, double* partial, double* out,
                         hipStream_t st) {
-  const int nb = (int)border_partial_blocks(ndof);
-  k_gram_partial<<<nb, 256, 0, st>>>(P, C, mask, ndof, h, kChunk, partial);
-  k_reduce_partials<<<(h * h + 255) / 256, 256, 0, st>>>(partial, nb, h * h,
-                                                        out, 1.0);
-}
-
-void launch_border_gemv(const double* P, const double* x, const int* mask,
-                        int64_t ndof, int h, double* partial, double* out,
-                        double sign, hipStream_t st) {
-  const int nb = (int)border_partial_blocks(ndof);
-  k_gemv_partial<<<nb, 64, 0, st>>>(P, x, mask, ndof, h, kChunk, partial);
-  k_reduce_partials<<<1, 64, 0, st>>>(partial, nb, h, out, sign);
+  const int nb = blocks_of(ndof, gram_chunk(h));
+  k_gram_partial<<<nb, 256, 0, st>>>(P, C, mask, ndof, h, gram_chunk(h), partial);
+  k_reduce_partials<<<h * h, 256, 0, st>>>(partial, nb, h * h, out, nullptr);
 }
 
 template <typename R>
-void launch_border_factor(const DevState& s, const double* mU,
-                          const double* mPsiT, const double* gram,
-                          int64_t ndof, int h, double* Smat, int* Spiv,
+void launch_border_factor(const DevState& s, const double* mU, const double* mPsiT,
+                          const double* gram, int h, double* Smat, double* Sinv, int* Spiv,
                           hipStream_t st) {
-  k_border_factor<R><<<1, 1024, 0, st>>>(s, mU, mPsiT, gram, ndof, h, Smat, Spiv);
+  const int piv_stride = s.ncap + h + kInvFlags;
+  k_border_assemble<R><<<128, 256, 0, st>>>(s, mU, mPsiT, gram, h, Smat,
+                                            Spiv + piv_stride - kInvFlags);
+  InvBlocks<double> blk;
+  blk.a = Smat;
+  blk.out = Sinv;
+  blk.stride = 0;
+  blk.piv = Spiv;
+  blk.piv_stride = piv_stride;
+  blk.extra = h;
+  launch_block_inverse<double>(s, blk, 1, 0, s.ncap + h, st);
 }
 
-void launch_border_solve(const DevState& s, const double* Smat,
-                         const int* Spiv, int h, double* x, const double* tail,
-                         const double* g, double* alpha, double* ybuf,
-                         hipStream_t st) {
-  k_border_solve<<<1, 64, 0, st>>>(s, Smat, Spiv, h, x, tail, g, alpha, ybuf);
+void launch_border_solve(const DevState& s, const double* mPsiT, const double* Sinv,
+                         const int* mask, int64_t ndof, int h, double* x, const double* g,
+                         double* alpha, double* partial, double* rhs, hipStream_t st) {
+  const int nb = blocks_of(ndof, kChunk), nmax = s.ncap + h;
+  k_gemv_partial<<<nb, 256, 0, st>>>(mPsiT, x, mask, ndof, h, kChunk, partial);
+  k_border_rhs<<<h + (s.ncap + 255) / 256, 256, 0, st>>>(s, x, partial, nb, h, g, rhs);
+  k_border_solve<<<(nmax + 15) / 16, 256, 0, st>>>(s, Sinv, h, rhs, x, alpha);
 }
 
 void launch_red_update(double* x, const double* C, const int* mask,
                        const double* alpha, int64_t ndof, int h,
                        hipStream_t st) {
-  k_red_update<<<512, 256, 0, st>>>(x, C, mask, alpha, ndof, h);
+  k_red_update<<<1024, 256, 0, st>>>(x, C, mask, alpha, ndof, h);
 }
 
-template void launch_border_factor<double>(const DevState&, const double*,
-                                           const double*, const double*,
-                                           int64_t, int, double*, int*,
+void launch_border_apply(const double* U, const double* PsiT, const double* x,
+                         const double* alpha, int64_t ndof, int h, double* partial, double* y,
+                         double* z, hipStream_t st) {
+  const int nb = blocks_of(ndof, kChunk);
+  k_border_apply_u<<<1024, 256, 0, st>>>(y, U, alpha, ndof, h);
+  k_gemv_partial<<<nb, 256, 0, st>>>(PsiT, x, nullptr, ndof, h, kChunk, partial);
+  k_reduce_partials<<<h, 256, 0, st>>>(partial, nb, h, z, alpha);
+}
+
+template void launch_border_factor<double>(const DevState&, const double*, const double*,
+                                           const double*, int, double*, double*, int*,
                                            hipStream_t);
-template void launch_border_factor<float>(const DevState&, const double*,
-                                          const double*, const double*,
-                                          int64_t, int, double*, int*,
+template void launch_border_factor<float>(const DevState&, const double*, const double*,
+                                          const double*, int, double*, double*, int*,
                                           hipStream_t);
 
 }  // namespace iegpu

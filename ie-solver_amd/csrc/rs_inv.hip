@@ -1,0 +1,296 @@
+// Inverse of a dense block over many workgroups: the root blocks above
+// kRootRegMax DOFs (skel_factorization.cpp:172-186) and the bordered system
+// of multiply connected domains (:188-305), which the reference LU-factors.
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "rs_device.hpp"
+#include "rs_inv.hpp"
+
+namespace iegpu {
+
+namespace {
+
+// ---------------------------------------------------------------------------
+// Blocked Gauss-Jordan with partial pivoting, rows not moved.  Workgroup j
+// of a block's group owns the kInvB = 16 columns of panel j, thread t the
+// rows t, t + 512, ...: a panel's 16 elimination steps run on registers
+// (pivot row: largest |entry| among the rows not yet pivoted, one barrier
+// per step), and the other columns take them at once: with W the final slab
+// of panel q and P its pivot rows' old values, the steps turn a column x
+// into x + sum_k W_k x_{p_k}, a pivot row's own value being replaced rather
+// than added to.
+//
+// k_inv_panel: workgroup j applies panels 0 .. j-1 to its columns as they
+// are published, eliminates its own and publishes it (the slab over its own
+// columns of the block, the pivot rows, then the panel's flag).  It waits
+// only for workgroups of lower index in its own launch, which the
+// dispatcher starts first, so a wait ends wherever the others run.
+// k_inv_finish: the columns of panel j take the panels j+1, ... (all
+// published), four columns per workgroup, and the unpermuted inverse is
+// written.
+//
+// Bound by the chain of panels (wait, one update, 16 pivot steps, publish):
+// about 18 us per panel in FP64.  A 212-DOF root: 277 us (986 us with one
+// workgroup streaming the block from L2); 393 DOFs: 530 us (2,984 us); the
+// 354-DOF bordered system of Stokes with 8 holes: 525 us (7,570 us by an LU
+// in one workgroup).
+// ---------------------------------------------------------------------------
+
+constexpr int kInvB = 16;       // columns of a panel
+constexpr int kInvNT = 512;     // threads: rows per pass
+constexpr int kInvCF = 4;       // columns of a k_inv_finish workgroup
+constexpr int kInvNW = kInvNT / 64;
+constexpr int kRowBits = 11;    // row index bits of a pivot key
+static_assert(kInvMax <= (1 << kRowBits) && kInvMax <= 3 * kInvNT, "rows per thread");
+
+__device__ inline unsigned mag_bits(double v) {
+  return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffffu;
+}
+__device__ inline unsigned mag_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+
+__device__ inline unsigned wave_max_u32(unsigned v) {
+  v = max(v, (unsigned)dpp_i32<dpp::kQuadSwap1, 0xF>((int)v));
+  v = max(v, (unsigned)dpp_i32<dpp::kQuadSwap2, 0xF>((int)v));
+  v = max(v, (unsigned)dpp_i32<dpp::kRowHalfMirror, 0xF>((int)v));
+  v = max(v, (unsigned)dpp_i32<dpp::kRowMirror, 0xF>((int)v));
+  v = max(v, (unsigned)dpp_i32<dpp::kRowBcast15, 0xA>((int)v));
+  v = max(v, (unsigned)dpp_i32<dpp::kRowBcast31, 0xC>((int)v));
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// A pivot candidate's key: the leading magnitude bits above the row index
+// (a magnitude within 2^-9 of the largest may win; the smaller row on
+// ties), 0 for a row that is no candidate.
+template <typename R>
+__device__ inline unsigned inv_key(R v, int row) {
+  constexpr unsigned kMask = (1u << kRowBits) - 1;
+  return (mag_bits(v) & ~kMask) | (kMask - (unsigned)row);
+}
+
+// Wait of a workgroup for panel flag *f: bounded (about two seconds), false
+// if it never came.
+__device__ inline bool wait_flag(const int* f) {
+  for (int spin = 0; spin < (1 << 22); spin++) {
+    if (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      return true;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return false;
+}
+
+// x (columns CB of the thread's RT rows) takes panel q: W from the block's
+// columns, the pivot rows' old values through LDS.  pstep[row] is the step
+// that pivots on a row (kInvMax: none yet) and is extended by the panel's.
+// All threads of the workgroup.
+template <typename R, int RT, int CB>
+__device__ inline void apply_panel(const R* A, const int* prow, int n, int q, R (&x)[RT][CB],
+                                   short* pstep, R (*P)[CB]) {
+  const int tid = threadIdx.x, q0 = q * kInvB, bw = min(kInvB, n - q0);
+  R w[RT][kInvB];
+#pragma unroll
+  for (int u = 0; u < RT; u++) {
+    const int i = tid + kInvNT * u;
+#pragma unroll
+    for (int k = 0; k < kInvB; k++)
+      w[u][k] = (i < n && k < bw) ? A[i + (int64_t)n * (q0 + k)] : R(0);
+  }
+  if (tid < bw) pstep[prow[q0 + tid]] = (short)(q0 + tid);
+  if (bw < kInvB && tid < kInvB * CB) P[tid / CB][tid % CB] = R(0);  // steps past the last
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < RT; u++) {
+    const int i = tid + kInvNT * u;
+    const int st = i < n ? pstep[i] - q0 : -1;
+    if (st >= 0 && st < bw) {
+#pragma unroll
+      for (int c = 0; c < CB; c++) {
+        P[st][c] = x[u][c];
+        x[u][c] = R(0);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kInvB; k++)
+#pragma unroll
+    for (int c = 0; c < CB; c++) {
+      const R p = P[k][c];
+#pragma unroll
+      for (int u = 0; u < RT; u++) x[u][c] = fma(w[u][k], p, x[u][c]);
+    }
+}
+
+template <typename R, int RT>
+__global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> blk, int nmin,
+                                                      int nmax) {
+  __shared__ R P[kInvB][kInvB];
+  __shared__ R cand[2][kInvNW][kInvB];  // each wave's candidate row, by step parity
+  __shared__ unsigned keys[2][kInvNW];
+  __shared__ short pstep[kInvMax];
+  __shared__ int ok;
+  if (!pools_ok(s)) return;
+  const int root = blockIdx.y, j = blockIdx.x, j0 = j * kInvB;
+  const int n = s.act_cnt[root] + blk.extra;
+  if (n <= nmin || n > nmax || j0 >= n) return;
+  R* A = blk.a + blk.stride * root;
+  int* prow = blk.piv + (int64_t)blk.piv_stride * root;
+  int* flags = prow + blk.piv_stride - kInvFlags;
+  const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
+  const int bw = min(kInvB, n - j0);
+  R x[RT][kInvB];
+#pragma unroll
+  for (int u = 0; u < RT; u++) {
+    const int i = tid + kInvNT * u;
+#pragma unroll
+    for (int k = 0; k < kInvB; k++)
+      x[u][k] = (i < n && k < bw) ? A[i + (int64_t)n * (j0 + k)] : R(0);
+  }
+  for (int i = tid; i < n; i += kInvNT) pstep[i] = (short)kInvMax;
+  for (int q = 0; q < j; q++) {
+    if (tid == 0) ok = wait_flag(flags + q) ? 1 : 0;
+    __syncthreads();
+    if (!ok) {
+      if (tid == 0) atomicOr(s.err, kErrWait);
+      return;
+    }
+    apply_panel<R, RT, kInvB>(A, prow, n, q, x, pstep, P);
+    __syncthreads();
+  }
+  // the panel's own steps
+  bool used[RT];
+#pragma unroll
+  for (int u = 0; u < RT; u++) {
+    const int i = tid + kInvNT * u;
+    used[u] = i >= n || pstep[i] != kInvMax;
+  }
+  int info = 0;
+#pragma unroll
+  for (int k = 0; k < kInvB; k++) {
+    if (k < bw) {
+      unsigned key = 0;
+#pragma unroll
+      for (int u = 0; u < RT; u++)
+        key = max(key, used[u] ? 0u : inv_key(x[u][k], tid + kInvNT * u));
+      const unsigned best = wave_max_u32(key);
+      if (best != 0 && key == best) {
+#pragma unroll
+        for (int u = 0; u < RT; u++)
+          if (!used[u] && inv_key(x[u][k], tid + kInvNT * u) == best) {
+#pragma unroll
+            for (int c = 0; c < kInvB; c++) cand[k & 1][wv][c] = x[u][c];
+          }
+      }
+      if (lane == 0) keys[k & 1][wv] = best;
+      __syncthreads();
+      unsigned top = keys[k & 1][0];
+      int tw = 0;
+#pragma unroll
+      for (int q = 1; q < kInvNW; q++) {
+        const unsigned v = keys[k & 1][q];
+        tw = v > top ? q : tw;
+        top = max(top, v);
+      }
+      const int p = (1 << kRowBits) - 1 - (int)(top & ((1u << kRowBits) - 1));
+      R rv[kInvB];
+#pragma unroll
+      for (int c = 0; c < kInvB; c++) rv[c] = cand[k & 1][tw][c];
+      const R piv = rv[k];
+      if (piv == R(0) && info == 0) info = j0 + k + 1;
+      const R inv = R(1) / piv;
+#pragma unroll
+      for (int c = 0; c < kInvB; c++) rv[c] = c == k ? inv : rv[c] * inv;
+#pragma unroll
+      for (int u = 0; u < RT; u++) {
+        const R m = x[u][k];
+        const bool me = tid + kInvNT * u == p;
+        x[u][k] = R(0);
+#pragma unroll
+        for (int c = 0; c < kInvB; c++) x[u][c] = me ? rv[c] : fma(-m, rv[c], x[u][c]);
+        used[u] = used[u] || me;
+      }
+      if (tid == 0) prow[j0 + k] = p;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < RT; u++) {
+    const int i = tid + kInvNT * u;
+#pragma unroll
+    for (int k = 0; k < kInvB; k++)
+      if (i < n && k < bw) A[i + (int64_t)n * (j0 + k)] = x[u][k];
+  }
+  if (info != 0 && tid == 0) atomicOr(s.err, kErrSingular);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // every thread's part of the slab
+  __syncthreads();
+  if (tid == 0)
+    __hip_atomic_store(flags + j, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <typename R, int RT>
+__global__ __launch_bounds__(kInvNT) void k_inv_finish(DevState s, InvBlocks<R> blk, int nmin,
+                                                       int nmax) {
+  __shared__ R P[2][kInvB][kInvCF];
+  __shared__ short pstep[kInvMax];
+  if (!pools_ok(s) || (s.err[0] & kErrWait)) return;
+  const int root = blockIdx.y, c0 = blockIdx.x * kInvCF;
+  const int n = s.act_cnt[root] + blk.extra;
+  if (n <= nmin || n > nmax || c0 >= n) return;
+  const R* A = blk.a + blk.stride * root;
+  R* B = blk.out ? blk.out + blk.stride * root : blk.a + blk.stride * root + (int64_t)n * n;
+  const int* prow = blk.piv + (int64_t)blk.piv_stride * root;
+  const int tid = threadIdx.x;
+  R x[RT][kInvCF];
+#pragma unroll
+  for (int u = 0; u < RT; u++) {
+    const int i = tid + kInvNT * u;
+#pragma unroll
+    for (int c = 0; c < kInvCF; c++)
+      x[u][c] = (i < n && c0 + c < n) ? A[i + (int64_t)n * (c0 + c)] : R(0);
+  }
+  for (int st = tid; st < n; st += kInvNT) pstep[prow[st]] = (short)st;
+  const int np = (n + kInvB - 1) / kInvB;
+  for (int q = c0 / kInvB + 1; q < np; q++)
+    apply_panel<R, RT, kInvCF>(A, prow, n, q, x, pstep, P[q & 1]);
+  __syncthreads();
+  // entry (row i, column c): inverse row = the step that pivoted on i,
+  // column = the row step c pivoted on
+#pragma unroll
+  for (int u = 0; u < RT; u++) {
+    const int i = tid + kInvNT * u;
+    if (i >= n) continue;
+    const int row = pstep[i];
+#pragma unroll
+    for (int c = 0; c < kInvCF; c++)
+      if (c0 + c < n) B[row + (int64_t)n * prow[c0 + c]] = x[u][c];
+  }
+}
+
+}  // namespace
+
+template <typename R>
+void launch_block_inverse(const DevState& s, const InvBlocks<R>& blk, int n_blocks, int nmin,
+                          int nmax, hipStream_t st) {
+  // one row per thread, or three
+  const int m1 = nmax < kInvNT ? nmax : kInvNT;
+  auto grid = [&](int n, int cols) { return dim3((n + cols - 1) / cols, n_blocks); };
+  if (nmin < kInvNT) {
+    k_inv_panel<R, 1><<<grid(m1, kInvB), kInvNT, 0, st>>>(s, blk, nmin, m1);
+    k_inv_finish<R, 1><<<grid(m1, kInvCF), kInvNT, 0, st>>>(s, blk, nmin, m1);
+  }
+  if (nmax > kInvNT) {
+    const int lo = nmin > kInvNT ? nmin : kInvNT;
+    k_inv_panel<R, 3><<<grid(nmax, kInvB), kInvNT, 0, st>>>(s, blk, lo, nmax);
+    k_inv_finish<R, 3><<<grid(nmax, kInvCF), kInvNT, 0, st>>>(s, blk, lo, nmax);
+  }
+}
+
+template void launch_block_inverse<double>(const DevState&, const InvBlocks<double>&, int, int,
+                                           int, hipStream_t);
+template void launch_block_inverse<float>(const DevState&, const InvBlocks<float>&, int, int,
+                                          int, hipStream_t);
+
+}  // namespace iegpu

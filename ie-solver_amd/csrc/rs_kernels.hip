@@ -20,6 +20,7 @@
 #include <cstdint>
 
 #include "rs_device.hpp"
+#include "rs_inv.hpp"
 #include "rs_kernels.hpp"
 
 namespace iegpu {
@@ -2527,6 +2528,8 @@ __global__ __launch_bounds__(NT) void k_root(DevGeom g, DevTree t, DevState s) {
     s.m_rows[b] = 0;
     s.out_cnt[b] = s.act_cnt[b];
   }
+  if (blockIdx.y == 0)  // the block inverse's panel flags
+    for (int i = tid; i < kInvFlags; i += NT) root_pivots(s, b)[s.ncap + i] = 0;
   if (b == 0 && lead && s.plan_skip != nullptr) {
     // The launch plan skipped kernels whose lists it expected empty: any
     // that is not makes the host run the factorization again in full.
@@ -2607,7 +2610,7 @@ constexpr int kRootTR = 32, kRootTC = 32, kRootRU = 6, kRootCV = 6;
 constexpr int kRootPB = 8;
 
 template <typename R>
-__global__ __launch_bounds__(kRootTR * kRootTC) void k_root_inv(DevState s, int factor_lu) {
+__global__ __launch_bounds__(kRootTR * kRootTC) void k_root_inv(DevState s) {
   constexpr int NMAX = kRootRegMax, PB = kRootPB, NS = NMAX / 64;
   static_assert(kRootTC % PB == 0 && NMAX == kRootTR * kRootRU && NMAX == kRootTC * kRootCV &&
                 NMAX % 64 == 0 && NMAX % PB == 0 && NMAX <= 256 && PB * PB <= 64,
@@ -2622,7 +2625,7 @@ __global__ __launch_bounds__(kRootTR * kRootTC) void k_root_inv(DevState s, int 
   __shared__ int prow[NMAX];
   __shared__ int invrow[NMAX];
   __shared__ R park[kRootRU * kRootCV][64];
-  if (!factor_lu || !pools_ok(s)) return;
+  if (!pools_ok(s)) return;
   const int n = s.act_cnt[blockIdx.x];
   if (n == 0 || n > NMAX) return;
   const int n8 = (n + PB - 1) / PB * PB;
@@ -2873,402 +2876,6 @@ __global__ __launch_bounds__(kRootTR * kRootTC) void k_root_inv(DevState s, int 
     }
   if (info != 0 && tid == 0) atomicOr(s.err, kErrSingular);
 }
-// ---------------------------------------------------------------------------
-// Solve sweeps (skel_factorization.cpp:507-592).  One wave per box; the
-// box's skeleton and redundant entries are gathered to LDS, updated and
-// scattered back (boxes of one level touch disjoint DOFs).
-// ---------------------------------------------------------------------------
-
-// sum_j p[stride j] v[j], j < len: eight loads in flight, four partial
-// sums (a sweep's per-lane loop is otherwise one load latency per term).
-template <typename R>
-__device__ inline double dot_ld(const R* p, int64_t stride, const double* v, int len) {
-  double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
-  int j = 0;
-  for (; j + 8 <= len; j += 8) {
-    R q[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) q[u] = p[stride * (j + u)];
-    a0 += (double)q[0] * v[j] + (double)q[4] * v[j + 4];
-    a1 += (double)q[1] * v[j + 1] + (double)q[5] * v[j + 5];
-    a2 += (double)q[2] * v[j + 2] + (double)q[6] * v[j + 6];
-    a3 += (double)q[3] * v[j + 3] + (double)q[7] * v[j + 7];
-  }
-  for (; j < len; j++) a0 += (double)p[stride * j] * v[j];
-  return (a0 + a1) + (a2 + a3);
-}
-
-// x <- X^{-1} x with an explicit inverse (r x r, ld r): one wave, x and
-// tmp in LDS.
-template <typename R>
-__device__ void wave_inv_apply(const R* Xi, int r, double* x, double* tmp) {
-  const int lane = threadIdx.x & 63;
-  for (int i = lane; i < r; i += 64) tmp[i] = dot_ld(Xi + i, r, x, r);
-  wave_sync();
-  for (int i = lane; i < r; i += 64) x[i] = tmp[i];
-  wave_sync();
-}
-
-template <typename R>
-__global__ __launch_bounds__(64) void k_sweep_up(DevState s, int start,
-                                                 SolveVec v, int use_Ut,
-                                                 int diag) {
-  __shared__ double xs[kMaxBoxDofs];
-  __shared__ double xr[kMaxBoxDofs];
-  __shared__ double tmp[kMaxBoxDofs];
-  const int b = start + blockIdx.x;
-  const int k = s.rank[b];
-  if (k == 0) return;
-  const int lane = threadIdx.x;
-  const int r = s.act_cnt[b] - k;
-  const FacLayout fl = FacLayout::make(k, r);
-  const R* F = reinterpret_cast<const R*>(s.fac_pool) + s.fac_off[b];
-  const int* sk = s.out_list + (int64_t)b * s.ncap;
-  const int* rd = s.red_list + (int64_t)b * s.ncap;
-  for (int c = 0; c < v.nrhs; c++) {
-    double* x = v.x + v.ldx * c;
-    for (int a = lane; a < k; a += 64) xs[a] = x[sk[a]];
-    for (int i = lane; i < r; i += 64) xr[i] = x[rd[i]];
-    wave_sync();
-    for (int i = lane; i < r; i += 64) xr[i] -= dot_ld(F + fl.T + (int64_t)k * i, 1, xs, k);
-    wave_sync();
-    for (int a = lane; a < k; a += 64) {
-      if (use_Ut) xs[a] -= dot_ld(F + fl.U + (int64_t)r * a, 1, xr, r);
-      else xs[a] -= dot_ld(F + fl.L + a, k, xr, r);
-    }
-    wave_sync();
-    if (diag) wave_inv_apply(F + fl.X, r, xr, tmp);
-    for (int a = lane; a < k; a += 64) x[sk[a]] = xs[a];
-    for (int i = lane; i < r; i += 64) x[rd[i]] = xr[i];
-    wave_sync();
-  }
-}
-
-template <typename R>
-__global__ __launch_bounds__(64) void k_diag(DevState s, int start, SolveVec v) {
-  __shared__ double xr[kMaxBoxDofs];
-  __shared__ double tmp[kMaxBoxDofs];
-  const int b = start + blockIdx.x;
-  const int k = s.rank[b];
-  if (k == 0) return;
-  const int lane = threadIdx.x;
-  const int r = s.act_cnt[b] - k;
-  const FacLayout fl = FacLayout::make(k, r);
-  const R* F = reinterpret_cast<const R*>(s.fac_pool) + s.fac_off[b];
-  const int* rd = s.red_list + (int64_t)b * s.ncap;
-  for (int c = 0; c < v.nrhs; c++) {
-    double* x = v.x + v.ldx * c;
-    for (int i = lane; i < r; i += 64) xr[i] = x[rd[i]];
-    wave_sync();
-    wave_inv_apply(F + fl.X, r, xr, tmp);
-    for (int i = lane; i < r; i += 64) x[rd[i]] = xr[i];
-    wave_sync();
-  }
-}
-
-template <typename R>
-__global__ __launch_bounds__(64) void k_sweep_down(DevState s, int start,
-                                                   SolveVec v) {
-  __shared__ double xs[kMaxBoxDofs];
-  __shared__ double xr[kMaxBoxDofs];
-  const int b = start + blockIdx.x;
-  const int k = s.rank[b];
-  if (k == 0) return;
-  const int lane = threadIdx.x;
-  const int r = s.act_cnt[b] - k;
-  const FacLayout fl = FacLayout::make(k, r);
-  const R* F = reinterpret_cast<const R*>(s.fac_pool) + s.fac_off[b];
-  const int* sk = s.out_list + (int64_t)b * s.ncap;
-  const int* rd = s.red_list + (int64_t)b * s.ncap;
-  for (int c = 0; c < v.nrhs; c++) {
-    double* x = v.x + v.ldx * c;
-    for (int a = lane; a < k; a += 64) xs[a] = x[sk[a]];
-    for (int i = lane; i < r; i += 64) xr[i] = x[rd[i]];
-    wave_sync();
-    for (int i = lane; i < r; i += 64) xr[i] -= dot_ld(F + fl.U + i, r, xs, k);
-    wave_sync();
-    for (int a = lane; a < k; a += 64) xs[a] -= dot_ld(F + fl.T + a, k, xr, r);
-    wave_sync();
-    for (int a = lane; a < k; a += 64) x[sk[a]] = xs[a];
-    for (int i = lane; i < r; i += 64) x[rd[i]] = xr[i];
-    wave_sync();
-  }
-}
-
-// Blocked in-place Gauss-Jordan inverse of a root block with
-// kRootRegMax < n <= kRootBlkMax, one workgroup per root, thread t owning
-// row t.  Per panel of 16 columns J:
-//   1. the panel's 16 elimination steps run on the n x 16 slab in
-//      registers (pivot row: largest |value| among the rows not yet
-//      pivoted, as gj_invert; one barrier per step);
-//   2. the other columns take all 16 steps at once: with W the final slab
-//      and P the panel's pivot rows, the steps multiply every other column
-//      x by G = I + sum_k (W_k - e_{p_k}) e_{p_k}^T, so
-//      x_i += sum_k W_ik x_{p_k} (old values of the pivot rows), and a
-//      pivot row's own value is replaced rather than added to.
-// The result equals the column-by-column algorithm up to rounding order.
-// The inverse, unpermuted, goes after the matrix, as in k_root_inv.
-constexpr int kRootBlkB = 16;
-
-template <typename R>
-__global__ __launch_bounds__(kRootBlkMax) void k_root_inv_blk(DevState s, int factor_lu) {
-  constexpr int B = kRootBlkB, NW = kRootBlkMax / 64;
-  __shared__ R rowv[2][NW][B];
-  __shared__ double keys[2][NW];
-  __shared__ R Rl[kRootBlkMax * B];
-  __shared__ int prow[kRootBlkMax];
-  __shared__ int invrow[kRootBlkMax];
-  __shared__ int pan[B];
-  if (!factor_lu || !pools_ok(s)) return;
-  const int root = blockIdx.x;
-  const int n = s.act_cnt[root];
-  if (n <= kRootRegMax) return;
-  if (n > kRootBlkMax) {
-    // Gauss-Jordan inverse (the reference LU-factors the root block) in
-    // global memory for blocks too large for the register forms; the
-    // inverse, unpermuted, goes after the assembled matrix
-    R* A = root_block<R>(s, root);
-    R* B = A + (int64_t)n * n;
-    int* gp = root_pivots(s, root);
-    const int info = gj_invert_into<R, kRootBlkMax>(A, B, n, gp);
-    if (info != 0 && threadIdx.x == 0) atomicOr(s.err, kErrSingular);
-    for (int64_t idx = threadIdx.x; idx < (int64_t)n * n; idx += kRootBlkMax) {
-      const int j = (int)(idx % n), jj = (int)(idx / n);
-      B[j + (int64_t)n * gp[jj]] = A[gp[j] + (int64_t)n * jj];
-    }
-    return;
-  }
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int i = tid;  // own row
-  const bool live = i < n;
-  R* A = root_block<R>(s, root);
-  bool used = !live;
-  int info = 0;
-  for (int j0 = 0; j0 < n; j0 += B) {
-    const int bw = min(B, n - j0);
-    R w[B];
-#pragma unroll
-    for (int k = 0; k < B; k++) w[k] = (live && k < bw) ? A[i + (int64_t)n * (j0 + k)] : R(0);
-    bool inpan = false;
-#pragma unroll
-    for (int k = 0; k < B; k++) {
-      if (k < bw) {
-        R v = fabs(w[k]);
-        if (!isfinite(v)) v = R(0);  // every unpivoted row stays a candidate
-        const double key = used ? -1.0 : pivot_key<R, 9>(v, i);
-        const double wbest = wave_max(key);
-        const int buf = k & 1;
-        if (!used && key == wbest) {
-#pragma unroll
-          for (int c = 0; c < B; c++) rowv[buf][wv][c] = w[c];
-        }
-        if (lane == 0) keys[buf][wv] = wbest;
-        __syncthreads();
-        double best = keys[buf][0];
-        int bwv = 0;
-#pragma unroll
-        for (int q = 1; q < NW; q++)
-          if (keys[buf][q] > best) {
-            best = keys[buf][q];
-            bwv = q;
-          }
-        const int p = pivot_key_pos<9>(best);
-        R rv[B];
-#pragma unroll
-        for (int c = 0; c < B; c++) rv[c] = rowv[buf][bwv][c];
-        const R piv = rv[k];
-        if (piv == R(0) && info == 0) info = j0 + k + 1;
-        const R inv = R(1) / piv;
-#pragma unroll
-        for (int c = 0; c < B; c++) rv[c] = (c == k) ? inv : rv[c] * inv;
-        const R cv = w[k];
-        w[k] = R(0);
-#pragma unroll
-        for (int c = 0; c < B; c++) w[c] -= cv * rv[c];
-        if (i == p) {
-#pragma unroll
-          for (int c = 0; c < B; c++) w[c] = rv[c];
-          used = true;
-          inpan = true;
-        }
-        if (tid == 0) {
-          prow[j0 + k] = p;
-          pan[k] = p;
-        }
-      }
-    }
-    __syncthreads();
-    // old values of the panel's pivot rows in every other column
-    for (int idx = tid; idx < n * B; idx += kRootBlkMax) {
-      const int c = idx / B, k = idx % B;
-      const bool skip = k >= bw || (c >= j0 && c < j0 + bw);
-      Rl[idx] = skip ? R(0) : A[pan[k] + (int64_t)n * c];
-    }
-    __syncthreads();
-    // Own row, 16 columns per chunk; the next chunk's loads are issued
-    // before the current chunk's arithmetic so one load latency is exposed
-    // per panel rather than per chunk.
-    constexpr int CH = 16;
-    auto load_chunk = [&](int c0, R* x) {
-#pragma unroll
-      for (int q = 0; q < CH; q++) {
-        const int c = c0 + q;
-        const bool other = c < n && (c < j0 || c >= j0 + bw);
-        x[q] = (live && other && !inpan) ? A[i + (int64_t)n * c] : R(0);
-      }
-    };
-    R x[CH], xn[CH];
-    load_chunk(0, x);
-    for (int c0 = 0; c0 < n; c0 += CH) {
-      if (c0 + CH < n) load_chunk(c0 + CH, xn);
-#pragma unroll
-      for (int q = 0; q < CH; q++) {
-        const int c = c0 + q;
-        if (c < n && (c < j0 || c >= j0 + bw)) {
-          R acc = x[q];
-#pragma unroll
-          for (int k = 0; k < B; k++) acc += w[k] * Rl[c * B + k];
-          if (live) A[i + (int64_t)n * c] = acc;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < CH; q++) x[q] = xn[q];
-    }
-#pragma unroll
-    for (int k = 0; k < B; k++)
-      if (live && k < bw) A[i + (int64_t)n * (j0 + k)] = w[k];
-    __syncthreads();
-  }
-  if (tid < n) invrow[prow[tid]] = tid;
-  __syncthreads();
-  R* Bm = A + (int64_t)n * n;
-  for (int64_t idx = tid; idx < (int64_t)n * n; idx += kRootBlkMax) {
-    const int r = (int)(idx % n), c = (int)(idx / n);
-    Bm[invrow[r] + (int64_t)n * prow[c]] = A[idx];
-  }
-  if (info != 0 && tid == 0) atomicOr(s.err, kErrSingular);
-}
-
-// x_root <- (root inverse) x_root: 256 threads, one row each per pass.
-template <typename R>
-__global__ __launch_bounds__(256) void k_root_solve(DevState s, SolveVec v) {
-  __shared__ double xa[kMaxBoxDofs];
-  const int tid = threadIdx.x;
-  const int n = s.act_cnt[blockIdx.x];
-  const int* act = s.act_list + (int64_t)blockIdx.x * s.ncap;
-  const R* Ai = root_block<R>(s, blockIdx.x) + (int64_t)n * n;
-  for (int c = 0; c < v.nrhs; c++) {
-    double* x = v.x + v.ldx * c;
-    for (int i = tid; i < n; i += 256) xa[i] = x[act[i]];
-    __syncthreads();
-    double y[kMaxBoxDofs / 256];
-#pragma unroll
-    for (int q = 0; q < kMaxBoxDofs / 256; q++) {
-      const int i = tid + 256 * q;
-      y[q] = i < n ? dot_ld(Ai + i, n, xa, n) : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kMaxBoxDofs / 256; q++) {
-      const int i = tid + 256 * q;
-      if (i < n) x[act[i]] = y[q];
-    }
-    __syncthreads();
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Compressed forward apply b = A x (SkelFactorization::sparse_matvec,
-// skel_factorization.cpp:429-504): the solve's steps undone in reverse
-// order.  Per compressed box, levels leaves first:
-//   b_s += T b_r;  b_r += U b_s;  b_r = X_rr b_r
-// (X_rr may follow each box at once: no later box touches its redundant
-// entries); then every root b = A_root b; then, root side first,
-//   b_s += L b_r;  b_r += T^T b_s.
-// One wave per box.
-// ---------------------------------------------------------------------------
-
-template <typename R>
-__global__ __launch_bounds__(64) void k_fwd_up(DevState s, int start, double* x) {
-  __shared__ double xs[kMaxBoxDofs];
-  __shared__ double xr[kMaxBoxDofs];
-  const int b = start + blockIdx.x;
-  const int k = s.rank[b];
-  if (k == 0) return;
-  const int lane = threadIdx.x;
-  const int r = s.act_cnt[b] - k;
-  const FacLayout fl = FacLayout::make(k, r);
-  const R* F = reinterpret_cast<const R*>(s.fac_pool) + s.fac_off[b];
-  const R* Xf = reinterpret_cast<const R*>(s.fwd_pool) + s.fac_off[b];
-  const int* sk = s.out_list + (int64_t)b * s.ncap;
-  const int* rd = s.red_list + (int64_t)b * s.ncap;
-  for (int a = lane; a < k; a += 64) xs[a] = x[sk[a]];
-  for (int i = lane; i < r; i += 64) xr[i] = x[rd[i]];
-  wave_sync();
-  for (int a = lane; a < k; a += 64) xs[a] += dot_ld(F + fl.T + a, k, xr, r);
-  wave_sync();
-  for (int i = lane; i < r; i += 64) xr[i] += dot_ld(F + fl.U + i, r, xs, k);
-  wave_sync();
-  double y[kMaxBoxDofs / 64];
-#pragma unroll
-  for (int q = 0; q < kMaxBoxDofs / 64; q++) {
-    const int i = lane + 64 * q;
-    y[q] = i < r ? dot_ld(Xf + i, r, xr, r) : 0.0;
-  }
-  for (int a = lane; a < k; a += 64) x[sk[a]] = xs[a];
-#pragma unroll
-  for (int q = 0; q < kMaxBoxDofs / 64; q++) {
-    const int i = lane + 64 * q;
-    if (i < r) x[rd[i]] = y[q];
-  }
-}
-
-template <typename R>
-__global__ __launch_bounds__(256) void k_fwd_root(DevState s, double* x) {
-  __shared__ double xa[kMaxBoxDofs];
-  const int tid = threadIdx.x;
-  const int n = s.act_cnt[blockIdx.x];
-  const int* act = s.act_list + (int64_t)blockIdx.x * s.ncap;
-  const R* A = reinterpret_cast<const R*>(s.root_fwd) + (int64_t)s.ncap * s.ncap * blockIdx.x;
-  for (int i = tid; i < n; i += 256) xa[i] = x[act[i]];
-  __syncthreads();
-  double y[kMaxBoxDofs / 256];
-#pragma unroll
-  for (int q = 0; q < kMaxBoxDofs / 256; q++) {
-    const int i = tid + 256 * q;
-    y[q] = i < n ? dot_ld(A + i, n, xa, n) : 0.0;
-  }
-#pragma unroll
-  for (int q = 0; q < kMaxBoxDofs / 256; q++) {
-    const int i = tid + 256 * q;
-    if (i < n) x[act[i]] = y[q];
-  }
-}
-
-template <typename R>
-__global__ __launch_bounds__(64) void k_fwd_down(DevState s, int start, double* x) {
-  __shared__ double xs[kMaxBoxDofs];
-  __shared__ double xr[kMaxBoxDofs];
-  const int b = start + blockIdx.x;
-  const int k = s.rank[b];
-  if (k == 0) return;
-  const int lane = threadIdx.x;
-  const int r = s.act_cnt[b] - k;
-  const FacLayout fl = FacLayout::make(k, r);
-  const R* F = reinterpret_cast<const R*>(s.fac_pool) + s.fac_off[b];
-  const int* sk = s.out_list + (int64_t)b * s.ncap;
-  const int* rd = s.red_list + (int64_t)b * s.ncap;
-  for (int a = lane; a < k; a += 64) xs[a] = x[sk[a]];
-  for (int i = lane; i < r; i += 64) xr[i] = x[rd[i]];
-  wave_sync();
-  for (int a = lane; a < k; a += 64) xs[a] += dot_ld(F + fl.L + a, k, xr, r);
-  wave_sync();
-  for (int i = lane; i < r; i += 64) xr[i] += dot_ld(F + fl.T + (int64_t)k * i, 1, xs, k);
-  wave_sync();
-  for (int a = lane; a < k; a += 64) x[sk[a]] = xs[a];
-  for (int i = lane; i < r; i += 64) x[rd[i]] = xr[i];
-}
-
 }  // namespace
 
 void launch_reset(const DevState& s, hipStream_t st) {
@@ -3401,47 +3008,22 @@ void launch_root(const DevGeom& g, const DevTree& t, const DevState& s,
                  int n_roots, bool factor_lu, hipStream_t st) {
   k_active<<<n_roots, 64, 0, st>>>(t, s, 0);
   k_root<R, 256><<<dim3(n_roots, kRootSplit), 256, 0, st>>>(g, t, s);
-  k_root_inv<R><<<n_roots, kRootTR * kRootTC, 0, st>>>(s, factor_lu ? 1 : 0);
-  k_root_inv_blk<R><<<n_roots, kRootBlkMax, 0, st>>>(s, factor_lu ? 1 : 0);
-}
-
-template <typename R>
-void launch_sweep_up(const DevState& s, int start, int count, SolveVec v,
-                     bool use_Ut, bool diag, hipStream_t st) {
-  if (count <= 0) return;
-  k_sweep_up<R><<<count, 64, 0, st>>>(s, start, v, use_Ut ? 1 : 0, diag ? 1 : 0);
-}
-
-template <typename R>
-void launch_diag(const DevState& s, int start, int count, SolveVec v,
-                 hipStream_t st) {
-  if (count <= 0) return;
-  k_diag<R><<<count, 64, 0, st>>>(s, start, v);
-}
-
-template <typename R>
-void launch_sweep_down(const DevState& s, int start, int count, SolveVec v,
-                       hipStream_t st) {
-  if (count <= 0) return;
-  k_sweep_down<R><<<count, 64, 0, st>>>(s, start, v);
-}
-
-template <typename R>
-void launch_root_solve(const DevState& s, int n_roots, SolveVec v, hipStream_t st) {
-  k_root_solve<R><<<n_roots, 256, 0, st>>>(s, v);
-}
-
-template <typename R>
-void launch_fwd_up(const DevState& s, int start, int count, double* x, hipStream_t st) {
-  if (count > 0) k_fwd_up<R><<<count, 64, 0, st>>>(s, start, x);
-}
-template <typename R>
-void launch_fwd_root(const DevState& s, int n_roots, double* x, hipStream_t st) {
-  k_fwd_root<R><<<n_roots, 256, 0, st>>>(s, x);
-}
-template <typename R>
-void launch_fwd_down(const DevState& s, int start, int count, double* x, hipStream_t st) {
-  if (count > 0) k_fwd_down<R><<<count, 64, 0, st>>>(s, start, x);
+  if (!factor_lu) return;  // with holes the bordered system holds the root block
+  // A batch inverts the blocks that fit one workgroup's registers there (one
+  // workgroup per root fills the chip: 256 roots of about 130 DOFs take 253
+  // us, 1,721 us over many workgroups each); a few roots leave it idle and
+  // take the panels of k_inv_panel at every size (150 DOFs: 195 against 210
+  // us, 12 DOFs: 19 against 28 us).
+  const int one_wg = n_roots >= kRootBatch ? kRootRegMax : 0;
+  if (one_wg) k_root_inv<R><<<n_roots, kRootTR * kRootTC, 0, st>>>(s);
+  InvBlocks<R> blk;
+  blk.a = reinterpret_cast<R*>(s.root_mat);
+  blk.out = nullptr;
+  blk.stride = 2 * (int64_t)s.ncap * s.ncap;
+  blk.piv = s.root_piv;
+  blk.piv_stride = s.ncap + kRootPiv;
+  blk.extra = 0;
+  launch_block_inverse<R>(s, blk, n_roots, one_wg, s.ncap, st);
 }
 
 #define IEGPU_INSTANTIATE(R)                                                   \
@@ -3450,17 +3032,7 @@ void launch_fwd_down(const DevState& s, int start, int count, double* x, hipStre
                                        const LaunchCaps&, hipStream_t, int,    \
                                        hipStream_t);                           \
   template void launch_root<R>(const DevGeom&, const DevTree&,                \
-                               const DevState&, int, bool, hipStream_t);       \
-  template void launch_sweep_up<R>(const DevState&, int, int, SolveVec, bool, \
-                                   bool, hipStream_t);                         \
-  template void launch_diag<R>(const DevState&, int, int, SolveVec,           \
-                               hipStream_t);                                   \
-  template void launch_sweep_down<R>(const DevState&, int, int, SolveVec,     \
-                                     hipStream_t);                             \
-  template void launch_root_solve<R>(const DevState&, int, SolveVec, hipStream_t); \
-  template void launch_fwd_up<R>(const DevState&, int, int, double*, hipStream_t); \
-  template void launch_fwd_root<R>(const DevState&, int, double*, hipStream_t);    \
-  template void launch_fwd_down<R>(const DevState&, int, int, double*, hipStream_t);
+                               const DevState&, int, bool, hipStream_t);
 
 IEGPU_INSTANTIATE(double)
 IEGPU_INSTANTIATE(float)

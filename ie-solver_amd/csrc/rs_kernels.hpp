@@ -7,9 +7,10 @@
 
 namespace iegpu {
 
+// Right-hand sides on the device: entry (dof i, column c) at x[si i + sc c].
 struct SolveVec {
-  double* x;      // device, ldx x nrhs column-major
-  int64_t ldx;
+  double* x;
+  int64_t si, sc;
   int nrhs;
 };
 
@@ -76,15 +77,11 @@ void launch_root(const DevGeom& g, const DevTree& t, const DevState& s,
                  int n_roots, bool factor_lu, hipStream_t st);
 
 // Upward sweep of one level: x_r -= T^T x_s; x_s -= L x_r (or U^T x_r when
-// `use_Ut`); then x_r = X_rr^{-1} x_r when `diag`.
+// `use_Ut`); then x_r = X_rr^{-1} x_r when `diag`, written to dx (laid out
+// as x) instead when it is given.
 template <typename R>
 void launch_sweep_up(const DevState& s, int start, int count, SolveVec v,
-                     bool use_Ut, bool diag, hipStream_t st);
-
-// Block-diagonal X_rr^{-1} on the redundant rows of one level.
-template <typename R>
-void launch_diag(const DevState& s, int start, int count, SolveVec v,
-                 hipStream_t st);
+                     bool use_Ut, bool diag, hipStream_t st, double* dx = nullptr);
 
 // Downward sweep of one level: x_r -= U x_s; x_s -= T x_r.
 template <typename R>
@@ -94,6 +91,10 @@ void launch_sweep_down(const DevState& s, int start, int count, SolveVec v,
 // x(allskel) = A_root^{-1} x(allskel) for every root.
 template <typename R>
 void launch_root_solve(const DevState& s, int n_roots, SolveVec v, hipStream_t st);
+
+// dst (row-major n x h) <- src (column-major), or back.
+void launch_transpose(double* dst, const double* src, int64_t n, int h, bool to_rows,
+                      hipStream_t st);
 
 // Compressed forward apply b = A x in place on x (ndof), from the factors
 // and the X_rr / root blocks kept in fwd_pool / root_fwd: per level,

@@ -206,35 +206,6 @@ __global__ __launch_bounds__(kTile) void k_apply(DevGeom g, const double* x,
   }
 }
 
-// y[i] += sum_c U[i + ld c] a[c]  and  z[c] = sum_i P[i + ld c] x[i] - a[c].
-__global__ void k_border_apply_u(double* y, const double* U, const double* a,
-                                 int64_t ndof, int h) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ndof;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double acc = y[i];
-    for (int c = 0; c < h; c++) acc += U[i + ndof * c] * a[c];
-    y[i] = acc;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_border_apply_psi(const double* P,
-                                                          const double* x,
-                                                          const double* a,
-                                                          int64_t ndof, int h,
-                                                          double* z) {
-  __shared__ double red[256];
-  const int c = blockIdx.x;
-  double acc = 0;
-  for (int64_t i = threadIdx.x; i < ndof; i += 256) acc += P[i + ndof * c] * x[i];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) z[c] = red[0] - a[c];
-}
-
 // r = b - y (in place on y); partial sums of r^2 and b^2 per block.
 __global__ __launch_bounds__(256) void k_residual(const double* b, double* y,
                                                   int64_t n, double* partial) {
@@ -301,13 +272,6 @@ void launch_matvec(const DevGeom& g, const double* x, double* y, double* partial
                    hipStream_t st) {
   if (g.pde == kPdeStokes || g.pde == kPdeLaplaceNeumann) launch_wn_dot(g, x, partial, st);
   k_apply<<<(g.n_points + kTile - 1) / kTile, kTile, 0, st>>>(g, x, partial, y);
-}
-
-void launch_border_apply(const double* U, const double* PsiT, const double* x,
-                         const double* alpha, int64_t ndof, int h, double* y,
-                         double* z, hipStream_t st) {
-  k_border_apply_u<<<512, 256, 0, st>>>(y, U, alpha, ndof, h);
-  k_border_apply_psi<<<h, 256, 0, st>>>(PsiT, x, alpha, ndof, h, z);
 }
 
 }  // namespace iegpu

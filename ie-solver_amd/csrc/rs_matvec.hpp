@@ -28,9 +28,4 @@ void launch_residual(const double* b, double* y, int64_t n, double* partial,
 // y += x.
 void launch_axpy(double* y, const double* x, int64_t n, hipStream_t st);
 
-// Border of the multiply connected system: y += U alpha; z = Psi x - alpha.
-void launch_border_apply(const double* U, const double* PsiT, const double* x,
-                         const double* alpha, int64_t ndof, int h, double* y,
-                         double* z, hipStream_t st);
-
 }  // namespace iegpu

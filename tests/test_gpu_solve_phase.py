@@ -1,0 +1,101 @@
+"""The solve phase at the edges of its kernels' tiles: interior evaluation
+(128 targets and 512 sources per tile), the dense inverse of root blocks
+(panels of 16 columns), and multi-column solves (16 columns at a time)."""
+import numpy as np
+import pytest
+
+import geometry as G
+import iesolver
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+PDES = [iesolver.PDE_LAPLACE, iesolver.PDE_LAPLACE_NEUMANN, iesolver.PDE_STOKES]
+
+
+@pytest.mark.parametrize("pde", PDES)
+@pytest.mark.parametrize("n,nt", [(63, 1), (511, 127), (513, 129), (8193, 1000)])
+def test_evaluate_tile_edges(pde, n, nt):
+    g = G.star(n)
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g, pde)
+    mu = np.random.default_rng(n + nt).standard_normal(s.ndof)
+    tg = G.interior_points(nt, nt, radius=0.2)
+    u, uo = s.evaluate(tg, mu), oracle.evaluate(g, tg, mu, pde)
+    # both sums round each term by a few ulp: 8 eps per term against the sum
+    # of the terms' magnitudes, which the field of |mu| with every sign equal
+    # bounds by at most n max|term|; at these distances terms stay below
+    # w |mu| / (2 pi 0.04)
+    bound = 8 * 2.3e-16 * np.abs(mu).sum() * g["weights"].max() * 25 + 1e-300
+    assert np.abs(u - uo).max() <= bound
+
+
+def test_evaluate_far_and_nan_targets():
+    g = G.star(600)
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g)
+    mu = np.ones(600)
+    tg = G.interior_points(3, 130, radius=0.2)
+    u0 = s.evaluate(tg, mu)
+    tg[5] = [1e200, 0.5]   # |r|^2 overflows: the quotient is 0
+    tg[129] = [np.nan, 0.5]
+    u = s.evaluate(tg, mu)
+    assert u[5] == 0.0 and np.isnan(u[129])
+    keep = np.ones(130, bool)
+    keep[[5, 129]] = False
+    # the other targets: the division instead of the refined reciprocal
+    assert np.abs(u - u0)[keep].max() <= 600 * 8 * 2.3e-16 * g["weights"].max() * 25
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 192, 193, 500, 512])
+def test_root_inverse_panel_edges(n):
+    """A tree of one leaf: the root block is the whole operator."""
+    g = G.star(n, amp=0.1, k=3)
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g)
+    s.build_tree(512)
+    s.factor(1e-10)
+    f = np.random.default_rng(n).standard_normal(n)
+    mu, _ = s.solve(f)
+    K = oracle.dense_matrix(g)
+    # Gauss-Jordan with partial pivoting: n eps cond, with growth below 64
+    tol = 64 * n * 2.3e-16 * np.linalg.cond(K)
+    assert np.linalg.norm(mu - np.linalg.solve(K, f)) <= tol * np.linalg.norm(f)
+
+
+@pytest.mark.parametrize("problems", [15, 16])
+def test_batch_roots_either_inverse(problems):
+    """Batches below and from the size that inverts roots one per workgroup:
+    each problem as it is solved alone."""
+    geoms = [G.star(600 + 37 * p, k=3 + p % 5, amp=0.15) for p in range(problems)]
+    f = G.batch_data(geoms)
+    s = iesolver.RSSolver(0)
+    s.set_geometry_batch(geoms)
+    s.build_tree(64)
+    s.factor(1e-10)
+    mu, _ = s.solve(f)
+    for p in range(0, problems, 7):
+        sl = slice(s.dof_offsets[p], s.dof_offsets[p + 1])
+        a = iesolver.RSSolver(0)
+        a.set_geometry(geoms[p])
+        a.build_tree(64)
+        a.factor(1e-10)
+        mp, _ = a.solve(f[sl])
+        assert np.linalg.norm(mu[sl] - mp) <= 1e-12 * np.linalg.norm(mp)
+
+
+@pytest.mark.parametrize("pde,leaf", [(iesolver.PDE_LAPLACE, 64), (iesolver.PDE_STOKES, 300)])
+@pytest.mark.parametrize("prec", [iesolver.FP64, iesolver.FP32])
+def test_multi_column_tiles_equal_columns(pde, leaf, prec):
+    """2, 16, 17 and 33 columns (leaves of up to 300 DOFs: boxes too large for
+    16 columns in LDS): every column bit for bit as solved alone."""
+    g = G.star(3001)
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g, pde)
+    s.build_tree(leaf)
+    s.factor(1e-6, prec)
+    B = np.random.default_rng(2).standard_normal((s.ndof, 33))
+    for nrhs in (2, 16, 17, 33):
+        MU, _ = s.solve_many(B[:, :nrhs])
+        for j in {0, 1, nrhs // 2, nrhs - 1}:
+            assert np.array_equal(MU[:, j], s.solve(B[:, j])[0]), (nrhs, j)

@@ -622,13 +622,13 @@ void enqueue_factor(iegpu_ctx* c, double tol, const double* fb = nullptr,
       HIP_TRY(hipEventRecord(c->evs[1 + lv], st));
       HIP_TRY(hipStreamWaitEvent(st2, c->evs[1 + lv], 0));
     }
-    const bool fork = split && lv == 1;
+    const bool fork = split && lv == 1 && !(skip & kSkipDecBig);
     if (fork) {
       HIP_TRY(hipEventRecord(c->evs[T.n_levels + 2], st2));
       HIP_TRY(hipStreamWaitEvent(st, c->evs[T.n_levels + 2], 0));
     }
     c->prof.run(kStageDecouple, lv, st2, [&] {
-      launch_factor_stage<R>(kStageDecouple, g, t, s, lv, start, count, tol, c->caps, st2, 0,
+      launch_factor_stage<R>(kStageDecouple, g, t, s, lv, start, count, tol, c->caps, st2, skip,
                              fork ? st : nullptr);
     });
     // After the fork the ID stream joins the decouple chain's last work and
@@ -1532,7 +1532,7 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
     c->plan_on = plan_ok && c->plan_valid && key == c->plan_key;
     if (plan_ok && c->plan_mode == 2) {  // every list claimed empty (a test of the check)
       c->plan_skip.assign(kMaxLevels, kSkipAssemble | kSkipRegQrcp | kSkipReg8Qrcp | kSkipRid |
-                                          kSkipRidWide);
+                                          kSkipRidWide | kSkipDecBig);
       c->d_plan_skip.upload(c->plan_skip, c->stream);
       c->plan_on = true;
       c->plan_mode = 1;
@@ -1668,6 +1668,7 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
         if (cnt(kLstReg8) == 0) m |= kSkipReg8Qrcp;
         if (cnt(kLstRid) == wide) m |= kSkipRid;
         if (wide == 0) m |= kSkipRidWide;
+        if (cnt(kLstBig) == 0) m |= kSkipDecBig;
         c->plan_skip[lv] = m;
       }
       c->d_plan_skip.upload(c->plan_skip, c->stream);

@@ -28,7 +28,8 @@ enum : int {
   kErrWait = 128,      // a bounded wait between workgroups did not end
 };
 
-// Launch plan (DevState::plan_skip, per level): the ID-stage kernels not
+// Launch plan (DevState::plan_skip, per level): the ID-stage kernels and the
+// large-box decouple not
 // launched because their lists were empty in the last factorization of the
 // same inputs.  k_root checks every skipped list and raises kErrPlan.
 enum : int {
@@ -37,6 +38,7 @@ enum : int {
   kSkipReg8Qrcp = 4,   // k_rowcomp<8>, k_qrcp_id<8, 4, 16>
   kSkipRid = 8,        // k_rid (no 16- or 32-row sketch on the level)
   kSkipRidWide = 16,   // k_rid_wide (no 64-row sketch on the level)
+  kSkipDecBig = 32,    // k_decouple (no box above kSmallBox DOFs)
 };
 
 // How a box's interpolative decomposition runs.
@@ -67,7 +69,8 @@ enum : int {
   kLstRegHalf = 3,  // register QRCP, n <= 32 (8-wave workgroups)
   kLstRid = 4,      // randomized ID (sketch width > 0)
   kLstFallback = 5, // randomized mode: register-QRCP boxes without a successful sketch
-  kNumLists = 6,
+  kLstBig = 6,      // boxes above kSmallBox DOFs (k_decouple)
+  kNumLists = 7,
 };
 constexpr int kHalfCols = 32;
 
@@ -259,6 +262,7 @@ __device__ inline int plan_skippable(const DevState& s, int level) {
   if (list_count(s, level, kLstReg8) == 0) m |= kSkipReg8Qrcp;
   if (list_count(s, level, kLstRid) == wide) m |= kSkipRid;
   if (wide == 0) m |= kSkipRidWide;
+  if (list_count(s, level, kLstBig) == 0) m |= kSkipDecBig;
   return m;
 }
 __device__ inline int list_at(const DevState& s, int start, int L, int idx) {
@@ -748,6 +752,40 @@ __device__ const R* carried_block(const DevState& s, int c) {
   const int k = s.rank[c];
   if (k == 0) return F;
   return F + FacLayout::make(k, s.act_cnt[c] - k).S;
+}
+
+// An uncompressed box's carried block (n x n): its children's blocks on the
+// diagonal, or none when no child carries one.  All nt threads of the
+// workgroup; nothing is shared.
+template <typename R>
+__device__ inline void pass_children(const DevTree& t, const DevState& s, int b, int n, int nt) {
+  const int tid = threadIdx.x;
+  const R* S[4];
+  int at[4], cn[4];
+  bool any = false;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int c = (n == 0 || t.leaf[b]) ? -1 : t.child[4 * b + u];
+    S[u] = c >= 0 ? carried_block<R>(s, c) : nullptr;
+    cn[u] = c >= 0 ? s.out_cnt[c] : 0;
+    at[u] = c >= 0 ? s.chpos[4 * b + u] : 0;
+    any = any || S[u] != nullptr;
+  }
+  if (any) {
+    R* F = reinterpret_cast<R*>(s.fac_pool) + s.fac_off[b];
+    for (int64_t idx = tid; idx < (int64_t)n * n; idx += nt) {
+      const int i = (int)(idx % n), j = (int)(idx / n);
+      R v = R(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int a = i - at[u], c = j - at[u];
+        if (S[u] != nullptr && a >= 0 && a < cn[u] && c >= 0 && c < cn[u])
+          v = S[u][a + (int64_t)cn[u] * c];
+      }
+      F[idx] = v;
+    }
+  }
+  if (tid == 0) s.upd_kind[b] = any ? 1 : 0;
 }
 
 // Dense block (matrix, then its inverse) and pivots of root r (slot r).

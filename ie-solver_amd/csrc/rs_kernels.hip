@@ -283,8 +283,8 @@ __device__ inline bool rid_full_qrcp(const DevState& s, int b, int kind) {
 
 // Scanned per box: ID scratch, row-list and factor sizes, register-QRCP
 // and general-QRCP list entries, row-compression jobs, sketches, decouple
-// operands.
-constexpr int kScanQ = 12;
+// operands, boxes above kSmallBox DOFs.
+constexpr int kScanQ = 13;
 constexpr int kScanLd = 16;      // words per block in scan_blk
 constexpr int kScanMulti = 2048; // levels of at least this many boxes: three kernels
 
@@ -303,6 +303,7 @@ __device__ inline void scan_counts(const DevState& s, int b, int64_t (&own)[kSca
   own[9] += rid_full_qrcp(s, b, kind) ? 1 : 0;
   own[10] += s.dec_sz[b];
   own[11] += (s.sk_w[b] == kRidRowsW) ? 1 : 0;
+  own[12] += (s.act_cnt[b] > kSmallBox) ? 1 : 0;
 }
 
 // Box b's slots and list entries from the exclusive offsets off (advanced
@@ -340,6 +341,7 @@ __device__ inline void scan_place(const DevState& s, int b, int start, int level
   if (kind == kQrcpReg8 || kind == kQrcpStack8) lreg8[off[6]++] = b;
   if (s.sk_w[b] > 0) lrid[off[8]++] = b;
   if (rid_full_qrcp(s, b, kind)) lfb[off[9]++] = b;
+  if (s.act_cnt[b] > kSmallBox) s.lists[(int64_t)kLstBig * s.nbox + start + off[12]++] = b;
   const int nch = row_jobs(s, b);
   for (int q = 0; q < nch; q++) {
     jobs[2 * off[5]] = b;
@@ -359,6 +361,7 @@ __device__ inline void scan_finish(const DevState& s, int level, const int64_t* 
   list_slot(s, level, kLstRid)[0] = (int)tot[8];
   list_slot(s, level, kLstRid)[1] = (int)tot[11];  // of which 64-row sketches
   list_slot(s, level, kLstFallback)[0] = (int)tot[9];  // k_rid appends
+  list_slot(s, level, kLstBig)[0] = (int)tot[12];
   s.njobs[level] = (int)tot[5];
   int e = 0;
   if (ta > s.id_cap) {
@@ -425,7 +428,7 @@ __global__ __launch_bounds__(1024) void k_scan(DevState s, int start,
   const int tid = threadIdx.x;
   const int chunk = (count + 1023) / 1024;
   const int lo = min(count, tid * chunk), hi = min(count, lo + chunk);
-  int64_t own[kScanQ] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  int64_t own[kScanQ] = {};
   for (int i = lo; i < hi; i++) scan_counts(s, start + i, own);
   int64_t off[kScanQ];
   block_scan<1024>(own, off, wtot, tot);
@@ -445,7 +448,7 @@ __global__ __launch_bounds__(256) void k_scan_blocks(DevState s, int start, int 
   __shared__ int64_t wtot[kScanQ][4];
   __shared__ int64_t tot[kScanQ];
   const int i = blockIdx.x * 256 + threadIdx.x;
-  int64_t own[kScanQ] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  int64_t own[kScanQ] = {};
   if (i < count) scan_counts(s, start + i, own);
   int64_t off[kScanQ];
   block_scan<256>(own, off, wtot, tot);
@@ -458,7 +461,7 @@ __global__ __launch_bounds__(1024) void k_scan_totals(DevState s, int nblk, int 
   const int tid = threadIdx.x;
   const int chunk = (nblk + 1023) / 1024;
   const int lo = min(nblk, tid * chunk), hi = min(nblk, lo + chunk);
-  int64_t own[kScanQ] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  int64_t own[kScanQ] = {};
   for (int j = lo; j < hi; j++)
 #pragma unroll
     for (int q = 0; q < kScanQ; q++) own[q] += s.scan_blk[(int64_t)j * kScanLd + q];
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(256) void k_scan_place(DevState s, int start, int c
   __shared__ int64_t wtot[kScanQ][4];
   __shared__ int64_t tot[kScanQ];
   const int i = blockIdx.x * 256 + threadIdx.x;
-  int64_t own[kScanQ] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  int64_t own[kScanQ] = {};
   if (i < count) scan_counts(s, start + i, own);
   int64_t off[kScanQ];
   block_scan<256>(own, off, wtot, tot);
@@ -2340,7 +2343,11 @@ __global__ __launch_bounds__(256) void k_decouple_small(DevGeom g, DevTree t,
   const int tid = threadIdx.x;
   if (!pools_ok(s) || box_clean(s, b)) return;
   const int n = s.act_cnt[b], k = s.rank[b];
-  if (n <= NMIN || n > NMAX || k == 0) return;  // the other class's or k_decouple's box
+  if (n > NMAX || (n <= NMIN && (NMIN > 0 || n > 0))) return;  // another kernel's box
+  if (k == 0) {
+    pass_children<R>(t, s, b, n, NT);
+    return;
+  }
   load_child_blocks<R>(t, s, b, n, chS, chN, pch, ploc, NT);
   const int* act = s.act_list + (int64_t)b * s.ncap;
   for (int i = tid; i < n; i += NT) {
@@ -2400,16 +2407,17 @@ __global__ __launch_bounds__(256) void k_decouple_small(DevGeom g, DevTree t,
   if (tid == 0) s.upd_kind[b] = 1;
 }
 
-// Every other box: uncompressed boxes pass their children's blocks on;
-// compressed boxes with |active| > 64 keep P and X_rr in LDS when they fit
-// and in the box's scratch slot otherwise.  Few boxes of a level are
-// these, so a small grid walks the level (the others are skipped after
-// two loads) instead of one workgroup per box.
+// The boxes above kSmallBox DOFs, walked by a small grid from their list
+// (few boxes of a level are these; walking the whole level for them took
+// 167 us per factorization at N = 262,144 against 26, and 7.8 ms against 2.3
+// for a batch of 256 problems): compressed ones keep P and X_rr in LDS when they fit and in the
+// box's scratch slot otherwise, uncompressed ones pass their children's
+// blocks on.
 constexpr int kDecGeoMax = 96;
 
 template <typename R, int NT>
 __global__ __launch_bounds__(NT) void k_decouple(DevGeom g, DevTree t,
-                                                 DevState s, int start, int count) {
+                                                 DevState s, int start, int level) {
   // 128 KB: P, X_rr, K_rs and K_sr of a box up to 90 DOFs (FP64) stay in
   // LDS; the Schur products are then LDS-bound, not bound by L2 latency.
   constexpr int kLdsElems = 131072 / sizeof(R);
@@ -2425,35 +2433,24 @@ __global__ __launch_bounds__(NT) void k_decouple(DevGeom g, DevTree t,
 
   const int tid = threadIdx.x;
   if (!pools_ok(s)) return;
-  for (int bi = blockIdx.x; bi < count; bi += gridDim.x) {
-  const int b = start + bi;
-  if (box_clean(s, b)) continue;
+  const int nl = list_count(s, level, kLstBig);
+  for (int bi = blockIdx.x; bi < nl; bi += gridDim.x) {
+  const int b = list_at(s, start, kLstBig, bi);
   const int n = s.act_cnt[b];
-  if (n == 0) {
-    if (tid == 0) s.upd_kind[b] = 0;
+  if (s.rank[b] == 0) {
+    pass_children<R>(t, s, b, n, NT);
     continue;
   }
-  if (n <= kSmallBox && s.rank[b] > 0) continue;  // k_decouple_small's box
   __syncthreads();  // the previous box's LDS
   load_child_blocks<R>(t, s, b, n, chS, chN, pch, ploc, NT);
   __syncthreads();
   ChildUpdates<R> upd;
   upd.S = chS;
   upd.N = chN;
-  bool any = false;
-  for (int u = 0; u < 4; u++) any = any || chS[u] != nullptr;
   upd.pch = pch;
   upd.ploc = ploc;
   const int k = s.rank[b];
   R* F = reinterpret_cast<R*>(s.fac_pool) + s.fac_off[b];
-  if (k == 0) {
-    if (any) {
-      for (int64_t idx = tid; idx < (int64_t)n * n; idx += NT)
-        F[idx] = upd((int)(idx % n), (int)(idx / n));
-    }
-    if (tid == 0) s.upd_kind[b] = any ? 1 : 0;
-    continue;
-  }
   const int r = n - k;
   const FacLayout fl = FacLayout::make(k, r);
   const int* act = s.act_list + (int64_t)b * s.ncap;
@@ -2993,10 +2990,13 @@ void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
       // own stream: the two kernels touch different boxes), there with
       // 1024 threads (level 1's two 84-DOF boxes: the P fill 47k -> 16k
       // cycles, 12 % less in all)
-      if (st_big)
-        k_decouple<R, 1024><<<min(count, 512), 1024, 0, st_big>>>(g, t, s, start, count);
-      else
-        k_decouple<R, 256><<<min(count, 512), 256, 0, st>>>(g, t, s, start, count);
+      if (skip & kSkipDecBig) {
+        // no such box on this level (launch plan)
+      } else if (st_big) {
+        k_decouple<R, 1024><<<min(count, 512), 1024, 0, st_big>>>(g, t, s, start, level);
+      } else {
+        k_decouple<R, 256><<<min(count, 512), 256, 0, st>>>(g, t, s, start, level);
+      }
       break;
     default:
       break;

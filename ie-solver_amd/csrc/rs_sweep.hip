@@ -137,7 +137,11 @@ __global__ __launch_bounds__(64, (NB <= 2 ? 4 : 2)) void k_decouple_sweep(
   const int lane = threadIdx.x;
   if (!pools_ok(s) || box_clean(s, b)) return;
   const int n = s.act_cnt[b], k = s.rank[b];
-  if (n <= nmin || n > NMAX || k == 0) return;  // another launch's box
+  if (n > NMAX || (n <= nmin && (nmin > 0 || n > 0))) return;  // another launch's box
+  if (k == 0) {
+    pass_children<R>(t, s, b, n, 64);
+    return;
+  }
   const int r = n - k;
   const int* act = s.act_list + (int64_t)b * s.ncap;
   R* F = reinterpret_cast<R*>(s.fac_pool) + s.fac_off[b];

@@ -243,7 +243,7 @@ struct iegpu_ctx {
   int64_t id_cap = 0, row_cap = 0, fac_cap = 0, dec_cap = 0;
   // randomized ID
   int rid_mode = 0, rid_width = 0;
-  DevBuf<double> d_omega, d_omega_w;
+  DevBuf<double> d_omega, d_omega_w, d_omega_b;
   // factorization replayed as a captured HIP graph (iegpu_set_graphs)
   bool use_graphs = false;
   hipGraphExec_t fgraph = nullptr;
@@ -409,6 +409,7 @@ struct iegpu_ctx {
     s.rid_done = s_rid_done.p;
     s.omega = d_omega.p;
     s.omega_w = d_omega_w.p;
+    s.omega_b = d_omega_b.p;
     s.rank_model = d_model.p;
     s.rid_margin = rid_margin;
     s.feat = record_features ? d_feat.p : nullptr;
@@ -614,7 +615,8 @@ void enqueue_factor(iegpu_ctx* c, double tol, const double* fb = nullptr,
     const int start = T.level_start[lv];
     const int count = T.level_start[lv + 1] - start;
     const int skip = c->plan_on ? c->plan_skip[lv] : 0;
-    for (int stage = 0; stage < kStageDecouple; stage++)
+    // the general QRCP's matrices after the sketches, for the boxes none took
+    for (int stage : {kStageActive, kStageRows, kStageScan, kStageRid, kStageAssemble, kStageQrcp})
       c->prof.run(stage, lv, st, [&] {
         launch_factor_stage<R>(stage, g, t, s, lv, start, count, tol, c->caps, st, skip);
       });
@@ -1509,6 +1511,9 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
       const int64_t nw = (int64_t)kRidTableRowsW * kRidRowsW;
       c->d_omega_w.alloc(nw);
       launch_gaussian(c->d_omega_w.p, nw, 0x5EEDull, c->stream);
+      const int64_t nb = (int64_t)kRidTableRowsW * kRidRowsB;
+      c->d_omega_b.alloc(nb);
+      launch_gaussian(c->d_omega_b.p, nb, 0x5EEDull, c->stream);
     }
     // After iegpu_update_geometry on the same tree, only the marked boxes
     // are re-factored (same tolerance and precision as the kept factors).
@@ -1531,8 +1536,7 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
     const bool plan_ok = !c->inc_run && !c->use_graphs && c->plan_mode != 0;
     c->plan_on = plan_ok && c->plan_valid && key == c->plan_key;
     if (plan_ok && c->plan_mode == 2) {  // every list claimed empty (a test of the check)
-      c->plan_skip.assign(kMaxLevels, kSkipAssemble | kSkipRegQrcp | kSkipReg8Qrcp | kSkipRid |
-                                          kSkipRidWide | kSkipDecBig);
+      c->plan_skip.assign(kMaxLevels, kSkipAll);
       c->d_plan_skip.upload(c->plan_skip, c->stream);
       c->plan_on = true;
       c->plan_mode = 1;
@@ -1661,13 +1665,13 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
       for (int lv = 1; lv < c->tree.n_levels; lv++) {
         auto cnt = [&](int L) { return lc[(size_t)2 * (lv * kNumLists + L)]; };
         const int reg = c->rid_mode != 0 ? cnt(kLstFallback) : cnt(kLstReg) + cnt(kLstRegHalf);
-        const int wide = lc[(size_t)2 * (lv * kNumLists + kLstRid) + 1];
         int m = 0;
         if (cnt(kLstLds) == 0) m |= kSkipAssemble;
         if (reg == 0) m |= kSkipRegQrcp;
         if (cnt(kLstReg8) == 0) m |= kSkipReg8Qrcp;
-        if (cnt(kLstRid) == wide) m |= kSkipRid;
-        if (wide == 0) m |= kSkipRidWide;
+        if (cnt(kLstRid) == 0) m |= kSkipRid;
+        if (cnt(kLstRidWide) == 0) m |= kSkipRidWide;
+        if (cnt(kLstRidBig) == 0) m |= kSkipRidBig;
         if (cnt(kLstBig) == 0) m |= kSkipDecBig;
         c->plan_skip[lv] = m;
       }

@@ -39,6 +39,8 @@ enum : int {
   kSkipRid = 8,        // k_rid (no 16- or 32-row sketch on the level)
   kSkipRidWide = 16,   // k_rid_wide (no 64-row sketch on the level)
   kSkipDecBig = 32,    // k_decouple (no box above kSmallBox DOFs)
+  kSkipRidBig = 64,    // k_rid_big_* (no 128-row sketch on the level)
+  kSkipAll = 127,
 };
 
 // How a box's interpolative decomposition runs.
@@ -67,10 +69,12 @@ enum : int {
   kLstLds = 1,      // general QRCP (kQrcpLds)
   kLstReg8 = 2,     // wide register QRCP (kQrcpReg8, kQrcpStack8)
   kLstRegHalf = 3,  // register QRCP, n <= 32 (8-wave workgroups)
-  kLstRid = 4,      // randomized ID (sketch width > 0)
+  kLstRid = 4,      // randomized ID, 16- and 32-row sketches
   kLstFallback = 5, // randomized mode: register-QRCP boxes without a successful sketch
   kLstBig = 6,      // boxes above kSmallBox DOFs (k_decouple)
-  kNumLists = 7,
+  kLstRidWide = 7,  // randomized ID, 64-row sketches
+  kLstRidBig = 8,   // randomized ID, 128-row sketches
+  kNumLists = 9,
 };
 constexpr int kHalfCols = 32;
 
@@ -82,14 +86,23 @@ constexpr int kRidRows = 32;
 constexpr int kRidOver = 6;
 constexpr int kRidMaxNear = 256;
 constexpr int kRidTableRows = 2 * kRidMaxNear + 4 * kNumProxy;  // Omega rows
-// The wide form for the few large boxes of the top levels (level <=
-// kRidWideTop): a sketch of kRidRowsW rows, up to kRidWideCols columns and
-// kRidMaxNearW row DOFs, with its own Gaussian table.
+// The wide form for larger boxes and ranks: a sketch of kRidRowsW rows, up
+// to kRidWideCols columns and kRidMaxNearW row DOFs, with its own Gaussian
+// table.
 constexpr int kRidRowsW = 64;
 constexpr int kRidWideCols = 128;
 constexpr int kRidMaxNearW = 1280;  // the level-1/2 row sets of small problems in a batch
-constexpr int kRidWideTop = 4;
 constexpr int kRidTableRowsW = 2 * kRidMaxNearW + 4 * kNumProxy;
+// The big form for the boxes of the top levels (level <= kRidBigTop) past
+// that: kRidRowsB rows, up to kRidBigCols columns.
+constexpr int kRidRowsB = 128;
+constexpr int kRidBigCols = 256;
+constexpr int kRidBigTop = 4;
+constexpr int kRidBigParts = 4;  // row parts of its sketch, a workgroup each
+// Its scratch: the parts' sketches and the rows of R, kRidRowsB x n16 each.
+__host__ __device__ inline int64_t rid_big_scratch(int n) {
+  return (int64_t)(kRidBigParts + 1) * kRidRowsB * ((n + 15) / 16 * 16);
+}
 
 // Rank model: an MLP kFeat -> kHid (tanh) -> kHid (tanh) -> 1 on per-box
 // features, predicting the ID rank.  Parameter blob (floats): feature
@@ -206,6 +219,7 @@ struct DevState {
   int* rid_done;       // per box: 1 once the randomized ID succeeded
   const double* omega; // kRidTableRows x kRidRows Gaussian table (row-major)
   const double* omega_w;  // kRidTableRowsW x kRidRowsW table of the wide form
+  const double* omega_b;  // kRidTableRowsW x kRidRowsB table of the big form
   const float* rank_model;  // kMlpLen floats (rid_mode 2)
   int rid_margin;           // ranks added to the prediction before sizing
   float* feat;              // kFeat per box, written by k_rows when non-null
@@ -254,14 +268,13 @@ __device__ inline int plan_skippable(const DevState& s, int level) {
   const int reg = s.rid_mode != 0 ? list_count(s, level, kLstFallback)
                                   : list_count(s, level, kLstReg) +
                                         list_count(s, level, kLstRegHalf);
-  // kLstRid's second slot int counts the level's 64-row sketches.
-  const int wide = list_slot(s, level, kLstRid)[1];
   int m = 0;
   if (list_count(s, level, kLstLds) == 0) m |= kSkipAssemble;
   if (reg == 0) m |= kSkipRegQrcp;
   if (list_count(s, level, kLstReg8) == 0) m |= kSkipReg8Qrcp;
-  if (list_count(s, level, kLstRid) == wide) m |= kSkipRid;
-  if (wide == 0) m |= kSkipRidWide;
+  if (list_count(s, level, kLstRid) == 0) m |= kSkipRid;
+  if (list_count(s, level, kLstRidWide) == 0) m |= kSkipRidWide;
+  if (list_count(s, level, kLstRidBig) == 0) m |= kSkipRidBig;
   if (list_count(s, level, kLstBig) == 0) m |= kSkipDecBig;
   return m;
 }

@@ -15,6 +15,8 @@ struct SolveVec {
 };
 
 void launch_reset(const DevState& s, hipStream_t st);
+// Active lists of boxes start .. start + count - 1 from their children's.
+void launch_active(const DevTree& t, const DevState& s, int start, int count, hipStream_t st);
 // Standard normal table (n entries) for the randomized-ID sketches.
 void launch_gaussian(double* out, int64_t n, uint64_t seed, hipStream_t st);
 
@@ -69,6 +71,25 @@ void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
 template <typename R>
 void launch_decouple_sweep(const DevGeom& g, const DevTree& t, const DevState& s, int start,
                            int count, hipStream_t st);
+
+// One level's randomized ID (rs_rid.hip), pivoted-QR ID (rs_qrcp.hip) and
+// decouple of the workgroup forms (rs_decouple.hip); `skip`, `st_big` as in
+// launch_factor_stage.
+template <typename R>
+void launch_rid(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
+                int count, double tol, hipStream_t st, int skip);
+template <typename R>
+void launch_qrcp(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
+                 int count, double tol, const LaunchCaps& caps, hipStream_t st, int skip);
+template <typename R>
+void launch_decouple(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
+                     int count, const LaunchCaps& caps, hipStream_t st, int skip,
+                     hipStream_t st_big);
+
+// Randomized ID of a level's kLstRidBig boxes (rs_rid_big.hip).
+template <typename R>
+void launch_rid_big(const DevGeom& g, const DevTree& t, const DevState& s, int start, int level,
+                    int count, double tol, hipStream_t st);
 
 // Roots (slots 0 .. n_roots-1, one per problem): active list, dense
 // skeleton block, inverse.

@@ -394,8 +394,12 @@ int iegpu_autotune(iegpu_ctx* ctx, double id_tol, int precision, int reps,
  * box from the rank model, iegpu_set_rank_model) with the
  * same cut applied to the sketch's R, |R_jj| scaled by 2 sqrt(l / (l - j))
  * (a sketch keeps l - j dimensions at step j); a box whose sketch shows no
- * cut within l - 6 pivots falls back to the full QRCP.  No reference
- * counterpart (the reference always factors the full ID matrix). */
+ * cut within l - 6 pivots falls back to the full QRCP.  Larger boxes (up
+ * to 128 active DOFs and 1,280 near-field row DOFs; with the rank model on
+ * every level, else on the top four) take a 64-row sketch, and on the top
+ * four levels boxes of up to 256 DOFs, or whose 64-row sketch shows no cut,
+ * a 128-row one.  No reference counterpart (the reference always factors
+ * the full ID matrix). */
 enum { IEGPU_ID_QRCP = 0, IEGPU_ID_RANDOMIZED = 1 };
 int iegpu_set_id_method(iegpu_ctx* ctx, int method, int sketch_rows);
 
@@ -441,8 +445,9 @@ int iegpu_rank_model_train(iegpu_ctx* ctx, const float* X, const float* y, int n
 int iegpu_rank_model_grad(iegpu_ctx* ctx, const float* model, const float* X, const float* y,
                           int n, float* grad, float* loss);
 /* Model used by iegpu_set_id_method(ctx, IEGPU_ID_RANDOMIZED, 0): a box's
- * sketch has 16 rows if (predicted rank + margin) <= 10, 32 rows if it is
- * <= 26, and none otherwise (the full QRCP takes the box directly). */
+ * sketch has 16 rows if (predicted rank + margin) <= 10 and 32 rows if it
+ * is <= 26; past that, and for larger boxes, see IEGPU_ID_RANDOMIZED (a box
+ * that none of the sketches fits goes straight to the full QRCP). */
 int iegpu_set_rank_model(iegpu_ctx* ctx, const float* model, int margin);
 
 #ifdef __cplusplus

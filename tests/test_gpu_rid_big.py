@@ -1,0 +1,57 @@
+"""The 128-row sketch of the top levels' large boxes, and the 64-row sketch
+walked over a list on levels of many boxes: backward error and ranks at the
+edges of their column tiles."""
+import os
+
+import numpy as np
+import pytest
+
+import geometry as G
+import iesolver
+
+pytestmark = pytest.mark.gpu
+
+MODEL = os.path.join(os.path.dirname(iesolver.__file__), "rank_model_default.npy")
+
+
+def _solver(g, pde, leaf, learned, prec=iesolver.FP64, tol=1e-10):
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g, pde)
+    s.build_tree(leaf)
+    if learned:
+        s.set_rank_model(np.load(MODEL), margin=3)
+        s.set_id_method(iesolver.ID_RANDOMIZED, 0)
+    s.factor(tol, prec)
+    return s
+
+
+# leaves of up to `leaf` DOFs on levels 1 to 4 make boxes of 65 to 256 columns
+@pytest.mark.parametrize("n,leaf,pde", [
+    (700, 128, iesolver.PDE_STOKES), (1100, 150, iesolver.PDE_STOKES),
+    (1500, 256, iesolver.PDE_STOKES), (3000, 300, iesolver.PDE_LAPLACE_NEUMANN),
+    (2049, 64, iesolver.PDE_STOKES), (16385, 64, iesolver.PDE_STOKES)])
+def test_large_box_sketches(n, leaf, pde):
+    tol = 1e-10
+    g = G.star(n, k=5)
+    s = _solver(g, pde, leaf, True)
+    b = np.random.default_rng(n).standard_normal(s.ndof)
+    x, _ = s.solve(b)
+    y, _ = s.apply(x)
+    # the backward error bar of every form (ie_solver_test.cpp:84-95)
+    assert np.linalg.norm(y - b) <= 50 * tol * np.linalg.norm(b)
+    info = s.box_info()
+    big = (info["n_active"] > 64) & (info["level"] > 0)
+    plain = _solver(g, pde, leaf, False).box_info()
+    assert big.any()
+    # first-level differences compound upward: the sketch's rank of a leaf
+    # stays within three of the full pivoted QR's
+    leafbig = big & (info["is_leaf"] == 1) & (info["rank"] > 0) & (plain["rank"] > 0)
+    assert np.abs(info["rank"] - plain["rank"])[leafbig].max(initial=0) <= 3
+
+
+def test_large_box_sketch_fp32():
+    g = G.star(1100, k=5)
+    s = _solver(g, iesolver.PDE_STOKES, 150, True, iesolver.FP32, 1e-5)
+    b = np.random.default_rng(3).standard_normal(s.ndof)
+    x, _, it, res = s.solve_refined(b, 1e-12, 10)
+    assert res <= 1e-12

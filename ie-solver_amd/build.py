@@ -19,8 +19,8 @@ HIP_FLAGS = [
     # keep hipcc from emitting packed FP32 arithmetic
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-HIP_SOURCES = ["rs_kernels.hip", "rs_qrcp.hip", "rs_rid.hip", "rs_rid_big.hip", "rs_decouple.hip",
-               "rs_sweep.hip", "rs_inv.hip", "rs_solve.hip",
+HIP_SOURCES = ["rs_kernels.hip", "rs_qrcp.hip", "rs_gram.hip", "rs_rid.hip", "rs_rid_big.hip",
+               "rs_decouple.hip", "rs_sweep.hip", "rs_inv.hip", "rs_solve.hip",
                "rs_holes.hip", "rs_eval.hip", "rs_matvec.hip", "rs_fmm.hip", "rs_mlp.hip", "capi.cpp"]
 HOST_SOURCES = ["tree.cpp", "fmm_tree.cpp"]
 

@@ -243,6 +243,7 @@ struct iegpu_ctx {
   int64_t id_cap = 0, row_cap = 0, fac_cap = 0, dec_cap = 0;
   // randomized ID
   int rid_mode = 0, rid_width = 0;
+  int gram = 0;  // of the factorization being enqueued
   DevBuf<double> d_omega, d_omega_w, d_omega_b;
   // factorization replayed as a captured HIP graph (iegpu_set_graphs)
   bool use_graphs = false;
@@ -405,6 +406,7 @@ struct iegpu_ctx {
     s.root_fwd = keep_operator ? s_root_fwd.p : nullptr;
     s.rid_mode = rid_mode;
     s.rid_width = rid_width;
+    s.gram = gram;
     s.sk_w = s_sk_w.p;
     s.rid_done = s_rid_done.p;
     s.omega = d_omega.p;
@@ -1445,7 +1447,7 @@ int iegpu_id_stats(iegpu_ctx* c, int* n_sketched, int* n_fallback, double* sketc
       HIP_TRY(hipMemcpy(n.data(), c->s_act_cnt.p, sizeof(int) * nb, hipMemcpyDeviceToHost));
       for (int b = lo; b < nb; b++) {
         if (w[b] <= 0) continue;
-        if (d[b]) ns++;
+        if (d[b] == kIdSketch) ns++;
         else nf++;
         fl += 2.0 * w[b] * m[b] * (16 * ((n[b] + 15) / 16));
       }
@@ -1496,6 +1498,7 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
       c->s_dec_pool.release();
     }
     c->precision = precision;
+    c->gram = precision == IEGPU_FP32 && id_tol >= kGramTol ? 1 : 0;
     if (c->ncap == 0) c->ncap = 256;
     // Register-QRCP boxes need no ID scratch; the pool holds the few
     // row-compressed or general-QRCP boxes of one level (grown to the

@@ -78,6 +78,21 @@ enum : int {
 };
 constexpr int kHalfCols = 32;
 
+// DevState::rid_done values: the ID is still the full QRCP's, came from a
+// sketch, or from the Gram matrix.
+enum : int { kIdOpen = 0, kIdSketch = 1, kIdGram = 2 };
+
+// FP32 factorizations at this tolerance or above take their full IDs from
+// FP64 Gram matrices (rs_gram.hip), whose R is good to 1e-8 of its norm.
+// Below, the FP32 QR's own noise (1e-7) decides the ranks: at 2e-7 it keeps
+// 1 to 5 % more columns and the Gram form's backward error was larger.
+constexpr double kGramTol = 5e-7;
+// Scratch (in FP32 elements) of a box above 64 DOFs there: G and R.
+__host__ __device__ inline int64_t gram_scratch(int n) {
+  const int64_t n16 = (n + 15) / 16 * 16;
+  return 4 * n16 * n16;
+}
+
 // Randomized ID: a Gaussian sketch of at most kRidRows rows (a multiple of
 // 16 per box); a cut must show within kRidRows - kRidOver pivots, else the
 // box goes through the full QRCP.  Boxes with at most kRidMaxNear row DOFs
@@ -215,8 +230,9 @@ struct DevState {
   // eligible box; 2: width from the rank model).
   int rid_mode;
   int rid_width;
+  int gram;            // 1: full IDs from Gram matrices
   int* sk_w;           // per box: sketch rows (0: full QRCP)
-  int* rid_done;       // per box: 1 once the randomized ID succeeded
+  int* rid_done;       // per box: kIdOpen, kIdSketch or kIdGram
   const double* omega; // kRidTableRows x kRidRows Gaussian table (row-major)
   const double* omega_w;  // kRidTableRowsW x kRidRowsW table of the wide form
   const double* omega_b;  // kRidTableRowsW x kRidRowsB table of the big form

@@ -221,6 +221,8 @@ __global__ __launch_bounds__(64) void k_rows(DevGeom g, DevTree t, DevState s,
     // those a failed 64-row sketch passes on to it.
     if (w == kRidRowsB || (w == kRidRowsW && eligb))
       s.id_sz[b] = max(s.id_sz[b], rid_big_scratch(n));
+    if (s.gram && n > kRegMaxCols) s.id_sz[b] = max(s.id_sz[b], gram_scratch(n));
+    s.id_sz[b] = (s.id_sz[b] + 3) & ~int64_t(3);  // slots hold doubles
   }
   // Until its ID succeeds a box passes its active DOFs on uncompressed:
   // boxes a failed (retried) attempt never reaches still hold a consistent
@@ -532,13 +534,22 @@ void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
       }
       break;
     case kStageAssemble:
-      if (!(skip & kSkipAssemble))
+      if (!(skip & kSkipAssemble) && !s.gram)
         k_assemble<R><<<min(count, caps.assemble), 256, 0, st>>>(g, t, s, start, level);
       break;
     case kStageRid:
       if (s.rid_mode != 0) launch_rid<R>(g, t, s, level, start, count, tol, st, skip);
       break;
     case kStageQrcp:
+      if constexpr (sizeof(R) == 4) {
+        if (s.gram) {
+          launch_gram<R>(g, t, s, level, start, count, tol, st, skip);
+          if (skip & kSkipAssemble) break;
+          // the boxes too large for it
+          k_assemble<R><<<min(count, caps.assemble), 256, 0, st>>>(g, t, s, start, level);
+          skip |= kSkipRegQrcp | kSkipReg8Qrcp;
+        }
+      }
       launch_qrcp<R>(g, t, s, level, start, count, tol, caps, st, skip);
       break;
     case kStageDecouple:

@@ -81,6 +81,11 @@ void launch_rid(const DevGeom& g, const DevTree& t, const DevState& s, int level
 template <typename R>
 void launch_qrcp(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
                  int count, double tol, const LaunchCaps& caps, hipStream_t st, int skip);
+// The full IDs of an FP32 level from Gram matrices (rs_gram.hip), but for
+// boxes above 256 DOFs or 2,048 row DOFs.
+template <typename R>
+void launch_gram(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
+                 int count, double tol, hipStream_t st, int skip);
 template <typename R>
 void launch_decouple(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
                      int count, const LaunchCaps& caps, hipStream_t st, int skip,

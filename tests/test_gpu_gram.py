@@ -1,0 +1,53 @@
+"""FP32 factorizations' IDs from FP64 Gram matrices, at the edges of the
+column tiles and on either side of the tolerance that selects them: backward
+error, and ranks against the FP64 factorization's pivoted QR."""
+import numpy as np
+import pytest
+
+import geometry as G
+import iesolver
+
+pytestmark = pytest.mark.gpu
+
+PDES = [iesolver.PDE_LAPLACE, iesolver.PDE_LAPLACE_NEUMANN, iesolver.PDE_STOKES]
+
+
+def _factored(g, pde, leaf, tol, prec):
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g, pde)
+    s.build_tree(leaf)
+    s.factor(tol, prec)
+    return s
+
+
+# leaves of up to 32, 33, 64, 65, 128 and 300 DOFs
+@pytest.mark.parametrize("pde", PDES)
+@pytest.mark.parametrize("n,leaf", [(400, 32), (401, 34), (1000, 64), (1003, 66), (1501, 128),
+                                    (3000, 300)])
+def test_gram_ids(pde, n, leaf):
+    tol = 1e-6
+    g = G.star(n, k=5)
+    s = _factored(g, pde, leaf, tol, iesolver.FP32)
+    b = np.random.default_rng(n).standard_normal(s.ndof)
+    x, _ = s.solve(b)
+    y, _ = s.apply(x)
+    # the backward error bar of every form (ie_solver_test.cpp:84-95)
+    assert np.linalg.norm(y - b) <= 50 * tol * np.linalg.norm(b)
+    i32 = s.box_info()
+    # The cut lies at 0.8 tol of the diagonal, which the Gram matrix gives to
+    # 1e-8 of its norm (1 % of it): on the deepest level, where a leaf's ID
+    # matrix is the same in every factorization, the rank lies between the
+    # pivoted QR's at tolerances a little either side.
+    lo, hi = (_factored(g, pde, leaf, t, iesolver.FP64).box_info() for t in (0.85e-6, 0.75e-6))
+    deep = (lo["level"] == lo["level"].max()) & (lo["rank"] > 0)
+    assert np.all(i32["rank"][deep] >= lo["rank"][deep])
+    assert np.all(i32["rank"][deep] <= hi["rank"][deep])
+
+
+@pytest.mark.parametrize("tol", [4.9e-7, 5e-7])
+def test_gram_tolerance_limit(tol):
+    g = G.star(2000)
+    s = _factored(g, iesolver.PDE_LAPLACE, 64, tol, iesolver.FP32)
+    b = np.random.default_rng(1).standard_normal(s.ndof)
+    x, _, it, res = s.solve_refined(b, 1e-12, 10)
+    assert res <= 1e-12 and it <= 5

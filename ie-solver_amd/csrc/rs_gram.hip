@@ -33,8 +33,8 @@ namespace {
 // k_gram_blocks / k_gram_chol: 65 to 256 columns, a workgroup per 32 x 32
 // block of G, then one per box.
 // Entry evaluation and its MFMAs bound k_gram_id, the latency of the steps
-// k_gram_chol.  Stokes with 8 holes, 131,072 points, plain FP32 at 1e-6: 4.9
-// ms per factorization (k_gram_id 2.5, k_gram_blocks 0.1, k_gram_chol 1.5)
+// k_gram_chol.  Stokes with 8 holes, 131,072 points, plain FP32 at 1e-6: 4.2
+// ms per factorization (k_gram_id 2.5, k_gram_blocks 0.15, k_gram_chol 1.5)
 // against 25.1 for row compression, register and general QR and assembly.
 // ---------------------------------------------------------------------------
 
@@ -52,34 +52,6 @@ struct RowItems {
   double x[kItems], y[kItems], n1[kItems], n2[kItems], w[kItems], k[kItems];
   int c[kItems];
 };
-
-// Entries of row point q and column c in both directions: et = K(q, c), es =
-// K(c, q) (rs_device.hpp's kernels).  NEAR: boundary DOFs, which may coincide.
-template <int PDE, bool NEAR>
-__device__ __forceinline__ void pair_entries(const DofGeo& q, const DofGeo& c, double& et,
-                                             double& es) {
-  const double r0 = q.x - c.x, r1 = q.y - c.y;
-  const double inv = recip(fma(r0, r0, r1 * r1));
-  const double rc = fma(r0, c.n1, r1 * c.n2), rq = fma(r0, q.n1, r1 * q.n2);
-  if constexpr (PDE == kPdeStokes) {
-    const double tn = q.c ? q.n2 : q.n1, cn = c.c ? c.n2 : c.n1;
-    const double rr = (q.c ? r1 : r0) * (c.c ? r1 : r0) * (inv * inv) * (1.0 / M_PI);
-    et = c.w * fma(rc, rr, tn * cn);
-    es = q.w * fma(-rq, rr, tn * cn);
-  } else if constexpr (PDE == kPdeLaplaceNeumann) {
-    const double s = inv * (1.0 / (2 * M_PI));
-    et = c.w * fma(rq, s, 1.0);
-    es = q.w * fma(-rc, s, 1.0);
-  } else {
-    const double s = inv * (1.0 / (2 * M_PI));
-    et = -c.w * rc * s;
-    es = q.w * rq * s;
-  }
-  if (NEAR && r0 == 0 && r1 == 0) {
-    et = kernel_entry(PDE, q, c, true);
-    es = kernel_entry(PDE, c, q, true);
-  }
-}
 
 __device__ inline void stage_item(RowItems& it, int i, const DofGeo& d) {
   it.x[i] = d.x;
@@ -117,7 +89,7 @@ __device__ __forceinline__ void for_row_blocks(const DevGeom& g, const DevTree& 
   __syncthreads();
   for (int base = 0; base < cnt; base += kItems) {
     const int ni = min(kItems, cnt - base);
-    if (tid < ni) stage_item(items, tid, dof_geo(g, rowdofs[base + tid]));
+    if (tid < ni) stage_item(items, tid, pair_geo<PDE>(dof_geo(g, rowdofs[base + tid])));
     __syncthreads();
     for (int i0 = 4 * wv; i0 < ni; i0 += 16) {
       const int i = min(i0 + kq, ni - 1);
@@ -136,7 +108,7 @@ __device__ __forceinline__ void for_row_blocks(const DevGeom& g, const DevTree& 
       d.w = proxy_weight(t, b);
       d.k = 0;
       d.c = stokes ? tid & 1 : 0;
-      stage_item(items, tid, d);
+      stage_item(items, tid, pair_geo<PDE>(d));
     }
     __syncthreads();
     for (int i0 = 4 * wv; i0 < ni; i0 += 16)
@@ -179,7 +151,7 @@ __global__ __launch_bounds__(256, NMAX == 32 ? 4 : 2) void k_gram_id(DevGeom g, 
   const int* act = s.act_list + (int64_t)b * s.ncap;
   DofGeo cg[NT];
 #pragma unroll
-  for (int q = 0; q < NT; q++) cg[q] = dof_geo(g, act[min(16 * q + cl, n - 1)]);
+  for (int q = 0; q < NT; q++) cg[q] = pair_geo<PDE>(dof_geo(g, act[min(16 * q + cl, n - 1)]));
   D4 acc[NT * (NT + 1) / 2];
 #pragma unroll
   for (int q = 0; q < NT * (NT + 1) / 2; q++) acc[q] = D4{0, 0, 0, 0};
@@ -341,8 +313,8 @@ __global__ __launch_bounds__(256) void k_gram_blocks(DevGeom g, DevTree t, DevSt
       const int a = 32 * bi + 16 * q + cl, c = 32 * bj + 16 * q + cl;
       oi[q] = a < n;
       oj[q] = c < n;
-      ci[q] = dof_geo(g, act[min(a, n - 1)]);
-      cj[q] = dof_geo(g, act[min(c, n - 1)]);
+      ci[q] = pair_geo<PDE>(dof_geo(g, act[min(a, n - 1)]));
+      cj[q] = pair_geo<PDE>(dof_geo(g, act[min(c, n - 1)]));
     }
     D4 acc[2][2];
 #pragma unroll

@@ -110,4 +110,126 @@ __device__ inline Mfma16<float>::V4 mfma16x16x4(float a, float b, Mfma16<float>:
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// A point as pair_entries takes it: for Laplace the normal scaled by w / (2
+// pi), so that an entry is one product.
+template <int PDE>
+__device__ inline DofGeo pair_geo(DofGeo d) {
+  if constexpr (PDE == kPdeLaplace) {
+    const double s = d.w * (1.0 / (2 * M_PI));
+    d.n1 *= s;
+    d.n2 *= s;
+  }
+  return d;
+}
+
+// Entries of row point q and column c in both directions, et = K(q, c) and
+// es = K(c, q) (the kernels of rs_device.hpp): they share r, |r|^2 and its
+// reciprocal, which are most of an entry's arithmetic.  NEAR: boundary DOFs,
+// which may coincide.
+template <int PDE, bool NEAR>
+__device__ __forceinline__ void pair_entries(const DofGeo& q, const DofGeo& c, double& et,
+                                             double& es) {
+  const double r0 = q.x - c.x, r1 = q.y - c.y;
+  const double inv = recip(fma(r0, r0, r1 * r1));
+  const double rc = fma(r0, c.n1, r1 * c.n2), rq = fma(r0, q.n1, r1 * q.n2);
+  if constexpr (PDE == kPdeStokes) {
+    const double tn = q.c ? q.n2 : q.n1, cn = c.c ? c.n2 : c.n1;
+    const double rr = (q.c ? r1 : r0) * (c.c ? r1 : r0) * (inv * inv) * (1.0 / M_PI);
+    et = c.w * fma(rc, rr, tn * cn);
+    es = q.w * fma(-rq, rr, tn * cn);
+  } else if constexpr (PDE == kPdeLaplaceNeumann) {
+    const double s = inv * (1.0 / (2 * M_PI));
+    et = c.w * fma(rq, s, 1.0);
+    es = q.w * fma(-rc, s, 1.0);
+  } else {
+    et = -rc * inv;
+    es = rq * inv;
+  }
+  if (NEAR && r0 == 0 && r1 == 0) {  // the source's diagonal value
+    if constexpr (PDE == kPdeLaplace) {
+      const double h = 0.25 / M_PI;
+      et = fma(h * c.k, c.w, 0.5);
+      es = fma(h * q.k, q.w, 0.5);
+    } else {
+      et = kernel_entry(PDE, q, c, true);
+      es = kernel_entry(PDE, c, q, true);
+    }
+  }
+}
+
+// Sketch of one part of a box's ID matrix: row points 0 .. items - 1 (NEAR:
+// near DOFs; else proxy rows), whose entries with the box as source are ID
+// rows trow + i and as target srow + i, times Omega (ld LD) into NQ 16-row
+// tiles.  The lane's column is cg; row geometry (pair_geo) comes from the LDS
+// table at idx0 + i (>> 1 for the proxy rows of Stokes).  Blocks of 4 U
+// points part, part + parts, ...; the next block's Omega operands are loaded
+// before this block's entries when AHEAD.  Points past the end carry zero
+// Omega; the tiles of columns past the box's are never read.
+// An entry pair's arithmetic is 40% less than two entries'; the MFMAs (64
+// cycles for a 16 x 16 x 4 product in FP64) then bound the large levels.
+// Learned widths, 262,144 points: k_rid 1430 us per factorization with one
+// direction at a time, 1264 with both; Stokes, 16,385 points: k_rid_wide
+// 2.1 and 1.9 ms.
+template <typename R, int PDE, bool NEAR, int NQ, int LD, int U, bool AHEAD, int TR>
+__device__ __forceinline__ void sketch_pairs(const double (*tab)[TR], const int* rowdofs,
+                                             const double* omega, int items, int trow, int srow,
+                                             int idx0, int part, int parts, const DofGeo& cg,
+                                             typename Mfma16<R>::V4 (&acc)[NQ]) {
+  constexpr bool stokes = PDE == kPdeStokes;
+  const int lane = threadIdx.x & 63, cl = lane & 15, kq = lane >> 4;
+  const int step = 4 * U * parts;
+  if (4 * U * part >= items) return;
+  auto load_omega = [&](int i0, R (&w)[U][2][NQ]) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + 4 * u + kq, ic = min(i, items - 1);
+      const double* ot = omega + (int64_t)(trow + ic) * LD + cl;
+      const double* os = omega + (int64_t)(srow + ic) * LD + cl;
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        w[u][0][q] = i < items ? static_cast<R>(ot[16 * q]) : R(0);
+        w[u][1][q] = i < items ? static_cast<R>(os[16 * q]) : R(0);
+      }
+    }
+  };
+  R nw[U][2][NQ];
+  if (AHEAD) load_omega(4 * U * part, nw);
+  for (int i0 = 4 * U * part; i0 < items; i0 += step) {
+    R w[U][2][NQ];
+    if (AHEAD) {
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+          w[u][0][q] = nw[u][0][q];
+          w[u][1][q] = nw[u][1][q];
+        }
+      if (i0 + step < items) load_omega(i0 + step, nw);
+    } else {
+      load_omega(i0, w);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = min(i0 + 4 * u + kq, items - 1);
+      const int idx = idx0 + ((stokes && !NEAR) ? i >> 1 : i);
+      DofGeo rg;
+      rg.x = tab[0][idx];
+      rg.y = tab[1][idx];
+      rg.n1 = tab[2][idx];
+      rg.n2 = tab[3][idx];
+      rg.w = tab[4][idx];
+      rg.k = tab[5][idx];
+      rg.c = stokes ? (NEAR ? rowdofs[i] & 1 : i & 1) : 0;
+      double et, es;
+      pair_entries<PDE, NEAR>(rg, cg, et, es);
+      const R a = static_cast<R>(et), b = static_cast<R>(es);
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        acc[q] = mfma16x16x4(w[u][0][q], a, acc[q]);
+        acc[q] = mfma16x16x4(w[u][1][q], b, acc[q]);
+      }
+    }
+  }
+}
+
 }  // namespace iegpu

@@ -30,69 +30,6 @@ namespace {
 // take it.
 // ---------------------------------------------------------------------------
 
-// Rows [s0, s1) of one segment of a box's ID matrix (all rows of a
-// segment share their role: TG the row point is the target, NEAR a
-// boundary DOF) times Omega into the sketch tiles acc0 (rows 0..15) and
-// acc1 (rows 16..31, when two).  Row geometry comes from the LDS table at
-// index idx0 + (r - s0) (>> 1 for proxy rows of Stokes); the next 16
-// rows' Omega operands are loaded before this iteration's entries.
-template <typename R, int PDE, bool TG, bool NEAR>
-__device__ __forceinline__ void rid_segment(const double (*tab)[kRidMaxNear + kNumProxy],
-                                            const int* rowdofs, const double* omega, int s0,
-                                            int s1, int idx0, const DofGeo& cg, bool cv,
-                                            bool two, typename Mfma16<R>::V4& acc0,
-                                            typename Mfma16<R>::V4& acc1) {
-  constexpr int LM = kRidRows;
-  constexpr bool stokes = PDE == kPdeStokes;
-  const int lane = threadIdx.x & 63, cl = lane & 15, kq = lane >> 4;
-  auto load_omega = [&](int k0, R* w0, R* w1) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = k0 + 4 * u + kq;
-      const double* om = omega + (int64_t)min(r, s1 - 1) * LM + cl;
-      w0[u] = r < s1 ? static_cast<R>(om[0]) : R(0);
-      w1[u] = (two && r < s1) ? static_cast<R>(om[16]) : R(0);
-    }
-  };
-  R nw0[4], nw1[4];
-  load_omega(s0, nw0, nw1);
-  for (int k0 = s0; k0 < s1; k0 += 16) {
-    R w0[4], w1[4], a[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      w0[u] = nw0[u];
-      w1[u] = nw1[u];
-    }
-    if (k0 + 16 < s1) load_omega(k0 + 16, nw0, nw1);
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = min(k0 + 4 * u + kq, s1 - 1);
-      const int rel = r - s0;
-      const int idx = idx0 + ((stokes && !NEAR) ? rel >> 1 : rel);
-      DofGeo rg;
-      rg.x = tab[0][idx];
-      rg.y = tab[1][idx];
-      rg.n1 = tab[2][idx];
-      rg.n2 = tab[3][idx];
-      rg.w = tab[4][idx];
-      rg.k = tab[5][idx];
-      rg.c = stokes ? (NEAR ? rowdofs[rel] & 1 : rel & 1) : 0;
-      const double e = TG ? kernel_entry(PDE, rg, cg, NEAR) : kernel_entry(PDE, cg, rg, NEAR);
-      a[u] = (cv && k0 + 4 * u + kq < s1) ? static_cast<R>(e) : R(0);
-    }
-    if (two) {
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        acc0 = mfma16x16x4(w0[u], a[u], acc0);
-        acc1 = mfma16x16x4(w1[u], a[u], acc1);
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < 4; u++) acc0 = mfma16x16x4(w0[u], a[u], acc0);
-    }
-  }
-}
-
 // One workgroup (4 waves) per box.  The box's row geometry (near DOFs,
 // then the proxy circle) is staged in LDS; wave w sketches the 16-column
 // tile w (n <= 64) segment by segment (near target rows, near source rows,
@@ -128,16 +65,18 @@ __global__ __launch_bounds__(256, 5) void k_rid(DevGeom g, DevTree t, DevState s
   if (level >= 3 && tid < kNumProxy) {
     double px, py, n1, n2;
     proxy_point(t.cx[b], t.cy[b], t.side[b] * kRadiusRatio, tid, &px, &py, &n1, &n2);
+    const double pw = proxy_weight(t, b);
+    const DofGeo d = pair_geo<PDE>(DofGeo{px, py, n1, n2, pw, 0, 0});
     tab[0][cnt + tid] = px;
     tab[1][cnt + tid] = py;
-    tab[2][cnt + tid] = n1;
-    tab[3][cnt + tid] = n2;
-    tab[4][cnt + tid] = proxy_weight(t, b);
+    tab[2][cnt + tid] = d.n1;
+    tab[3][cnt + tid] = d.n2;
+    tab[4][cnt + tid] = pw;
     tab[5][cnt + tid] = 0;
   }
   __syncthreads();
   for (int i = tid; i < cnt; i += 256) {
-    const DofGeo d = dof_geo(g, rowdofs[i]);
+    const DofGeo d = pair_geo<PDE>(dof_geo(g, rowdofs[i]));
     tab[0][i] = d.x;
     tab[1][i] = d.y;
     tab[2][i] = d.n1;
@@ -150,27 +89,30 @@ __global__ __launch_bounds__(256, 5) void k_rid(DevGeom g, DevTree t, DevState s
   // Sketch: wave wv takes columns 16 wv .. 16 wv + 15.
   const int kq = lane >> 4;
   const int c = 16 * wv + (lane & 15);
-  V4 acc0 = V4{0, 0, 0, 0}, acc1 = V4{0, 0, 0, 0};
+  V4 acc[2] = {V4{0, 0, 0, 0}, V4{0, 0, 0, 0}};
   if (16 * wv < n) {
-    const bool cv = c < n;
-    const DofGeo cg = dof_geo(g, act[cv ? c : n - 1]);
-    const bool two = l > 16;
-    rid_segment<R, PDE, true, true>(tab, rowdofs, s.omega, 0, cnt, 0, cg, cv, two, acc0, acc1);
-    rid_segment<R, PDE, false, true>(tab, rowdofs, s.omega, cnt, 2 * cnt, 0, cg, cv, two, acc0,
-                                     acc1);
-    if (P > 0) {
-      rid_segment<R, PDE, true, false>(tab, rowdofs, s.omega, 2 * cnt, 2 * cnt + P, cnt, cg, cv,
-                                       two, acc0, acc1);
-      rid_segment<R, PDE, false, false>(tab, rowdofs, s.omega, 2 * cnt + P, m, cnt, cg, cv, two,
-                                        acc0, acc1);
+    const DofGeo cg = pair_geo<PDE>(dof_geo(g, act[min(c, n - 1)]));
+    if (l > 16) {
+      sketch_pairs<R, PDE, true, 2, LM, 2, true>(tab, rowdofs, s.omega, cnt, 0, cnt, 0, 0, 1, cg,
+                                                 acc);
+      sketch_pairs<R, PDE, false, 2, LM, 2, true>(tab, rowdofs, s.omega, P, 2 * cnt, 2 * cnt + P,
+                                                  cnt, 0, 1, cg, acc);
+    } else {
+      V4 one[1] = {acc[0]};
+      sketch_pairs<R, PDE, true, 1, LM, 2, true>(tab, rowdofs, s.omega, cnt, 0, cnt, 0, 0, 1, cg,
+                                                 one);
+      sketch_pairs<R, PDE, false, 1, LM, 2, true>(tab, rowdofs, s.omega, P, 2 * cnt, 2 * cnt + P,
+                                                  cnt, 0, 1, cg, one);
+      acc[0] = one[0];
     }
   }
   __syncthreads();  // the row table becomes Y
-  // acc[v] = Y[16 it + row(kq, v)][c]; tiles past n and rows past l are 0.
+  // acc[q][v] = Y[16 q + row(kq, v)][c]; rows past l are 0, columns past n
+  // unused.
 #pragma unroll
   for (int v = 0; v < 4; v++) {
-    ybuf[Mfma16<R>::row(kq, v) * YLD + c] = acc0[v];
-    ybuf[(16 + Mfma16<R>::row(kq, v)) * YLD + c] = acc1[v];
+    ybuf[Mfma16<R>::row(kq, v) * YLD + c] = acc[0][v];
+    ybuf[(16 + Mfma16<R>::row(kq, v)) * YLD + c] = acc[1][v];
   }
   __syncthreads();
   if (wv != 0) return;
@@ -307,58 +249,6 @@ __global__ __launch_bounds__(256, 5) void k_rid(DevGeom g, DevTree t, DevState s
 // rid_done = 0: a register-QRCP box joins the fallback list, any other is
 // still on its full-QRCP list (whose kernels skip the boxes the sketch
 // took).
-template <typename R, int PDE, bool TG, bool NEAR>
-__device__ __forceinline__ void rid_segment_w(const double (*tab)[kRidMaxNearW + kNumProxy],
-                                              const int* rowdofs, const double* omega, int s0,
-                                              int s1, int idx0, int part, int parts,
-                                              const DofGeo& cg, bool cv,
-                                              typename Mfma16<R>::V4 (&acc)[4]) {
-  constexpr int LM = kRidRowsW;
-  constexpr bool stokes = PDE == kPdeStokes;
-  const int lane = threadIdx.x & 63, cl = lane & 15, kq = lane >> 4;
-  // the next block's Omega operands are loaded before this block's entries
-  auto load_omega = [&](int k0, R (&w)[4][4]) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = k0 + 4 * u + kq;
-      const double* om = omega + (int64_t)min(r, s1 - 1) * LM + cl;
-#pragma unroll
-      for (int q = 0; q < 4; q++) w[q][u] = r < s1 ? static_cast<R>(om[16 * q]) : R(0);
-    }
-  };
-  const int step = 16 * parts;
-  R nw[4][4];
-  load_omega(s0 + 16 * part, nw);
-  for (int k0 = s0 + 16 * part; k0 < s1; k0 += step) {
-    R w[4][4], a[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) w[q][u] = nw[q][u];
-    if (k0 + step < s1) load_omega(k0 + step, nw);
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = k0 + 4 * u + kq;
-      const int rel = min(r, s1 - 1) - s0;
-      const int idx = idx0 + ((stokes && !NEAR) ? rel >> 1 : rel);
-      DofGeo rg;
-      rg.x = tab[0][idx];
-      rg.y = tab[1][idx];
-      rg.n1 = tab[2][idx];
-      rg.n2 = tab[3][idx];
-      rg.w = tab[4][idx];
-      rg.k = tab[5][idx];
-      rg.c = stokes ? (NEAR ? rowdofs[rel] & 1 : rel & 1) : 0;
-      const double e = TG ? kernel_entry(PDE, rg, cg, NEAR) : kernel_entry(PDE, cg, rg, NEAR);
-      a[u] = (cv && r < s1) ? static_cast<R>(e) : R(0);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) acc[q] = mfma16x16x4(w[q][u], a[u], acc[q]);
-  }
-}
-
 constexpr int kRidWideWaves = 8;
 
 // LDS of the wide sketch: the row table, then Y, then the rows of R (a
@@ -403,16 +293,18 @@ __device__ __forceinline__ void rid_wide_box(const DevGeom& g, const DevTree& t,
   if (level >= 3 && tid < kNumProxy) {
     double px, py, n1, n2;
     proxy_point(t.cx[b], t.cy[b], t.side[b] * kRadiusRatio, tid, &px, &py, &n1, &n2);
+    const double pw = proxy_weight(t, b);
+    const DofGeo d = pair_geo<PDE>(DofGeo{px, py, n1, n2, pw, 0, 0});
     tab[0][cnt + tid] = px;
     tab[1][cnt + tid] = py;
-    tab[2][cnt + tid] = n1;
-    tab[3][cnt + tid] = n2;
-    tab[4][cnt + tid] = proxy_weight(t, b);
+    tab[2][cnt + tid] = d.n1;
+    tab[3][cnt + tid] = d.n2;
+    tab[4][cnt + tid] = pw;
     tab[5][cnt + tid] = 0;
   }
   __syncthreads();
   for (int i = tid; i < cnt; i += NT) {
-    const DofGeo d = dof_geo(g, rowdofs[i]);
+    const DofGeo d = pair_geo<PDE>(dof_geo(g, rowdofs[i]));
     tab[0][i] = d.x;
     tab[1][i] = d.y;
     tab[2][i] = d.n1;
@@ -430,18 +322,11 @@ __device__ __forceinline__ void rid_wide_box(const DevGeom& g, const DevTree& t,
   for (int q = 0; q < 4; q++) acc[q] = V4{0, 0, 0, 0};
   const int c = 16 * tile + (lane & 15);
   if (16 * tile < n) {
-    const bool cv = c < n;
-    const DofGeo cg = dof_geo(g, act[cv ? c : n - 1]);
-    rid_segment_w<R, PDE, true, true>(tab, rowdofs, s.omega_w, 0, cnt, 0, part, kParts, cg, cv,
-                                      acc);
-    rid_segment_w<R, PDE, false, true>(tab, rowdofs, s.omega_w, cnt, 2 * cnt, 0, part, kParts,
-                                       cg, cv, acc);
-    if (P > 0) {
-      rid_segment_w<R, PDE, true, false>(tab, rowdofs, s.omega_w, 2 * cnt, 2 * cnt + P, cnt,
-                                         part, kParts, cg, cv, acc);
-      rid_segment_w<R, PDE, false, false>(tab, rowdofs, s.omega_w, 2 * cnt + P, m, cnt, part,
-                                          kParts, cg, cv, acc);
-    }
+    const DofGeo cg = pair_geo<PDE>(dof_geo(g, act[min(c, n - 1)]));
+    sketch_pairs<R, PDE, true, 4, LM, 2, true>(tab, rowdofs, s.omega_w, cnt, 0, cnt, 0, part,
+                                               kParts, cg, acc);
+    sketch_pairs<R, PDE, false, 4, LM, 2, true>(tab, rowdofs, s.omega_w, P, 2 * cnt, 2 * cnt + P,
+                                                cnt, part, kParts, cg, acc);
   }
   __syncthreads();  // the row table becomes Y
   for (int p = 0; p < kParts; p++) {  // the row parts added in order

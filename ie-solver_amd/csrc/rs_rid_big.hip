@@ -21,9 +21,9 @@ namespace {
 // for them: a box's sketch is spread over a workgroup per 64 columns and
 // row part (kRidBigParts), its QR takes one workgroup.
 //
-// k_rid_big_sketch: the part's rows of A (every kRidBigParts-th block of 16
-// rows of a segment) times Omega into eight 16-row MFMA tiles per wave, the
-// partial sketch to the box's scratch.
+// k_rid_big_sketch: the part's row points (every kRidBigParts-th block of
+// four) times Omega into eight 16-row MFMA tiles per wave, the partial
+// sketch to the box's scratch.
 //
 // k_rid_big_qr: column-pivoted Householder QR of the summed sketch in
 // registers.  Thread (q, c) of 4 x 128 holds rows 4 i + q of columns c and
@@ -39,42 +39,6 @@ namespace {
 // and 2,000 ID rows, ranks up to 99): 38 + 356 us a level, against 7,263 and
 // 6,175 us for the full pivoted QR of their matrices in k_qrcp.
 // ---------------------------------------------------------------------------
-
-// Rows [s0, s1) of one segment of a box's ID matrix (TG: the row point is
-// the target; NEAR: a boundary DOF) times Omega, row blocks part, part +
-// kRidBigParts, ...; row geometry from the LDS table at idx0 + (r - s0)
-// (>> 1 for proxy rows of Stokes).
-template <typename R, int PDE, bool TG, bool NEAR>
-__device__ __forceinline__ void rid_segment_b(const double (*tab)[kRidMaxNearW + kNumProxy],
-                                              const int* rowdofs, const double* omega, int s0,
-                                              int s1, int idx0, int part, const DofGeo& cg,
-                                              bool cv, typename Mfma16<R>::V4 (&acc)[8]) {
-  constexpr bool stokes = PDE == kPdeStokes;
-  const int lane = threadIdx.x & 63, cl = lane & 15, kq = lane >> 4;
-  for (int k0 = s0 + 16 * part; k0 < s1; k0 += 16 * kRidBigParts) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = k0 + 4 * u + kq, rel = min(r, s1 - 1) - s0;
-      const double* om = omega + (int64_t)(s0 + rel) * kRidRowsB + cl;
-      R w[8];
-#pragma unroll
-      for (int q = 0; q < 8; q++) w[q] = static_cast<R>(om[16 * q]);
-      const int idx = idx0 + ((stokes && !NEAR) ? rel >> 1 : rel);
-      DofGeo rg;
-      rg.x = tab[0][idx];
-      rg.y = tab[1][idx];
-      rg.n1 = tab[2][idx];
-      rg.n2 = tab[3][idx];
-      rg.w = tab[4][idx];
-      rg.k = tab[5][idx];
-      rg.c = stokes ? (NEAR ? rowdofs[rel] & 1 : rel & 1) : 0;
-      const double e = TG ? kernel_entry(PDE, rg, cg, NEAR) : kernel_entry(PDE, cg, rg, NEAR);
-      const R a = (cv && r < s1) ? static_cast<R>(e) : R(0);
-#pragma unroll
-      for (int q = 0; q < 8; q++) acc[q] = mfma16x16x4(w[q], a, acc[q]);
-    }
-  }
-}
 
 template <typename R, int PDE>
 __global__ __launch_bounds__(256, 2) void k_rid_big_sketch(DevGeom g, DevTree t, DevState s,
@@ -100,16 +64,18 @@ __global__ __launch_bounds__(256, 2) void k_rid_big_sketch(DevGeom g, DevTree t,
     if (level >= 3 && tid < kNumProxy) {
       double px, py, n1, n2;
       proxy_point(t.cx[b], t.cy[b], t.side[b] * kRadiusRatio, tid, &px, &py, &n1, &n2);
+      const double pw = proxy_weight(t, b);
+      const DofGeo d = pair_geo<PDE>(DofGeo{px, py, n1, n2, pw, 0, 0});
       tab[0][cnt + tid] = px;
       tab[1][cnt + tid] = py;
-      tab[2][cnt + tid] = n1;
-      tab[3][cnt + tid] = n2;
-      tab[4][cnt + tid] = proxy_weight(t, b);
+      tab[2][cnt + tid] = d.n1;
+      tab[3][cnt + tid] = d.n2;
+      tab[4][cnt + tid] = pw;
       tab[5][cnt + tid] = 0;
     }
     __syncthreads();
     for (int i = tid; i < cnt; i += 256) {
-      const DofGeo d = dof_geo(g, rowdofs[i]);
+      const DofGeo d = pair_geo<PDE>(dof_geo(g, rowdofs[i]));
       tab[0][i] = d.x;
       tab[1][i] = d.y;
       tab[2][i] = d.n1;
@@ -121,21 +87,16 @@ __global__ __launch_bounds__(256, 2) void k_rid_big_sketch(DevGeom g, DevTree t,
     const int kq = lane >> 4;
     const int c = 64 * blockIdx.y + 16 * wv + (lane & 15);
     if (c - (lane & 15) >= n16) continue;
-    const bool cv = c < n;
     const int* act = s.act_list + (int64_t)b * s.ncap;
-    const DofGeo cg = dof_geo(g, act[cv ? c : n - 1]);
+    const DofGeo cg = pair_geo<PDE>(dof_geo(g, act[min(c, n - 1)]));
     V4 acc[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) acc[q] = V4{0, 0, 0, 0};
-    rid_segment_b<R, PDE, true, true>(tab, rowdofs, s.omega_b, 0, cnt, 0, part, cg, cv, acc);
-    rid_segment_b<R, PDE, false, true>(tab, rowdofs, s.omega_b, cnt, 2 * cnt, 0, part, cg, cv,
-                                       acc);
-    if (P > 0) {
-      rid_segment_b<R, PDE, true, false>(tab, rowdofs, s.omega_b, 2 * cnt, 2 * cnt + P, cnt, part,
-                                         cg, cv, acc);
-      rid_segment_b<R, PDE, false, false>(tab, rowdofs, s.omega_b, 2 * cnt + P, m, cnt, part, cg,
-                                          cv, acc);
-    }
+    sketch_pairs<R, PDE, true, 8, kRidRowsB, 1, false>(tab, rowdofs, s.omega_b, cnt, 0, cnt, 0,
+                                                       part, kRidBigParts, cg, acc);
+    sketch_pairs<R, PDE, false, 8, kRidRowsB, 1, false>(tab, rowdofs, s.omega_b, P, 2 * cnt,
+                                                        2 * cnt + P, cnt, part, kRidBigParts, cg,
+                                                        acc);
     R* Y = reinterpret_cast<R*>(s.id_pool) + s.id_off[b] + (int64_t)part * kRidRowsB * n16;
 #pragma unroll
     for (int q = 0; q < 8; q++)

@@ -267,9 +267,9 @@ __device__ inline int* list_slot(const DevState& s, int level, int L) {
 }
 // Row-compression jobs (chunks) of box b.
 __device__ inline int row_jobs(const DevState& s, int b) {
-  const int kind = s.qkind[b];
-  if (kind == kQrcpStack) return id_chunks(s.m_rows[b], kRegMaxRows);
-  if (kind == kQrcpStack8) return id_chunks(s.m_rows[b], kRegMaxRows8);
+  const int kind = s.qkind[b], m = s.m_rows[b];
+  if (kind == kQrcpStack) return id_chunks(m, kRegMaxRows);
+  if (kind == kQrcpStack8) return id_chunks(m, kRegMaxRows8);
   return 0;
 }
 
@@ -357,6 +357,10 @@ constexpr int kQuadSwap3 = 0x1B;     // quad_perm [3,2,1,0]
 constexpr int kQuadBitrev = 0xD8;    // quad_perm [0,2,1,3]
 constexpr int kRowRor4 = 0x124;
 constexpr int kRowRor8 = 0x128;
+constexpr int kRowShr1 = 0x111;
+constexpr int kRowShr2 = 0x112;
+constexpr int kRowShr4 = 0x114;
+constexpr int kRowShr8 = 0x118;
 }  // namespace dpp
 
 template <int CTRL, int ROWS>
@@ -373,6 +377,24 @@ __device__ inline float dpp_f32(float v) {
 template <int CTRL, int ROWS>
 __device__ inline int dpp_i32(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+
+template <int CTRL, int ROWS>
+__device__ inline int64_t dpp_i64(int64_t v) {
+  const int lo = dpp_i32<CTRL, ROWS>((int)v), hi = dpp_i32<CTRL, ROWS>((int)(v >> 32));
+  return ((int64_t)hi << 32) | (unsigned int)lo;
+}
+
+// Inclusive sum over the lanes up to the calling one (lanes a shift reads
+// from before its row add 0).
+__device__ inline int64_t wave_scan(int64_t v) {
+  v += dpp_i64<dpp::kRowShr1, 0xF>(v);
+  v += dpp_i64<dpp::kRowShr2, 0xF>(v);
+  v += dpp_i64<dpp::kRowShr4, 0xF>(v);
+  v += dpp_i64<dpp::kRowShr8, 0xF>(v);
+  v += dpp_i64<dpp::kRowBcast15, 0xA>(v);
+  v += dpp_i64<dpp::kRowBcast31, 0xC>(v);
+  return v;
 }
 
 // Index of the calling wave in its workgroup, as a wave-uniform (scalar)

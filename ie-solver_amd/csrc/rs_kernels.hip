@@ -236,12 +236,6 @@ __global__ __launch_bounds__(64) void k_rows(DevGeom g, DevTree t, DevState s,
   }
 }
 
-// A register-QRCP box the randomized ID does not sketch goes to the full
-// QRCP list at the scan.
-__device__ inline bool rid_full_qrcp(const DevState& s, int b, int kind) {
-  return s.rid_mode != 0 && (kind == kQrcpReg || kind == kQrcpStack) && s.sk_w[b] == 0;
-}
-
 // Scanned per box: ID scratch, row-list and factor sizes, register-QRCP
 // and general-QRCP list entries, row-compression jobs, sketches, decouple
 // operands, boxes above kSmallBox DOFs.
@@ -249,65 +243,85 @@ constexpr int kScanQ = 14;
 constexpr int kScanLd = 16;      // words per block in scan_blk
 constexpr int kScanMulti = 2048; // levels of at least this many boxes: three kernels
 
-__device__ inline void scan_counts(const DevState& s, int b, int64_t (&own)[kScanQ]) {
-  if (box_clean(s, b)) return;
-  const int kind = s.qkind[b];
-  own[0] += s.id_sz[b];
-  own[1] += s.row_sz[b];
-  own[2] += max(s.fac_sz[b], int64_t(0));
-  own[3] += ((kind == kQrcpReg || kind == kQrcpStack) && s.act_cnt[b] > kHalfCols) ? 1 : 0;
-  own[7] += ((kind == kQrcpReg || kind == kQrcpStack) && s.act_cnt[b] <= kHalfCols) ? 1 : 0;
-  own[4] += (kind == kQrcpLds) ? 1 : 0;
-  own[5] += row_jobs(s, b);
-  own[6] += (kind == kQrcpReg8 || kind == kQrcpStack8) ? 1 : 0;
-  own[8] += (s.sk_w[b] > 0 && s.sk_w[b] <= kRidRows) ? 1 : 0;
-  own[9] += rid_full_qrcp(s, b, kind) ? 1 : 0;
-  own[10] += s.dec_sz[b];
-  own[11] += (s.sk_w[b] == kRidRowsW) ? 1 : 0;
-  own[12] += (s.act_cnt[b] > kSmallBox) ? 1 : 0;
-  own[13] += (s.sk_w[b] == kRidRowsB) ? 1 : 0;
+// What the scan reads of a box, loaded before any store (a load behind a
+// store that may alias it waits for it).
+struct ScanBox {
+  int64_t id, row, fac, dec;
+  int kind, n, w, jobs;
+  bool on;
+};
+
+__device__ inline ScanBox scan_load(const DevState& s, int b) {
+  ScanBox v;
+  v.kind = s.qkind[b];
+  v.n = s.act_cnt[b];
+  v.w = s.sk_w[b];
+  v.id = s.id_sz[b];
+  v.row = s.row_sz[b];
+  v.fac = s.fac_sz[b];
+  v.dec = s.dec_sz[b];
+  v.jobs = row_jobs(s, b);
+  v.on = !box_clean(s, b);
+  return v;
+}
+
+__device__ inline bool reg_kind(const ScanBox& v) {
+  return v.kind == kQrcpReg || v.kind == kQrcpStack;
+}
+
+__device__ inline void scan_counts(const DevState& s, const ScanBox& v, int64_t (&own)[kScanQ]) {
+  if (!v.on) return;
+  own[0] += v.id;
+  own[1] += v.row;
+  own[2] += max(v.fac, int64_t(0));
+  own[3] += (reg_kind(v) && v.n > kHalfCols) ? 1 : 0;
+  own[7] += (reg_kind(v) && v.n <= kHalfCols) ? 1 : 0;
+  own[4] += (v.kind == kQrcpLds) ? 1 : 0;
+  own[5] += v.jobs;
+  own[6] += (v.kind == kQrcpReg8 || v.kind == kQrcpStack8) ? 1 : 0;
+  own[8] += (v.w > 0 && v.w <= kRidRows) ? 1 : 0;
+  own[9] += (s.rid_mode != 0 && reg_kind(v) && v.w == 0) ? 1 : 0;
+  own[10] += v.dec;
+  own[11] += (v.w == kRidRowsW) ? 1 : 0;
+  own[12] += (v.n > kSmallBox) ? 1 : 0;
+  own[13] += (v.w == kRidRowsB) ? 1 : 0;
 }
 
 // Box b's slots and list entries from the exclusive offsets off (advanced
 // past the box).
-__device__ inline void scan_place(const DevState& s, int b, int start, int level,
-                                  int64_t fbase, int64_t (&off)[kScanQ]) {
-  if (box_clean(s, b)) return;
-  int* lreg = s.lists + (int64_t)kLstReg * s.nbox + start;
-  int* llds = s.lists + (int64_t)kLstLds * s.nbox + start;
-  int* lreg8 = s.lists + (int64_t)kLstReg8 * s.nbox + start;
-  int* lhalf = s.lists + (int64_t)kLstRegHalf * s.nbox + start;
-  int* lrid = s.lists + (int64_t)kLstRid * s.nbox + start;
-  int* lfb = s.lists + (int64_t)kLstFallback * s.nbox + start;
+__device__ inline void scan_place(const DevState& s, const ScanBox& v, int b, int start,
+                                  int level, int64_t fbase, int64_t (&off)[kScanQ]) {
+  if (!v.on) return;
+  auto list = [&](int L) { return s.lists + (int64_t)L * s.nbox + start; };
   int* jobs = s.jobs + (int64_t)2 * kMaxChunks * start;
-  const int kind = s.qkind[b];
   // Scratch of odd and even levels in separate halves: a level's ID runs
   // while the level below it is still being decoupled.
   s.id_off[b] = (level & 1) * s.id_cap + off[0];
   s.row_off[b] = off[1];
-  if (s.fac_sz[b] < 0) {  // keeps its slot
-    s.fac_sz[b] = -s.fac_sz[b];
+  if (v.fac < 0) {  // keeps its slot
+    s.fac_sz[b] = -v.fac;
   } else {
     s.fac_off[b] = fbase + off[2];
-    off[2] += s.fac_sz[b];
+    off[2] += v.fac;
   }
   s.dec_off[b] = off[10];
-  off[10] += s.dec_sz[b];
-  off[0] += s.id_sz[b];
-  off[1] += s.row_sz[b];
-  if (kind == kQrcpReg || kind == kQrcpStack) {
-    if (s.act_cnt[b] > kHalfCols) lreg[off[3]++] = b;
-    else lhalf[off[7]++] = b;
+  off[10] += v.dec;
+  off[0] += v.id;
+  off[1] += v.row;
+  if (reg_kind(v)) {
+    if (v.n > kHalfCols) list(kLstReg)[off[3]++] = b;
+    else list(kLstRegHalf)[off[7]++] = b;
   }
-  if (kind == kQrcpLds) llds[off[4]++] = b;
-  if (kind == kQrcpReg8 || kind == kQrcpStack8) lreg8[off[6]++] = b;
-  if (s.sk_w[b] > 0 && s.sk_w[b] <= kRidRows) lrid[off[8]++] = b;
-  if (s.sk_w[b] == kRidRowsW) s.lists[(int64_t)kLstRidWide * s.nbox + start + off[11]++] = b;
-  if (s.sk_w[b] == kRidRowsB) s.lists[(int64_t)kLstRidBig * s.nbox + start + off[13]++] = b;
-  if (rid_full_qrcp(s, b, kind)) lfb[off[9]++] = b;
-  if (s.act_cnt[b] > kSmallBox) s.lists[(int64_t)kLstBig * s.nbox + start + off[12]++] = b;
-  const int nch = row_jobs(s, b);
-  for (int q = 0; q < nch; q++) {
+  if (v.kind == kQrcpLds) list(kLstLds)[off[4]++] = b;
+  if (v.kind == kQrcpReg8 || v.kind == kQrcpStack8) list(kLstReg8)[off[6]++] = b;
+  if (v.w > 0 && v.w <= kRidRows) list(kLstRid)[off[8]++] = b;
+  if (v.w == kRidRowsW) list(kLstRidWide)[off[11]++] = b;
+  if (v.w == kRidRowsB) list(kLstRidBig)[off[13]++] = b;
+  // A register-QRCP box the randomized ID does not sketch goes to the full
+  // QRCP list.
+  if (s.rid_mode != 0 && reg_kind(v) && v.w == 0) list(kLstFallback)[off[9]++] = b;
+  if (v.n > kSmallBox) list(kLstBig)[off[12]++] = b;
+  for (int q = 0; q < v.jobs; q++) {
     jobs[2 * off[5]] = b;
     jobs[2 * off[5] + 1] = q;
     off[5]++;
@@ -356,12 +370,7 @@ __device__ inline void block_scan(const int64_t (&own)[kScanQ], int64_t (&off)[k
   int64_t inc[kScanQ];
 #pragma unroll
   for (int q = 0; q < kScanQ; q++) {
-    int64_t v = own[q];
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int64_t u = __shfl_up(v, o, 64);
-      if (lane >= o) v += u;
-    }
+    const int64_t v = wave_scan(own[q]);
     inc[q] = v;
     if (lane == 63) wtot[q][wv] = v;
   }
@@ -380,25 +389,29 @@ __device__ inline void block_scan(const int64_t (&own)[kScanQ], int64_t (&off)[k
   for (int q = 0; q < kScanQ; q++) off[q] = wtot[q][wv] + inc[q] - own[q];
 }
 
-// Exclusive scans of the per-box sizes of one level (single workgroup;
-// each thread a contiguous chunk of boxes).  ID scratch and row lists are
+// Exclusive scans of the per-box sizes of one level (single workgroup of
+// one wave, four or sixteen by the level's boxes; each thread a contiguous
+// chunk of boxes).  Latency: sixteen waves at every level, scanning through
+// ds_bpermute with every load behind a store, took 11 to 14 us; 4.6, 5.6 and
+// 12 us with DPP scans, the loads first and the waves the level needs.  ID scratch and row lists are
 // level-local; factor slots append to the running pool offset.
 // With the randomized ID, a register-QRCP box that gets no sketch (not
 // eligible, or sent straight to the full QRCP by the rank model) starts the
 // level's full-QRCP list; k_rid appends the boxes whose sketch fails.
-__global__ __launch_bounds__(1024) void k_scan(DevState s, int start,
-                                               int count, int level) {
-  __shared__ int64_t wtot[kScanQ][16];
+template <int NT>
+__global__ __launch_bounds__(NT) void k_scan(DevState s, int start, int count, int level) {
+  __shared__ int64_t wtot[kScanQ][NT / 64];
   __shared__ int64_t tot[kScanQ];
   const int tid = threadIdx.x;
-  const int chunk = (count + 1023) / 1024;
+  const int chunk = (count + NT - 1) / NT;
   const int lo = min(count, tid * chunk), hi = min(count, lo + chunk);
   int64_t own[kScanQ] = {};
-  for (int i = lo; i < hi; i++) scan_counts(s, start + i, own);
+  for (int i = lo; i < hi; i++) scan_counts(s, scan_load(s, start + i), own);
   int64_t off[kScanQ];
-  block_scan<1024>(own, off, wtot, tot);
+  block_scan<NT>(own, off, wtot, tot);
   const int64_t fbase = *s.fac_top;
-  for (int i = lo; i < hi; i++) scan_place(s, start + i, start, level, fbase, off);
+  for (int i = lo; i < hi; i++)
+    scan_place(s, scan_load(s, start + i), start + i, start, level, fbase, off);
   __syncthreads();
   if (tid == 0) scan_finish(s, level, tot, fbase);
 }
@@ -414,7 +427,7 @@ __global__ __launch_bounds__(256) void k_scan_blocks(DevState s, int start, int 
   __shared__ int64_t tot[kScanQ];
   const int i = blockIdx.x * 256 + threadIdx.x;
   int64_t own[kScanQ] = {};
-  if (i < count) scan_counts(s, start + i, own);
+  if (i < count) scan_counts(s, scan_load(s, start + i), own);
   int64_t off[kScanQ];
   block_scan<256>(own, off, wtot, tot);
   if (threadIdx.x < kScanQ) s.scan_blk[(int64_t)blockIdx.x * kScanLd + threadIdx.x] = tot[threadIdx.x];
@@ -454,14 +467,18 @@ __global__ __launch_bounds__(256) void k_scan_place(DevState s, int start, int c
   __shared__ int64_t tot[kScanQ];
   const int i = blockIdx.x * 256 + threadIdx.x;
   int64_t own[kScanQ] = {};
-  if (i < count) scan_counts(s, start + i, own);
+  ScanBox v = {};
+  if (i < count) {
+    v = scan_load(s, start + i);
+    scan_counts(s, v, own);
+  }
   int64_t off[kScanQ];
   block_scan<256>(own, off, wtot, tot);
   if (i >= count) return;
   const int64_t* base = s.scan_blk + (int64_t)blockIdx.x * kScanLd;
 #pragma unroll
   for (int q = 0; q < kScanQ; q++) off[q] += base[q];
-  scan_place(s, start + i, start, level, s.scan_blk[(int64_t)nblk * kScanLd], off);
+  scan_place(s, v, start + i, start, level, s.scan_blk[(int64_t)nblk * kScanLd], off);
 }
 
 
@@ -529,8 +546,12 @@ void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
         k_scan_blocks<<<nblk, 256, 0, st>>>(s, start, count);
         k_scan_totals<<<1, 1024, 0, st>>>(s, nblk, level);
         k_scan_place<<<nblk, 256, 0, st>>>(s, start, count, level, nblk);
+      } else if (count > 256) {
+        k_scan<1024><<<1, 1024, 0, st>>>(s, start, count, level);
+      } else if (count > 64) {
+        k_scan<256><<<1, 256, 0, st>>>(s, start, count, level);
       } else {
-        k_scan<<<1, 1024, 0, st>>>(s, start, count, level);
+        k_scan<64><<<1, 64, 0, st>>>(s, start, count, level);
       }
       break;
     case kStageAssemble:

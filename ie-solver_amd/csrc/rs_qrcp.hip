@@ -586,6 +586,36 @@ __global__ __launch_bounds__(64 * NW, (QrcpShape<CPW, RPL, NW>::kWavesPerSimd)) 
   }
 }
 
+// Both n <= 64 shapes in one launch, for levels of at most kQrcpPairBoxes
+// boxes (one workgroup per box, all of them resident): a box of n <= 32
+// keeps eight of the sixteen waves.  Each shape's launch lasts as long as
+// its slowest box's chain of steps, one behind the other.
+// Circle of 4096 points: 50 + 43 us per level, 52 in one launch; star of
+// 65,536, levels of up to 256 boxes: 58 + 53 and 76.  With more boxes the
+// separate launches pack two n <= 32 boxes into a CU.
+constexpr int kQrcpPairBoxes = 256;
+
+template <typename R>
+__global__ __launch_bounds__(kXThreads, 4) void k_qrcp_pair(DevGeom g, DevTree t, DevState s,
+                                                            int start, int level, double tol_d) {
+  if (!pools_ok(s)) return;
+  int b;
+  if (s.rid_mode != 0) {  // the boxes without a successful sketch
+    if ((int)blockIdx.x >= list_count(s, level, kLstFallback)) return;
+    b = list_at(s, start, kLstFallback, blockIdx.x);
+  } else {
+    const int nb = list_count(s, level, kLstReg), i = (int)blockIdx.x - nb;
+    if (i >= list_count(s, level, kLstRegHalf)) return;
+    b = i < 0 ? list_at(s, start, kLstReg, blockIdx.x) : list_at(s, start, kLstRegHalf, i);
+  }
+  if (s.act_cnt[b] > kHalfCols) {
+    qrcp_id_box<R, 4, 8, 16>(g, t, s, start, level, b, tol_d);
+  } else {
+    if (wave_id() >= 8) return;
+    qrcp_id_box<R, 4, 8, 8>(g, t, s, start, level, b, tol_d);
+  }
+}
+
 // General form (any box the register form does not take): the matrix lives
 // in LDS when it fits, else in the box's scratch slot; each wave owns a
 // strided set of columns.
@@ -785,7 +815,9 @@ void launch_qrcp(const DevGeom& g, const DevTree& t, const DevState& s, int leve
     // Only the boxes without a successful sketch reach the full QRCP.
     k_rowcomp<R, 4><<<min(jobs_max, caps.rowcomp4), kXThreads, 0, st>>>(g, t, s, start,
                                                                         level);
-    if (count <= caps.qrcp_id) {
+    if (count <= min(kQrcpPairBoxes, caps.qrcp_id)) {
+      k_qrcp_pair<R><<<count, kXThreads, 0, st>>>(g, t, s, start, level, tol);
+    } else if (count <= caps.qrcp_id) {
       k_qrcp_id<R, 4, 8, 8, true, false><<<count, 512, 0, st>>>(g, t, s, start, level, tol);
       k_qrcp_id<R, 4, 8, 16, true, false><<<count, kXThreads, 0, st>>>(g, t, s, start,
                                                                        level, tol);
@@ -797,8 +829,12 @@ void launch_qrcp(const DevGeom& g, const DevTree& t, const DevState& s, int leve
   } else {
     k_rowcomp<R, 4><<<min(2 * count, caps.rowcomp4), kXThreads, 0, st>>>(g, t, s, start,
                                                                         level);
-    k_qrcp_id<R, 4, 8, 8, false><<<count, 512, 0, st>>>(g, t, s, start, level, tol);
-    k_qrcp_id<R, 4, 8, 16, false><<<count, kXThreads, 0, st>>>(g, t, s, start, level, tol);
+    if (count <= kQrcpPairBoxes) {
+      k_qrcp_pair<R><<<count, kXThreads, 0, st>>>(g, t, s, start, level, tol);
+    } else {
+      k_qrcp_id<R, 4, 8, 8, false><<<count, 512, 0, st>>>(g, t, s, start, level, tol);
+      k_qrcp_id<R, 4, 8, 16, false><<<count, kXThreads, 0, st>>>(g, t, s, start, level, tol);
+    }
   }
   if (!(skip & kSkipReg8Qrcp)) {
     k_rowcomp<R, 8><<<min(2 * count, caps.rowcomp8), kXThreads, 0, st>>>(g, t, s, start,

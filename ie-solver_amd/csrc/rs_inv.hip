@@ -33,10 +33,13 @@ namespace {
 // written.
 //
 // Bound by the chain of panels (wait, one update, 16 pivot steps, publish):
-// about 18 us per panel in FP64.  A 212-DOF root: 277 us (986 us with one
-// workgroup streaming the block from L2); 393 DOFs: 530 us (2,984 us); the
-// 354-DOF bordered system of Stokes with 8 holes: 525 us (7,570 us by an LU
-// in one workgroup).
+// about 16 us per panel in FP64, mostly the steps' instructions.  The root
+// of the 65,536-point star: 228 us (258 with the panels handed over through
+// agent-scope fences, every wave in every step and the pivot rows stored
+// step by step); of 16,385 Stokes points: 463 us (507).  One workgroup
+// streaming the block from L2 took 986 us for 212 DOFs and 2,984 for 393, an
+// LU in one workgroup 7,570 us for the 354-DOF bordered system of Stokes
+// with 8 holes.
 // ---------------------------------------------------------------------------
 
 constexpr int kInvB = 16;       // columns of a panel
@@ -74,20 +77,31 @@ __device__ inline unsigned inv_key(R v, int row) {
 // if it never came.
 __device__ inline bool wait_flag(const int* f) {
   for (int spin = 0; spin < (1 << 22); spin++) {
-    if (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      return true;
-    }
+    if (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return true;
     __builtin_amdgcn_s_sleep(1);
   }
   return false;
 }
 
+// What workgroups of one launch hand each other (slabs, pivot rows) goes
+// through agent-scope accesses, which pass the XCDs' L2s: a publisher waits
+// for its stores' acknowledgements before the flag, and neither side writes
+// back or invalidates a whole L2 (fences took a third of a panel).
+template <typename T>
+__device__ inline void publish(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool SHARED, typename T>
+__device__ inline T fetch(const T* p) {
+  return SHARED ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
+}
+
 // x (columns CB of the thread's RT rows) takes panel q: W from the block's
 // columns, the pivot rows' old values through LDS.  pstep[row] is the step
 // that pivots on a row (kInvMax: none yet) and is extended by the panel's.
-// All threads of the workgroup.
-template <typename R, int RT, int CB>
+// SHARED: the panel was published in this launch.  All threads of the
+// workgroup.
+template <typename R, int RT, int CB, bool SHARED>
 __device__ inline void apply_panel(const R* A, const int* prow, int n, int q, R (&x)[RT][CB],
                                    short* pstep, R (*P)[CB]) {
   const int tid = threadIdx.x, q0 = q * kInvB, bw = min(kInvB, n - q0);
@@ -96,10 +110,12 @@ __device__ inline void apply_panel(const R* A, const int* prow, int n, int q, R 
   for (int u = 0; u < RT; u++) {
     const int i = tid + kInvNT * u;
 #pragma unroll
-    for (int k = 0; k < kInvB; k++)
-      w[u][k] = (i < n && k < bw) ? A[i + (int64_t)n * (q0 + k)] : R(0);
+    for (int k = 0; k < kInvB; k++) {  // all loads in flight at once
+      const R v = fetch<SHARED>(A + min(i, n - 1) + (int64_t)n * (q0 + min(k, bw - 1)));
+      w[u][k] = (i < n && k < bw) ? v : R(0);
+    }
   }
-  if (tid < bw) pstep[prow[q0 + tid]] = (short)(q0 + tid);
+  if (tid < bw) pstep[fetch<SHARED>(prow + q0 + tid)] = (short)(q0 + tid);
   if (bw < kInvB && tid < kInvB * CB) P[tid / CB][tid % CB] = R(0);  // steps past the last
   __syncthreads();
 #pragma unroll
@@ -115,6 +131,7 @@ __device__ inline void apply_panel(const R* A, const int* prow, int n, int q, R 
     }
   }
   __syncthreads();
+  if (64 * wave_id() >= n) return;
 #pragma unroll
   for (int k = 0; k < kInvB; k++)
 #pragma unroll
@@ -132,7 +149,7 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
   __shared__ R cand[2][kInvNW][kInvB];  // each wave's candidate row, by step parity
   __shared__ unsigned keys[2][kInvNW];
   __shared__ short pstep[kInvMax];
-  __shared__ int ok;
+  __shared__ int ok, sprow[kInvB];
   if (!pools_ok(s)) return;
   const int root = blockIdx.y, j = blockIdx.x, j0 = j * kInvB;
   const int n = s.act_cnt[root] + blk.extra;
@@ -147,8 +164,10 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
   for (int u = 0; u < RT; u++) {
     const int i = tid + kInvNT * u;
 #pragma unroll
-    for (int k = 0; k < kInvB; k++)
-      x[u][k] = (i < n && k < bw) ? A[i + (int64_t)n * (j0 + k)] : R(0);
+    for (int k = 0; k < kInvB; k++) {
+      const R v = A[min(i, n - 1) + (int64_t)n * (j0 + min(k, bw - 1))];
+      x[u][k] = (i < n && k < bw) ? v : R(0);
+    }
   }
   for (int i = tid; i < n; i += kInvNT) pstep[i] = (short)kInvMax;
   for (int q = 0; q < j; q++) {
@@ -158,7 +177,7 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
       if (tid == 0) atomicOr(s.err, kErrWait);
       return;
     }
-    apply_panel<R, RT, kInvB>(A, prow, n, q, x, pstep, P);
+    apply_panel<R, RT, kInvB, true>(A, prow, n, q, x, pstep, P);
     __syncthreads();
   }
   // the panel's own steps
@@ -169,9 +188,14 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
     used[u] = i >= n || pstep[i] != kInvMax;
   }
   int info = 0;
+  // Waves past the block's rows only keep the barriers.
+  const bool live = 64 * wv < n;
+  if (!live && lane == 0) keys[0][wv] = keys[1][wv] = 0;
 #pragma unroll
   for (int k = 0; k < kInvB; k++) {
-    if (k < bw) {
+    if (k < bw && !live) {
+      __syncthreads();
+    } else if (k < bw) {
       unsigned key = 0;
 #pragma unroll
       for (int u = 0; u < RT; u++)
@@ -213,21 +237,27 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
         for (int c = 0; c < kInvB; c++) x[u][c] = me ? rv[c] : fma(-m, rv[c], x[u][c]);
         used[u] = used[u] || me;
       }
-      if (tid == 0) prow[j0 + k] = p;
+      if (tid == 0) sprow[k] = p;  // a global store here is waited for at the next step
     }
   }
 #pragma unroll
   for (int u = 0; u < RT; u++) {
     const int i = tid + kInvNT * u;
+    if (i >= n) continue;
+    if (bw == kInvB) {  // no branch, and so no wait, between the stores
 #pragma unroll
-    for (int k = 0; k < kInvB; k++)
-      if (i < n && k < bw) A[i + (int64_t)n * (j0 + k)] = x[u][k];
+      for (int k = 0; k < kInvB; k++) publish(A + i + (int64_t)n * (j0 + k), x[u][k]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < kInvB; k++)
+        if (k < bw) publish(A + i + (int64_t)n * (j0 + k), x[u][k]);
+    }
   }
   if (info != 0 && tid == 0) atomicOr(s.err, kErrSingular);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // every thread's part of the slab
+  if (tid < bw) publish(prow + j0 + tid, sprow[tid]);
+  __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the slab has arrived
   __syncthreads();
-  if (tid == 0)
-    __hip_atomic_store(flags + j, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) publish(flags + j, 1);
 }
 
 template <typename R, int RT>
@@ -254,7 +284,7 @@ __global__ __launch_bounds__(kInvNT) void k_inv_finish(DevState s, InvBlocks<R> 
   for (int st = tid; st < n; st += kInvNT) pstep[prow[st]] = (short)st;
   const int np = (n + kInvB - 1) / kInvB;
   for (int q = c0 / kInvB + 1; q < np; q++)
-    apply_panel<R, RT, kInvCF>(A, prow, n, q, x, pstep, P[q & 1]);
+    apply_panel<R, RT, kInvCF, false>(A, prow, n, q, x, pstep, P[q & 1]);
   __syncthreads();
   // entry (row i, column c): inverse row = the step that pivoted on i,
   // column = the row step c pivoted on

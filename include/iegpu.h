@@ -262,7 +262,8 @@ int iegpu_evaluate(iegpu_ctx* ctx, int n_targets, const double* targets,
  * array of 2^19 doubles per GPU (4 MiB, held until the process ends):
  * eval_chunks * sol_dim * n_targets must fit it (eval_chunks =
  * ceil(n_points / 8192), at most 64; e.g. 16384 targets at 262144 Laplace
- * nodes), else IEGPU_ERR_CAPACITY.  Every call on a GPU shares that GPU's
+ * nodes), else IEGPU_ERR_CAPACITY (few targets are cut into more chunks
+ * where those fit too).  Every call on a GPU shares that GPU's
  * array, so calls that overlap on one GPU (two streams, two contexts)
  * race.  No counterpart in the reference: it is for callers that cannot
  * allocate device memory (HIP graph capture, serving loops). */

@@ -233,7 +233,7 @@ struct iegpu_ctx {
   bool factored = false;
   DevBuf<int> s_act_cnt, s_act_list, s_chpos, s_out_cnt, s_out_list,
       s_red_list, s_perm, s_rank, s_upd_kind, s_m_rows, s_row_pool, s_err,
-      s_root_piv, s_qkind, s_jobs, s_njobs, s_lists, s_lcnt, s_sk_w, s_rid_done;
+      s_root_piv, s_qkind, s_jobs, s_njobs, s_halt, s_lists, s_lcnt, s_sk_w, s_rid_done;
   DevBuf<int64_t> s_id_sz, s_row_sz, s_fac_sz, s_id_off, s_row_off, s_fac_off,
       s_fac_top, s_dec_sz, s_dec_off, s_scan_blk;
   DevBuf<unsigned char> s_id_pool, s_fac_pool, s_root_mat, s_dec_pool;
@@ -381,6 +381,7 @@ struct iegpu_ctx {
     s.lcnt = s_lcnt.p;
     s.jobs = s_jobs.p;
     s.njobs = s_njobs.p;
+    s.halt = s_halt.p;
     s.id_sz = s_id_sz.p;
     s.row_sz = s_row_sz.p;
     s.fac_sz = s_fac_sz.p;
@@ -547,6 +548,7 @@ void alloc_state(iegpu_ctx* c) {
   c->s_lcnt.alloc((size_t)2 * kMaxLevels * kNumLists);
   c->s_jobs.alloc((size_t)2 * kMaxChunks * nb);
   c->s_njobs.alloc(kMaxLevels);
+  c->s_halt.alloc(kMaxLevels);
   c->s_scan_blk.alloc(((size_t)nb / 256 + 2) * 16);
   c->s_id_sz.alloc(nb);
   c->s_row_sz.alloc(nb);

@@ -366,7 +366,7 @@ __device__ void decouple_tail(const R* M, const int* prow, const R* Krs, const R
 // NMAX = 64, five for NMAX = 44.
 template <typename R, int NMIN, int NMAX>
 __global__ __launch_bounds__(256) void k_decouple_small(DevGeom g, DevTree t,
-                                                        DevState s, int start) {
+                                                        DevState s, int start, int level) {
   constexpr int NT = 256;
   // >= n^2 + 2 k r (k r <= n^2 / 4); the two size classes let the boxes
   // with n <= kSmallBox1 run at a higher occupancy
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256) void k_decouple_small(DevGeom g, DevTree t,
 
   const int b = start + blockIdx.x;
   const int tid = threadIdx.x;
-  if (!pools_ok(s) || box_clean(s, b)) return;
+  if (s.halt[level] || box_clean(s, b)) return;
   const int n = s.act_cnt[b], k = s.rank[b];
   if (n > NMAX || (n <= NMIN && (NMIN > 0 || n > 0))) return;  // another kernel's box
   if (k == 0) {
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(NT) void k_decouple(DevGeom g, DevTree t,
   __shared__ int chN[4];
 
   const int tid = threadIdx.x;
-  if (!pools_ok(s)) return;
+  if (s.halt[level]) return;
   const int nl = list_count(s, level, kLstBig);
   for (int bi = blockIdx.x; bi < nl; bi += gridDim.x) {
   const int b = list_at(s, start, kLstBig, bi);
@@ -923,12 +923,12 @@ void launch_decouple(const DevGeom& g, const DevTree& t, const DevState& s, int 
                      int count, const LaunchCaps& caps, hipStream_t st, int skip,
                      hipStream_t st_big) {
   if (count >= caps.dsweep) {  // one wave per box with |active| <= 64
-    launch_decouple_sweep<R>(g, t, s, start, count, st);
+    launch_decouple_sweep<R>(g, t, s, level, start, count, st);
   } else if (count >= caps.dsplit) {
-    k_decouple_small<R, 0, kSmallBox1><<<count, 256, 0, st>>>(g, t, s, start);
-    k_decouple_small<R, kSmallBox1, kSmallBox><<<count, 256, 0, st>>>(g, t, s, start);
+    k_decouple_small<R, 0, kSmallBox1><<<count, 256, 0, st>>>(g, t, s, start, level);
+    k_decouple_small<R, kSmallBox1, kSmallBox><<<count, 256, 0, st>>>(g, t, s, start, level);
   } else {
-    k_decouple_small<R, 0, kSmallBox><<<count, 256, 0, st>>>(g, t, s, start);
+    k_decouple_small<R, 0, kSmallBox><<<count, 256, 0, st>>>(g, t, s, start, level);
   }
   // the boxes above the small-box bound on st_big when given (their
   // own stream: the two kernels touch different boxes), there with

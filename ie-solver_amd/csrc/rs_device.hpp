@@ -217,6 +217,10 @@ struct DevState {
   int64_t* fac_top;    // running factor-pool offset across levels
   int64_t* scan_blk;   // a level's per-block scan totals (16 words per 256
                        // boxes, then the factor-pool base)
+  // Per level: 1 when a pool had overflowed by its scan.  A level's decouple
+  // goes by this word and not by err, into which the ID chain of the levels
+  // above writes while it runs.
+  int* halt;
   int* err;            // [0] error bits, [1] / [2] / [3] decouple / ID / row
                        // pool size a level needed on overflow (1024 elements)
   void* root_mat;      // per root: 2 ncap^2 elements (matrix + inverse)
@@ -253,7 +257,10 @@ struct DevState {
 };
 
 // False once a pool overflow was reported: the level's remaining kernels
-// stop and the host repeats the factorization with larger pools.
+// stop and the host repeats the factorization with larger pools.  For the
+// kernels ordered behind the scans that report one (the ID chain and the
+// root): beside a running scan the waves of one workgroup may read
+// different answers.
 __device__ inline bool pools_ok(const DevState& s) {
   return (s.err[0] & (kErrIdPool | kErrRowPool | kErrFacPool | kErrBoxCap | kErrDecPool)) == 0;
 }

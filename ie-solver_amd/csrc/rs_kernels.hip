@@ -328,9 +328,10 @@ __device__ inline void scan_place(const DevState& s, const ScanBox& v, int b, in
   }
 }
 
-// The level's list lengths, pool checks and the factor-pool top.
+// The level's list lengths, pool checks and the factor-pool top.  ok:
+// pools_ok before this level.
 __device__ inline void scan_finish(const DevState& s, int level, const int64_t* tot,
-                                   int64_t fbase) {
+                                   int64_t fbase, bool ok) {
   const int64_t ta = tot[0], tb = tot[1], tc = tot[2];
   list_slot(s, level, kLstReg)[0] = (int)tot[3];
   list_slot(s, level, kLstLds)[0] = (int)tot[4];
@@ -357,6 +358,7 @@ __device__ inline void scan_finish(const DevState& s, int level, const int64_t* 
     atomicMax(s.err + 1, (int)((tot[10] + 1023) >> 10));
   }
   if (e) atomicOr(s.err, e);
+  s.halt[level] = (e != 0 || !ok) ? 1 : 0;
   *s.fac_top = fbase + tc;
 }
 
@@ -410,10 +412,11 @@ __global__ __launch_bounds__(NT) void k_scan(DevState s, int start, int count, i
   int64_t off[kScanQ];
   block_scan<NT>(own, off, wtot, tot);
   const int64_t fbase = *s.fac_top;
+  const bool pools = pools_ok(s);
   for (int i = lo; i < hi; i++)
     scan_place(s, scan_load(s, start + i), start + i, start, level, fbase, off);
   __syncthreads();
-  if (tid == 0) scan_finish(s, level, tot, fbase);
+  if (tid == 0) scan_finish(s, level, tot, fbase, pools);
 }
 
 // The same for levels of kScanMulti boxes or more over many workgroups of
@@ -457,7 +460,7 @@ __global__ __launch_bounds__(1024) void k_scan_totals(DevState s, int nblk, int 
   if (tid == 0) {
     const int64_t fbase = *s.fac_top;
     s.scan_blk[(int64_t)nblk * kScanLd] = fbase;
-    scan_finish(s, level, tot, fbase);
+    scan_finish(s, level, tot, fbase, pools_ok(s));
   }
 }
 

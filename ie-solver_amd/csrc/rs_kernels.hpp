@@ -69,8 +69,8 @@ void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
 // Decouple of one level's compressed boxes with |active| <= 64, one wave
 // per box (rs_sweep.hip); the other boxes exit at once.
 template <typename R>
-void launch_decouple_sweep(const DevGeom& g, const DevTree& t, const DevState& s, int start,
-                           int count, hipStream_t st);
+void launch_decouple_sweep(const DevGeom& g, const DevTree& t, const DevState& s, int level,
+                           int start, int count, hipStream_t st);
 
 // One level's randomized ID (rs_rid.hip), pivoted-QR ID (rs_qrcp.hip) and
 // decouple of the workgroup forms (rs_decouple.hip); `skip`, `st_big` as in

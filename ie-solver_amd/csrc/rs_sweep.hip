@@ -126,7 +126,7 @@ __device__ inline double sweep_entry(const DofGeo& t, const DofGeo& s) {
 // Boxes with nmin < |active| <= 16 NB.
 template <typename R, int PDE, int NB>
 __global__ __launch_bounds__(64, (NB <= 2 ? 4 : 2)) void k_decouple_sweep(
-    DevGeom g, DevTree t, DevState s, int start, int nmin) {
+    DevGeom g, DevTree t, DevState s, int level, int start, int nmin) {
   using V = typename Vec16<R>::T;
   using VA = typename Vec16<R>::A;
   using L = SweepLds<R, NB>;
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(64, (NB <= 2 ? 4 : 2)) void k_decouple_sweep(
 
   const int b = start + blockIdx.x;
   const int lane = threadIdx.x;
-  if (!pools_ok(s) || box_clean(s, b)) return;
+  if (s.halt[level] || box_clean(s, b)) return;
   const int n = s.act_cnt[b], k = s.rank[b];
   if (n > NMAX || (n <= nmin && (nmin > 0 || n > 0))) return;  // another launch's box
   if (k == 0) {
@@ -386,26 +386,26 @@ __global__ __launch_bounds__(64, (NB <= 2 ? 4 : 2)) void k_decouple_sweep(
 }  // namespace
 
 template <typename R>
-void launch_decouple_sweep(const DevGeom& g, const DevTree& t, const DevState& s, int start,
-                           int count, hipStream_t st) {
+void launch_decouple_sweep(const DevGeom& g, const DevTree& t, const DevState& s, int level,
+                           int start, int count, hipStream_t st) {
   if (count <= 0) return;
   // Two register classes: |active| <= 32 (two 16-entry blocks per row) and
   // 32 < |active| <= 64 (four blocks).
   if (g.pde == kPdeStokes) {
-    k_decouple_sweep<R, kPdeStokes, 2><<<count, 64, 0, st>>>(g, t, s, start, 0);
-    k_decouple_sweep<R, kPdeStokes, 4><<<count, 64, 0, st>>>(g, t, s, start, 32);
+    k_decouple_sweep<R, kPdeStokes, 2><<<count, 64, 0, st>>>(g, t, s, level, start, 0);
+    k_decouple_sweep<R, kPdeStokes, 4><<<count, 64, 0, st>>>(g, t, s, level, start, 32);
   } else if (g.pde == kPdeLaplaceNeumann) {
-    k_decouple_sweep<R, kPdeLaplaceNeumann, 2><<<count, 64, 0, st>>>(g, t, s, start, 0);
-    k_decouple_sweep<R, kPdeLaplaceNeumann, 4><<<count, 64, 0, st>>>(g, t, s, start, 32);
+    k_decouple_sweep<R, kPdeLaplaceNeumann, 2><<<count, 64, 0, st>>>(g, t, s, level, start, 0);
+    k_decouple_sweep<R, kPdeLaplaceNeumann, 4><<<count, 64, 0, st>>>(g, t, s, level, start, 32);
   } else {
-    k_decouple_sweep<R, kPdeLaplace, 2><<<count, 64, 0, st>>>(g, t, s, start, 0);
-    k_decouple_sweep<R, kPdeLaplace, 4><<<count, 64, 0, st>>>(g, t, s, start, 32);
+    k_decouple_sweep<R, kPdeLaplace, 2><<<count, 64, 0, st>>>(g, t, s, level, start, 0);
+    k_decouple_sweep<R, kPdeLaplace, 4><<<count, 64, 0, st>>>(g, t, s, level, start, 32);
   }
 }
 
 template void launch_decouple_sweep<double>(const DevGeom&, const DevTree&, const DevState&, int,
-                                            int, hipStream_t);
+                                            int, int, hipStream_t);
 template void launch_decouple_sweep<float>(const DevGeom&, const DevTree&, const DevState&, int,
-                                           int, hipStream_t);
+                                           int, int, hipStream_t);
 
 }  // namespace iegpu

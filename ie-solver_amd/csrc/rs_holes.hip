@@ -68,8 +68,9 @@ __global__ __launch_bounds__(256) void k_gram_partial(const double* P, const dou
       const int rows = (int)min((int64_t)tr, hi - r0);
       __syncthreads();
       for (int i = threadIdx.x; i < rows * h; i += 256) {
-        sp[i] = mask[r0 + i / h] ? 0.0 : P[r0 * h + i];
-        sc[i] = C[r0 * h + i];
+        const bool skel = mask[r0 + i / h] != 0;  // C is not defined there
+        sp[i] = skel ? 0.0 : P[r0 * h + i];
+        sc[i] = skel ? 0.0 : C[r0 * h + i];
       }
       __syncthreads();
       for (int i = 0; i < rows; i++)

@@ -104,7 +104,8 @@ void launch_root(const DevGeom& g, const DevTree& t, const DevState& s,
 
 // Upward sweep of one level: x_r -= T^T x_s; x_s -= L x_r (or U^T x_r when
 // `use_Ut`); then x_r = X_rr^{-1} x_r when `diag`, written to dx (laid out
-// as x) instead when it is given.
+// as x) instead when it is given: the redundant DOFs' rows of dx only, the
+// rows of the root's active DOFs stay as they were.
 template <typename R>
 void launch_sweep_up(const DevState& s, int start, int count, SolveVec v,
                      bool use_Ut, bool diag, hipStream_t st, double* dx = nullptr);

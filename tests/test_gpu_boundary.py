@@ -99,3 +99,36 @@ def test_box_factors_t_is_the_interpolative_decomposition():
         assert fac["L"].shape == (k, r) and fac["U"].shape == (r, k)
         assert fac["Xinv"].shape == (r, r) and fac["S"].shape == (k, k)
         assert np.all(np.isfinite(fac["Xinv"]))
+
+
+@pytest.mark.parametrize("pde", [iesolver.PDE_LAPLACE, iesolver.PDE_STOKES])
+def test_border_after_a_non_finite_one(pde):
+    """A context whose border products overflowed, then an ordinary border at
+    a larger tolerance, where other DOFs reach the root: as a fresh context."""
+    g = G.annulus(2000) if pde == iesolver.PDE_LAPLACE else G.circle_with_holes(2000, 4, 1)
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g, pde)
+    s.build_tree(64)
+    s.set_holes(g["holes"]["centers"], g["holes"]["radii"])
+    U, Psi = oracle.OracleProblem(g, pde).U_Psi()
+    big = 1e307 * np.sign(np.random.default_rng(1).standard_normal(U.shape))
+    s.set_border(big, Psi)
+    try:
+        s.factor(TOL)
+        assert not np.all(np.isfinite(s.solve(np.ones(s.ndof))[0]))
+    except iesolver.IeGpuError:
+        pass  # an elimination that meets only zeros and infinities may stop
+    s.set_border(U, Psi)
+    f = np.random.default_rng(2).standard_normal(s.ndof)
+    for tol in (1e-4, 1e-6, TOL):
+        s.factor(tol)
+        mu, alpha = s.solve(f)
+        t = iesolver.RSSolver(0)
+        t.set_geometry(g, pde)
+        t.build_tree(64)
+        t.set_holes(g["holes"]["centers"], g["holes"]["radii"])
+        t.set_border(U, Psi)
+        t.factor(tol)
+        mf, af = t.solve(f)
+        assert np.all(np.isfinite(mf)) and np.all(np.isfinite(af))
+        assert np.array_equal(mu, mf) and np.array_equal(alpha, af)

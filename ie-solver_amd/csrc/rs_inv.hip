@@ -14,9 +14,9 @@ namespace iegpu {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Blocked Gauss-Jordan with partial pivoting, rows not moved.  Workgroup j
-// of a block's group owns the kInvB = 16 columns of panel j, thread t the
-// rows t, t + 512, ...: a panel's 16 elimination steps run on registers
+// Blocked Gauss-Jordan with partial pivoting, rows not moved.  One
+// workgroup owns the kInvB = 16 columns of panel j, thread t the rows
+// t, t + 512, ...: a panel's 16 elimination steps run on registers
 // (pivot row: largest |entry| among the rows not yet pivoted, one barrier
 // per step), and the other columns take them at once: with W the final slab
 // of panel q and P its pivot rows' old values, the steps turn a column x
@@ -25,9 +25,11 @@ namespace {
 //
 // k_inv_panel: workgroup j applies panels 0 .. j-1 to its columns as they
 // are published, eliminates its own and publishes it (the slab over its own
-// columns of the block, the pivot rows, then the panel's flag).  It waits
-// only for workgroups of lower index in its own launch, which the
-// dispatcher starts first, so a wait ends wherever the others run.
+// columns of the block, the pivot rows, then the panel's flag).  A
+// workgroup draws its panel when it starts (a counter per block), so the
+// panels it waits for belong to workgroups that run already: the wait ends
+// whatever order the workgroups start in and whatever other launches (a
+// second context's inverses) hold the rest of the chip.
 // k_inv_finish: the columns of panel j take the panels j+1, ... (all
 // published), four columns per workgroup, and the unpermuted inverse is
 // written.
@@ -149,15 +151,18 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
   __shared__ R cand[2][kInvNW][kInvB];  // each wave's candidate row, by step parity
   __shared__ unsigned keys[2][kInvNW];
   __shared__ short pstep[kInvMax];
-  __shared__ int ok, sprow[kInvB];
+  __shared__ int ok, panel, sprow[kInvB];
   if (!pools_ok(s)) return;
-  const int root = blockIdx.y, j = blockIdx.x, j0 = j * kInvB;
+  const int root = blockIdx.x;
   const int n = s.act_cnt[root] + blk.extra;
-  if (n <= nmin || n > nmax || j0 >= n) return;
+  if (n <= nmin || n > nmax || kInvB * (int)blockIdx.y >= n) return;
   R* A = blk.a + blk.stride * root;
   int* prow = blk.piv + (int64_t)blk.piv_stride * root;
   int* flags = prow + blk.piv_stride - kInvFlags;
   const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
+  if (tid == 0) panel = atomicAdd(flags + kInvFlags - 1, 1);
+  __syncthreads();
+  const int j = __builtin_amdgcn_readfirstlane(panel), j0 = j * kInvB;
   const int bw = min(kInvB, n - j0);
   R x[RT][kInvB];
 #pragma unroll
@@ -266,7 +271,7 @@ __global__ __launch_bounds__(kInvNT) void k_inv_finish(DevState s, InvBlocks<R> 
   __shared__ R P[2][kInvB][kInvCF];
   __shared__ short pstep[kInvMax];
   if (!pools_ok(s) || (s.err[0] & kErrWait)) return;
-  const int root = blockIdx.y, c0 = blockIdx.x * kInvCF;
+  const int root = blockIdx.x, c0 = blockIdx.y * kInvCF;
   const int n = s.act_cnt[root] + blk.extra;
   if (n <= nmin || n > nmax || c0 >= n) return;
   const R* A = blk.a + blk.stride * root;
@@ -306,7 +311,7 @@ void launch_block_inverse(const DevState& s, const InvBlocks<R>& blk, int n_bloc
                           int nmax, hipStream_t st) {
   // one row per thread, or three
   const int m1 = nmax < kInvNT ? nmax : kInvNT;
-  auto grid = [&](int n, int cols) { return dim3((n + cols - 1) / cols, n_blocks); };
+  auto grid = [&](int n, int cols) { return dim3(n_blocks, (n + cols - 1) / cols); };
   if (nmin < kInvNT) {
     k_inv_panel<R, 1><<<grid(m1, kInvB), kInvNT, 0, st>>>(s, blk, nmin, m1);
     k_inv_finish<R, 1><<<grid(m1, kInvCF), kInvNT, 0, st>>>(s, blk, nmin, m1);

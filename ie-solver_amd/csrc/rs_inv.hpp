@@ -10,14 +10,16 @@
 namespace iegpu {
 
 constexpr int kInvMax = 1024 + 192;  // the largest root with 64 holes' border
-constexpr int kInvFlags = 80;        // panel flags at the end of a block's piv row
-static_assert((kInvMax + 15) / 16 <= kInvFlags, "a flag per panel");
+// Panel flags at the end of a block's piv row, the last one its counter of
+// started panels.
+constexpr int kInvFlags = 80;
+static_assert((kInvMax + 15) / 16 < kInvFlags, "a flag per panel and the counter");
 
 // Blocks b = 0 .. n_blocks - 1 of size n = act_cnt[b] + extra, column-major
 // (ld n) at a + stride b, destroyed; the inverse goes to out + stride b, or
 // behind the block (a + stride b + n^2) when out is null.  piv + piv_stride
 // b: the pivot rows (n ints) and, in its last kInvFlags ints, the panel
-// flags, zeroed before the launch.
+// flags and counter, zeroed before the launch.
 template <typename R>
 struct InvBlocks {
   R* a;

@@ -1,6 +1,8 @@
 """The solve phase at the edges of its kernels' tiles: interior evaluation
 (128 targets and 512 sources per tile), the dense inverse of root blocks
 (panels of 16 columns), and multi-column solves (16 columns at a time)."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -99,3 +101,32 @@ def test_multi_column_tiles_equal_columns(pde, leaf, prec):
         MU, _ = s.solve_many(B[:, :nrhs])
         for j in {0, 1, nrhs // 2, nrhs - 1}:
             assert np.array_equal(MU[:, j], s.solve(B[:, j])[0]), (nrhs, j)
+
+
+@pytest.mark.parametrize("prec", [iesolver.FP64, iesolver.FP32])
+def test_two_contexts_invert_roots_at_once(prec):
+    """Batches whose roots take 25 workgroups each, more than fit the card,
+    factored by two threads: each as it is factored alone, bit for bit."""
+    runs = []
+    for q in range(2):
+        s = iesolver.RSSolver(0)
+        s.set_geometry_batch([G.star(390 + p % 11, k=3 + p % 5, amp=0.1 + 0.05 * q)
+                              for p in range(64)])
+        s.build_tree(512)  # a tree of one leaf: the root block is the operator
+        f = np.random.default_rng(q).standard_normal(s.ndof)
+        s.factor(1e-10, prec)
+        runs.append((s, f, s.solve(f)[0]))
+    bad = []
+
+    def work(s, f, want):
+        for _ in range(10):
+            s.factor(1e-10, prec)
+            if not np.array_equal(s.solve(f)[0], want):
+                bad.append(1)
+
+    th = [threading.Thread(target=work, args=r) for r in runs]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad

@@ -235,7 +235,7 @@ struct iegpu_ctx {
       s_red_list, s_perm, s_rank, s_upd_kind, s_m_rows, s_row_pool, s_err,
       s_root_piv, s_qkind, s_jobs, s_njobs, s_halt, s_lists, s_lcnt, s_sk_w, s_rid_done;
   DevBuf<int64_t> s_id_sz, s_row_sz, s_fac_sz, s_id_off, s_row_off, s_fac_off,
-      s_fac_top, s_dec_sz, s_dec_off, s_scan_blk;
+      s_big_off, s_id_top, s_fac_top, s_dec_sz, s_dec_off, s_scan_blk;
   DevBuf<unsigned char> s_id_pool, s_fac_pool, s_root_mat, s_dec_pool;
   // X_rr and root blocks kept for the compressed forward apply
   bool keep_operator = false;
@@ -382,6 +382,8 @@ struct iegpu_ctx {
     s.jobs = s_jobs.p;
     s.njobs = s_njobs.p;
     s.halt = s_halt.p;
+    s.big_off = s_big_off.p;
+    s.id_top = s_id_top.p;
     s.id_sz = s_id_sz.p;
     s.row_sz = s_row_sz.p;
     s.fac_sz = s_fac_sz.p;
@@ -554,6 +556,8 @@ void alloc_state(iegpu_ctx* c) {
   c->s_row_sz.alloc(nb);
   c->s_fac_sz.alloc(nb);
   c->s_id_off.alloc(nb);
+  c->s_big_off.alloc(nb);
+  c->s_id_top.alloc(kMaxLevels);
   c->s_row_off.alloc(nb);
   c->s_fac_off.alloc(nb);
   c->s_dec_sz.alloc(nb);

@@ -87,6 +87,8 @@ enum : int { kIdOpen = 0, kIdSketch = 1, kIdGram = 2 };
 // Below, the FP32 QR's own noise (1e-7) decides the ranks: at 2e-7 it keeps
 // 1 to 5 % more columns and the Gram form's backward error was larger.
 constexpr double kGramTol = 5e-7;
+constexpr int kGramNear = 2048;  // row DOFs of a box it takes (LDS list)
+constexpr int kGramCols = 256;   // columns
 // Scratch (in FP32 elements) of a box above 64 DOFs there: G and R.
 __host__ __device__ inline int64_t gram_scratch(int n) {
   const int64_t n16 = (n + 15) / 16 * 16;
@@ -200,6 +202,8 @@ struct DevState {
   int64_t* row_sz;
   int64_t* fac_sz;
   int64_t* id_off;
+  int64_t* big_off;    // slot of the 128-row sketch: id_off, or one taken past id_top
+  int64_t* id_top;     // per level: ID scratch in use
   int64_t* row_off;
   int64_t* fac_off;
   // Operands of a general decouple (boxes above kSmallBox DOFs whose blocks

@@ -38,8 +38,6 @@ namespace {
 // against 25.1 for row compression, register and general QR and assembly.
 // ---------------------------------------------------------------------------
 
-constexpr int kGramNear = 2048;  // row DOFs of a box (LDS list)
-constexpr int kGramCols = 256;
 constexpr int kItems = 256;      // row points staged at a time
 // The cut |R_jj| < kGramCut tol |R_00|: rounding in FP32 kept the QR's
 // diagonal slightly above the exact one, and with the exact diagonal cut at

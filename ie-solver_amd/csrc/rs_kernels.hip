@@ -168,6 +168,13 @@ __global__ __launch_bounds__(64) void k_rows(DevGeom g, DevTree t, DevState s,
     int64_t scratch = kind == kQrcpLds ? ld * n : 0;
     if (kind == kQrcpStack || kind == kQrcpStack8)
       scratch = (int64_t)id_chunks(m, kind == kQrcpStack ? kRegMaxRows : kRegMaxRows8) * n * n;
+    // A box that the Gram form takes needs its G and R instead, above 64 DOFs.
+    if (s.gram && n > kRegMaxCols) {
+      if (m > 0 && n <= kGramCols && m - proxy_rows(g, level) <= 2 * kGramNear)
+        scratch = gram_scratch(n);
+    } else if (s.gram && kind == kQrcpStack) {
+      scratch = 0;
+    }
     s.id_sz[b] = scratch;
     // k_decouple keeps the operands of a box with more than kSmallBox
     // active DOFs (n^2 + r^2 + 2 r k <= 2 n^2 entries) in the decouple pool
@@ -217,11 +224,9 @@ __global__ __launch_bounds__(64) void k_rows(DevGeom g, DevTree t, DevState s,
   if (threadIdx.x == 0) {
     s.sk_w[b] = w;
     s.rid_done[b] = 0;
-    // The 128-row sketch's partial sums and rows of R, for its boxes and
-    // those a failed 64-row sketch passes on to it.
-    if (w == kRidRowsB || (w == kRidRowsW && eligb))
-      s.id_sz[b] = max(s.id_sz[b], rid_big_scratch(n));
-    if (s.gram && n > kRegMaxCols) s.id_sz[b] = max(s.id_sz[b], gram_scratch(n));
+    // The 128-row sketch's partial sums and rows of R (a box that a failed
+    // 64-row sketch passes on to it takes its slot then).
+    if (w == kRidRowsB) s.id_sz[b] = max(s.id_sz[b], rid_big_scratch(n));
     s.id_sz[b] = (s.id_sz[b] + 3) & ~int64_t(3);  // slots hold doubles
   }
   // Until its ID succeeds a box passes its active DOFs on uncompressed:
@@ -297,6 +302,7 @@ __device__ inline void scan_place(const DevState& s, const ScanBox& v, int b, in
   // Scratch of odd and even levels in separate halves: a level's ID runs
   // while the level below it is still being decoupled.
   s.id_off[b] = (level & 1) * s.id_cap + off[0];
+  s.big_off[b] = s.id_off[b];
   s.row_off[b] = off[1];
   if (v.fac < 0) {  // keeps its slot
     s.fac_sz[b] = -v.fac;
@@ -343,6 +349,7 @@ __device__ inline void scan_finish(const DevState& s, int level, const int64_t* 
   list_slot(s, level, kLstFallback)[0] = (int)tot[9];  // k_rid appends
   list_slot(s, level, kLstBig)[0] = (int)tot[12];
   s.njobs[level] = (int)tot[5];
+  s.id_top[level] = ta;
   int e = 0;
   if (ta > s.id_cap) {
     e |= kErrIdPool;

@@ -470,6 +470,17 @@ __device__ __forceinline__ void rid_wide_box(const DevGeom& g, const DevTree& t,
   if (k < 0) {
     if (j < n) {  // no cut within the sketch: a wider one or the full QRCP takes the box
       if (level <= kRidBigTop && tid == 0) {
+        // Its slot comes from what the level's scan left of the ID pool: few
+        // 64-row sketches fail, and a slot for each of them is 330 KB at 64
+        // columns.
+        const int64_t need = rid_big_scratch(n);
+        const int64_t off = (int64_t)atomicAdd(
+            reinterpret_cast<unsigned long long*>(s.id_top + level), (unsigned long long)need);
+        s.big_off[b] = (level & 1) * s.id_cap + off;
+        if (off + need > s.id_cap) {  // k_rid_big_* stop; the host repeats with more
+          atomicOr(s.err, kErrIdPool);
+          atomicMax(s.err + 2, (int)((off + need + 1023) >> 10));
+        }
         const int pos = atomicAdd(list_slot(s, level, kLstRidBig), 1);
         s.lists[(int64_t)kLstRidBig * s.nbox + start + pos] = b;
         s.sk_w[b] = kRidRowsB;
@@ -538,7 +549,7 @@ template <typename R, int PDE, bool LOOP>
 __global__ __launch_bounds__(64 * kRidWideWaves, 1) void k_rid_wide(
     DevGeom g, DevTree t, DevState s, int start, int level, double tol_d) {
   __shared__ RidWideLds<R> sh;
-  if (!pools_ok(s)) return;
+  if (s.halt[level]) return;  // not err, which this kernel's own boxes write
   const int nl = list_count(s, level, kLstRidWide);
   for (int li = blockIdx.x; li < nl; li += LOOP ? (int)gridDim.x : nl) {
     const int b = list_at(s, start, kLstRidWide, li);

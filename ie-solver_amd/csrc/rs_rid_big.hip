@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256, 2) void k_rid_big_sketch(DevGeom g, DevTree t,
     sketch_pairs<R, PDE, false, 8, kRidRowsB, 1, false>(tab, rowdofs, s.omega_b, P, 2 * cnt,
                                                         2 * cnt + P, cnt, part, kRidBigParts, cg,
                                                         acc);
-    R* Y = reinterpret_cast<R*>(s.id_pool) + s.id_off[b] + (int64_t)part * kRidRowsB * n16;
+    R* Y = reinterpret_cast<R*>(s.id_pool) + s.big_off[b] + (int64_t)part * kRidRowsB * n16;
 #pragma unroll
     for (int q = 0; q < 8; q++)
 #pragma unroll
@@ -257,8 +257,8 @@ __global__ __launch_bounds__(kBigNT) void k_rid_big_qr(DevState s, int start, in
     const int b = list_at(s, start, kLstRidBig, li);
     const int n = s.act_cnt[b];
     const int n16 = (n + 15) / 16 * 16;
-    const R* Y = reinterpret_cast<const R*>(s.id_pool) + s.id_off[b];
-    R* rr = reinterpret_cast<R*>(s.id_pool) + s.id_off[b] + (int64_t)kRidBigParts * L * n16;
+    const R* Y = reinterpret_cast<const R*>(s.id_pool) + s.big_off[b];
+    R* rr = reinterpret_cast<R*>(s.id_pool) + s.big_off[b] + (int64_t)kRidBigParts * L * n16;
     bool avail[2] = {(tid & 127) < n, (tid & 127) + 128 < n};
     const int k = n > 128 ? big_qr<R, 2>(sh, Y, rr, n, static_cast<R>(tol_d), avail)
                           : big_qr<R, 1>(sh, Y, rr, n, static_cast<R>(tol_d), avail);

@@ -142,12 +142,9 @@ __global__ __launch_bounds__(256, 5) void k_rid(DevGeom g, DevTree t, DevState s
     const R alpha = lane_value(y[0], p), xt = lane_value(tl, p);
     R beta, tau, sc;
     householder_scalars(alpha, xt, &beta, &tau, &sc);
-    // A sketch of l rows keeps l - j dimensions at step j, which shrinks
-    // |R_jj| by about sqrt((l - j) / l) against |R_00|: the cut compares
-    // |R_jj| sqrt(l / (l - j)), with a factor 2 margin, to tol |R_00|.
     if (j == 0) {
       thresh = fabs(tol * beta);
-    } else if (2 * fabs(beta) * sqrt(static_cast<R>(l) / static_cast<R>(l - j)) < thresh) {
+    } else if (sketch_diag<false>(beta, l, j) < thresh) {
       k = j;
       break;
     }
@@ -270,6 +267,13 @@ struct RidWideLds {
   int nred0;        // two QR waves: redundant columns of wave 0
 };
 
+// Fixed widths, which keep this sketch to the top levels' boxes, cut as the
+// narrow sketches do.
+template <typename R>
+__device__ inline R wide_diag(const DevState& s, R beta, int l, int j) {
+  return s.rid_mode == 2 ? sketch_diag<true>(beta, l, j) : sketch_diag<false>(beta, l, j);
+}
+
 template <typename R, int PDE, int QW, bool LOOP>
 __device__ __forceinline__ void rid_wide_box(const DevGeom& g, const DevTree& t,
                                              const DevState& s, int start, int level,
@@ -356,7 +360,7 @@ __device__ __forceinline__ void rid_wide_box(const DevGeom& g, const DevTree& t,
         const double best = fmax(kbest[2 * par], kbest[2 * par + 1]);
         const R beta = sh.hs[2 * par + (pivot_key_pos<7>(best) >> 6)][0];
         if (j == 0) thresh = fabs(static_cast<R>(tol_d) * beta);
-        else cut = 2 * fabs(beta) * sqrt(static_cast<R>(l) / static_cast<R>(l - j)) < thresh;
+        else cut = wide_diag(s, beta, l, j) < thresh;
       }
       if (cut || j >= n) __syncthreads();  // the redundant counts
     }
@@ -424,7 +428,7 @@ __device__ __forceinline__ void rid_wide_box(const DevGeom& g, const DevTree& t,
     }
     if (j == 0) {
       thresh = fabs(tol * beta);
-    } else if (2 * fabs(beta) * sqrt(static_cast<R>(l) / static_cast<R>(l - j)) < thresh) {
+    } else if (wide_diag(s, beta, l, j) < thresh) {
       k = j;
       break;
     }

@@ -181,11 +181,8 @@ __device__ __forceinline__ int big_qr(RidBigLds<R>& sh, const R* Y, R* rr, int n
     const R a1 = lane + 64 == NR * jq ? R(0) : v[lane + 64];
     R beta, tau, sc;
     householder_scalars(alpha, wave_total(a0 * a0 + a1 * a1), &beta, &tau, &sc);
-    // the cut of the 16- to 64-row sketches (rs_rid.hip)
-    if (j == 0)
-      thresh = fabs(tol * beta);
-    else if (2 * fabs(beta) * sqrt(static_cast<R>(L) / static_cast<R>(L - j)) < thresh)
-      return j;
+    if (j == 0) thresh = fabs(tol * beta);
+    else if (sketch_diag<true>(beta, L, j) < thresh) return j;
     if (tid == 0) sh.spiv[j] = p;
     // the pivot column's rows of the quarter, eight at a time (all 32 do not
     // fit the registers beside two columns)

@@ -394,7 +394,9 @@ int iegpu_autotune(iegpu_ctx* ctx, double id_tol, int precision, int reps,
  * of a Gaussian sketch Omega A of l = sketch_rows rows (16 or 32; 0: per
  * box from the rank model, iegpu_set_rank_model) with the
  * same cut applied to the sketch's R, |R_jj| scaled by 2 sqrt(l / (l - j))
- * (a sketch keeps l - j dimensions at step j); a box whose sketch shows no
+ * (a sketch keeps l - j dimensions at step j), by 2 l / (l - j) for the
+ * 128-row sketch and, with the rank model, the 64-row one (their ranks come
+ * closer to their width); a box whose sketch shows no
  * cut within l - 6 pivots falls back to the full QRCP.  Larger boxes (up
  * to 128 active DOFs and 1,280 near-field row DOFs; with the rank model on
  * every level, else on the top four) take a 64-row sketch, and on the top

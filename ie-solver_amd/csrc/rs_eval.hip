@@ -33,21 +33,29 @@ namespace {
 // k_eval_partial: 8 waves share kTargets = 128 targets, two per lane; wave
 // w takes sources 64 w .. 64 w + 63 of every staged tile of kTile, and the
 // eight waves' sums are added in wave order.  FP64 issue bounds it: a
-// Laplace pair costs ten FP64 instructions and one reciprocal (v_rcp_f64
-// with one Newton step, within two ulp; a full division alone costs as much
-// again), and two targets per lane share each source's LDS reads, which
-// one per lane would make the bound (two b128 broadcasts per pair and
-// wave).  10,000 targets x 65,536 Laplace sources: 954 us with one target
-// per thread, divisions and 320 workgroups of four waves; 353 us.
+// Laplace pair costs eight FP64 instructions and a reciprocal of five (a
+// division alone costs as much as both), and two targets per lane share each
+// source's LDS reads, which one per lane would make the bound (two b128
+// broadcasts per pair and wave).  10,000 targets x 65,536 Laplace sources:
+// 954 us with one target per thread, divisions and 320 workgroups of four
+// waves; 367 us (353 with one Newton step, which is not as accurate).
 constexpr int kTargets = 128, kTile = 512;
-// Targets past this magnitude (and NaN) take the division: |r|^2 would
-// overflow, and the Newton step turns the reciprocal's 0 into NaN.
-constexpr double kFarTarget = 1e150;
+// Points past this magnitude (and NaN) take the division: |r|^2 would
+// overflow, and the Newton steps turn the reciprocal's 0 into NaN.
+constexpr double kFar = 1e150;
+__device__ inline bool is_far(double2 p) { return !(fabs(p.x) < kFar && fabs(p.y) < kFar); }
+
+// 1 / d from v_rcp_f64 (2e8 eps off) and two Newton steps: within half an
+// eps, as the division; one step is up to 9.6 eps off (a million values).
+__device__ inline double recip_full(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(y, fma(-d, y, 1.0), y);
+  return fma(y, fma(-d, y, 1.0), y);
+}
 
 // One source's contribution at the target p, added to a: xy the point; ab
 // -w mu n / (2 pi) (Laplace), (w mu / (4 pi), 0) (Neumann) or w n / pi
-// (Stokes); m the Stokes density.  FAST: reciprocal by v_rcp_f64 and a
-// Newton step, else the IEEE division.
+// (Stokes); m the Stokes density.  FAST: recip_full, else the division.
 template <int PDE, bool FAST>
 __device__ inline void eval_pair(double2 p, double2 xy, double2 ab, double2 m, double2& a) {
   const double r0 = p.x - xy.x, r1 = p.y - xy.y;
@@ -55,7 +63,7 @@ __device__ inline void eval_pair(double2 p, double2 xy, double2 ab, double2 m, d
   if constexpr (PDE == kPdeLaplaceNeumann) {
     a.x = fma(ab.x, log(d2), a.x);  // single layer w (1/2 pi) log|r| (kernel.cpp:95-102)
   } else {
-    const double inv = FAST ? recip(d2) : 1.0 / d2;
+    const double inv = FAST ? recip_full(d2) : 1.0 / d2;
     const double rn = fma(r0, ab.x, r1 * ab.y);
     if constexpr (PDE == kPdeStokes) {
       const double pot = rn * inv * inv * fma(r0, m.x, r1 * m.y);
@@ -86,13 +94,14 @@ __global__ __launch_bounds__(kTile) void k_eval_partial(DevGeom g, int nt, const
     const int t = min(t0 + 64 * u, nt - 1);
     p[u] = make_double2(tg[2 * (int64_t)t], tg[2 * (int64_t)t + 1]);
     acc[u] = make_double2(0, 0);
-    far = far || !(fabs(p[u].x) < kFarTarget && fabs(p[u].y) < kFarTarget);
+    far = far || is_far(p[u]);
   }
-  far = __any(far);  // the same in every wave: all hold the same targets
   for (int64_t base = lo; base < hi; base += kTile) {
     const int64_t j = base + tid;
+    bool slow = far;
     if (j < hi) {
       sxy[tid] = make_double2(g.pts[2 * j], g.pts[2 * j + 1]);
+      slow = slow || is_far(sxy[tid]);
       const double n0 = g.nrm[2 * j], n1 = g.nrm[2 * j + 1], w = g.wts[j];
       if constexpr (stokes) {
         sab[tid] = make_double2(w * (1.0 / M_PI) * n0, w * (1.0 / M_PI) * n1);
@@ -106,7 +115,8 @@ __global__ __launch_bounds__(kTile) void k_eval_partial(DevGeom g, int nt, const
     }
     __syncthreads();
     const int q0 = 64 * wv, q1 = min((int64_t)q0 + 64, hi - base);
-    if (!far) {
+    // a wave's targets, and its own 64 sources of the tile
+    if (!__any(slow)) {
 #pragma unroll 4
       for (int q = q0; q < q1; q++)
 #pragma unroll
@@ -198,9 +208,9 @@ int64_t eval_scratch_need(int64_t n_points, int sol_dim, int64_t n_targets) {
 
 // At least one chunk per 8192 sources (64 at most), and more where the
 // target blocks alone leave the chip idle: enough for 1024 workgroups (four
-// per CU; a host call with 65,536 sources takes 127 us at 100 targets and
-// 124 at 1,000, against 222 and 194 with 8 chunks, 407 against 417 at
-// 10,000), while a chunk keeps a tile of sources and the partial sums stay
+// per CU; a host call with 65,536 sources takes 98 us at 100 targets and 126
+// at 1,000, against 203 and 205 with 8 chunks, 432 against 440 at 10,000),
+// while a chunk keeps a tile of sources and the partial sums stay
 // within the static scratch of the allocation-free call.
 int eval_chunks(int64_t n_points, int sol_dim, int64_t n_targets) {
   const int64_t c = std::min<int64_t>(std::max<int64_t>((n_points + 8191) / 8192, 1), 64);

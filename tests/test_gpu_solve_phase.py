@@ -130,3 +130,55 @@ def test_two_contexts_invert_roots_at_once(prec):
     for t in th:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("pde", [iesolver.PDE_LAPLACE, iesolver.PDE_STOKES])
+def test_evaluate_term_rounds_as_a_division(pde):
+    """One source: every target's single term to the roundings of its
+    operations, none of which may be a reciprocal short of full accuracy."""
+    g = G.star(600)
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g, pde)
+    sd = 2 if pde == iesolver.PDE_STOKES else 1
+    j = 77
+    mu = np.zeros(s.ndof)
+    mu[sd * j:sd * j + sd] = (0.7, 0.3)[:sd]
+    tg = G.interior_points(5, 20000, radius=0.2)
+    u = s.evaluate(tg, mu).reshape(-1, sd)
+    L = np.longdouble
+    r = tg.astype(L) - g["points"][j].astype(L)
+    n, w, m = g["normals"][j].astype(L), L(g["weights"][j]), mu[sd * j:sd * j + sd].astype(L)
+    d2, rn = (r * r).sum(1), (r * n).sum(1)
+    an = (abs(r) * abs(n)).sum(1)  # what rn's rounding is relative to
+    pi = L("3.14159265358979323846")
+    # In units of half an eps, to first order: the scaled weight 3, times n 1,
+    # r 1, the two products of a dot 2, d2 4, its reciprocal 1, the sum 1; for
+    # Stokes the reciprocal (and d2) twice, the dot with mu and the product
+    # with r besides.
+    if pde == iesolver.PDE_STOKES:
+        am = (abs(r) * abs(m)).sum(1)
+        want = (w / pi * rn * (r * m).sum(1) / d2 ** 2)[:, None] * r
+        size, c = (w / pi * an * am / d2 ** 2)[:, None] * abs(r), 3 + 1 + 1 + 2 + 10 + 1 + 2 + 1 + 4
+    else:
+        want = (-w / (2 * pi) * rn / d2 * m[0])[:, None]
+        size, c = (w / (2 * pi) * an / d2 * abs(m[0]))[:, None], 3 + 1 + 1 + 2 + 4 + 1 + 1
+    err = float((abs(u - want) / size).max()) / 2.2e-16
+    print(f"largest error {err:.1f} eps, bound {c / 2} eps", flush=True)
+    assert err <= c / 2
+
+
+def test_evaluate_far_sources():
+    """A source whose |r|^2 overflows contributes the quotient, 0."""
+    g = G.star(600)
+    tg = G.interior_points(3, 130, radius=0.2)
+    far = {k: np.array(v) for k, v in g.items() if isinstance(v, np.ndarray)}
+    far["points"][100] = [1e200, 0.5]
+    mu = np.ones(600)
+    s, t = iesolver.RSSolver(0), iesolver.RSSolver(0)
+    s.set_geometry(g)
+    t.set_geometry(far)
+    mu0 = mu.copy()
+    mu0[100] = 0
+    u, u0 = t.evaluate(tg, mu), s.evaluate(tg, mu0)
+    assert np.all(np.isfinite(u))
+    assert np.abs(u - u0).max() <= 600 * 8 * 2.3e-16 * g["weights"].max() * 25

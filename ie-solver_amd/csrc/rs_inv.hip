@@ -35,26 +35,21 @@ namespace {
 // written.
 //
 // Bound by the chain of panels (wait, one update, 16 pivot steps, publish):
-// about 16 us per panel in FP64, mostly the steps' instructions.  The root
-// of the 65,536-point star: 228 us (258 with the panels handed over through
-// agent-scope fences, every wave in every step and the pivot rows stored
-// step by step); of 16,385 Stokes points: 463 us (507).  One workgroup
-// streaming the block from L2 took 986 us for 212 DOFs and 2,984 for 393, an
-// LU in one workgroup 7,570 us for the 354-DOF bordered system of Stokes
-// with 8 holes.
+// about 17 us per panel in FP64, mostly the steps' instructions.  A block of
+// 212 DOFs takes 235 us (224 with pivots picked on nine bits of the
+// mantissa, 250 with the panels handed over through agent-scope fences,
+// every wave in every step and the pivot rows stored step by step), one of
+// 393 504 us (495, 540), and k_inv_finish 21 and 42.  One workgroup streaming
+// the block from L2 took 986 us for 212 DOFs and 2,984 for 393, an LU in one
+// workgroup 7,570 us for the 354-DOF bordered system of Stokes with 8 holes.
 // ---------------------------------------------------------------------------
 
 constexpr int kInvB = 16;       // columns of a panel
 constexpr int kInvNT = 512;     // threads: rows per pass
 constexpr int kInvCF = 4;       // columns of a k_inv_finish workgroup
 constexpr int kInvNW = kInvNT / 64;
-constexpr int kRowBits = 11;    // row index bits of a pivot key
-static_assert(kInvMax <= (1 << kRowBits) && kInvMax <= 3 * kInvNT, "rows per thread");
-
-__device__ inline unsigned mag_bits(double v) {
-  return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffffu;
-}
-__device__ inline unsigned mag_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+static_assert(kInvMax <= 3 * kInvNT, "rows per thread");
+static_assert(kInvNW == 8, "the waves' candidates fill half a DPP row");
 
 __device__ inline unsigned wave_max_u32(unsigned v) {
   v = max(v, (unsigned)dpp_i32<dpp::kQuadSwap1, 0xF>((int)v));
@@ -66,13 +61,33 @@ __device__ inline unsigned wave_max_u32(unsigned v) {
   return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// A pivot candidate's key: the leading magnitude bits above the row index
-// (a magnitude within 2^-9 of the largest may win; the smaller row on
-// ties), 0 for a row that is no candidate.
+// A pivot candidate's magnitude in two words that order as it does, the
+// first one up so that 0 is left for a row that is no candidate.  A
+// non-finite entry counts as zero: every unpivoted row stays a candidate.
+__device__ inline void pivot_words(double v, bool used, unsigned& hi, unsigned& lo) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned h = (unsigned)(b >> 32) & 0x7fffffffu;
+  const bool fin = h < 0x7ff00000u;
+  hi = used ? 0u : (fin ? h + 1 : 1u);
+  lo = fin ? (unsigned)b : 0u;
+}
+__device__ inline void pivot_words(float v, bool used, unsigned& hi, unsigned& lo) {
+  const unsigned h = __float_as_uint(v) & 0x7fffffffu;
+  hi = used ? 0u : (h < 0x7f800000u ? h + 1 : 1u);
+  lo = 0u;
+}
+
+// The first of the lanes in `lanes` with the largest (hi, lo); best: the
+// largest hi.  Lanes that share it are rare, so the low words are mostly not
+// looked at.
 template <typename R>
-__device__ inline unsigned inv_key(R v, int row) {
-  constexpr unsigned kMask = (1u << kRowBits) - 1;
-  return (mag_bits(v) & ~kMask) | (kMask - (unsigned)row);
+__device__ inline int top_lane(unsigned hi, unsigned lo, unsigned best, uint64_t lanes) {
+  uint64_t m = __ballot(hi == best) & lanes;
+  if (sizeof(R) == 8 && (m & (m - 1)) != 0) {
+    const unsigned bl = wave_max_u32(hi == best ? lo : 0u);
+    m = __ballot(hi == best && lo == bl) & lanes;
+  }
+  return __ffsll((unsigned long long)m) - 1;
 }
 
 // Wait of a workgroup for panel flag *f: bounded (about two seconds), false
@@ -149,7 +164,8 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
                                                       int nmax) {
   __shared__ R P[kInvB][kInvB];
   __shared__ R cand[2][kInvNW][kInvB];  // each wave's candidate row, by step parity
-  __shared__ unsigned keys[2][kInvNW];
+  __shared__ unsigned keyh[2][kInvNW], keyl[2][kInvNW];  // its magnitude
+  __shared__ int crow[2][kInvNW];                        // its row
   __shared__ short pstep[kInvMax];
   __shared__ int ok, panel, sprow[kInvB];
   if (!pools_ok(s)) return;
@@ -195,39 +211,53 @@ __global__ __launch_bounds__(kInvNT) void k_inv_panel(DevState s, InvBlocks<R> b
   int info = 0;
   // Waves past the block's rows only keep the barriers.
   const bool live = 64 * wv < n;
-  if (!live && lane == 0) keys[0][wv] = keys[1][wv] = 0;
+  if (!live && lane == 0) keyh[0][wv] = keyh[1][wv] = keyl[0][wv] = keyl[1][wv] = 0;
 #pragma unroll
   for (int k = 0; k < kInvB; k++) {
     if (k < bw && !live) {
       __syncthreads();
     } else if (k < bw) {
-      unsigned key = 0;
+      // The wave's candidate: the largest |entry| of the step's column among
+      // its rows not yet pivoted.
+      const int par = k & 1;
+      unsigned hi, lo;
+      int best_u = 0;
+      pivot_words(x[0][k], used[0], hi, lo);
 #pragma unroll
-      for (int u = 0; u < RT; u++)
-        key = max(key, used[u] ? 0u : inv_key(x[u][k], tid + kInvNT * u));
-      const unsigned best = wave_max_u32(key);
-      if (best != 0 && key == best) {
+      for (int u = 1; u < RT; u++) {
+        unsigned h, l;
+        pivot_words(x[u][k], used[u], h, l);
+        const bool up = h > hi || (h == hi && l > lo);
+        hi = up ? h : hi;
+        lo = up ? l : lo;
+        best_u = up ? u : best_u;
+      }
+      const unsigned best = wave_max_u32(hi);
+      if (best == 0) {
+        if (lane == 0) keyh[par][wv] = keyl[par][wv] = 0;
+      } else if (lane == top_lane<R>(hi, lo, best, ~0ull)) {
+        keyh[par][wv] = hi;
+        keyl[par][wv] = lo;
+        crow[par][wv] = tid + kInvNT * best_u;
 #pragma unroll
         for (int u = 0; u < RT; u++)
-          if (!used[u] && inv_key(x[u][k], tid + kInvNT * u) == best) {
+          if (u == best_u) {
 #pragma unroll
-            for (int c = 0; c < kInvB; c++) cand[k & 1][wv][c] = x[u][c];
+            for (int c = 0; c < kInvB; c++) cand[par][wv][c] = x[u][c];
           }
       }
-      if (lane == 0) keys[k & 1][wv] = best;
       __syncthreads();
-      unsigned top = keys[k & 1][0];
-      int tw = 0;
-#pragma unroll
-      for (int q = 1; q < kInvNW; q++) {
-        const unsigned v = keys[k & 1][q];
-        tw = v > top ? q : tw;
-        top = max(top, v);
-      }
-      const int p = (1 << kRowBits) - 1 - (int)(top & ((1u << kRowBits) - 1));
+      // the waves' candidates, eight lanes each
+      const unsigned wh = keyh[par][lane & 7], wl = keyl[par][lane & 7];
+      unsigned top = wh;
+      top = max(top, (unsigned)dpp_i32<dpp::kQuadSwap1, 0xF>((int)top));
+      top = max(top, (unsigned)dpp_i32<dpp::kQuadSwap2, 0xF>((int)top));
+      top = max(top, (unsigned)dpp_i32<dpp::kRowHalfMirror, 0xF>((int)top));
+      const int tw = top_lane<R>(wh, wl, top, 0xffull);
+      const int p = crow[par][tw];
       R rv[kInvB];
 #pragma unroll
-      for (int c = 0; c < kInvB; c++) rv[c] = cand[k & 1][tw][c];
+      for (int c = 0; c < kInvB; c++) rv[c] = cand[par][tw][c];
       const R piv = rv[k];
       if (piv == R(0) && info == 0) info = j0 + k + 1;
       const R inv = R(1) / piv;

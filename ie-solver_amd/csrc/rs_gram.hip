@@ -39,12 +39,19 @@ namespace {
 // ---------------------------------------------------------------------------
 
 constexpr int kItems = 256;      // row points staged at a time
-// The cut |R_jj| < kGramCut tol |R_00|: rounding in FP32 kept the QR's
-// diagonal slightly above the exact one, and with the exact diagonal cut at
-// tol the solve's backward error came out 6 % larger on average (stars of
-// 900 to 40,000 points, tol 1e-6, three kernels; 3 %, within the spread of
-// the 90 cases, at 0.8).
-constexpr double kGramCut = 0.8;
+// A column's squared norm is enlarged by kGramRound^2 of itself, about what
+// FP32's rounding of the entries and of the steps (2^-24 each) added to it in
+// the QR: without it T's rows at diagonals near that level grow, and the FP32
+// blocks formed with T lose more (Stokes, tolerance 1e-6: backward error of
+// the unrefined solve 5 to 8 % larger than with the QR, whatever the cut
+// between 0.5 and 1).  The cut is |R_jj| < kGramCut tol |R_00|, the factor
+// offsetting what the enlargement adds to |R_jj|.  Backward error against the
+// FP32 QR's, means over 320 stars, wavy boundaries and circles with holes of
+// 900 and 3,000 points in three kernels per tolerance: 0.70 at 5e-7, 0.94 at
+// 1e-6, 0.98 at 1e-5, 0.91 at 1e-4; ranks 1 % larger (3 % at 5e-7).
+constexpr double kGramRound = 2e-7;
+constexpr double kGramCut = 0.9;
+__device__ inline double rounded_norm2(double g) { return fma(g, kGramRound * kGramRound, g); }
 
 struct RowItems {
   double x[kItems], y[kItems], n1[kItems], n2[kItems], w[kItems], k[kItems];
@@ -198,7 +205,7 @@ __global__ __launch_bounds__(256, NMAX == 32 ? 4 : 2) void k_gram_id(DevGeom g, 
   double* G = sh.m.G;
   double* Rm = sh.m.rr;
   bool avail = lane < n;
-  double d = avail ? G[lane * LD + lane] : 0.0;
+  double d = avail ? rounded_norm2(G[lane * LD + lane]) : 0.0;
   int k = 0;
   double thresh = 0;
   const int kmax = min(m, n);
@@ -384,7 +391,7 @@ __global__ __launch_bounds__(256) void k_gram_chol(DevGeom g, DevState s, int st
     const int jl = kCholLds / n16;  // rows of R in LDS
     bool avail = tid < n;
     const int c = min(tid, n - 1);
-    double d = avail ? G[(int64_t)c * n16 + c] : 0.0;
+    double d = avail ? rounded_norm2(G[(int64_t)c * n16 + c]) : 0.0;
     double thresh = 0;
     int k = 0;
     const int kmax = min(s.m_rows[b], n);

@@ -148,7 +148,12 @@ int iegpu_set_holes(iegpu_ctx* ctx, int n_holes, const double* centers,
 /* Recursive-skeletonization factorization with ID tolerance id_tol
  * (> 0) in IEGPU_FP64 or IEGPU_FP32.  Replaces
  * SkelFactorization::skeletonize, skel_factorization.h:55
- * (skel_factorization.cpp:140-310). */
+ * (skel_factorization.cpp:140-310).  A box's rank is the first j with
+ * |R_jj| < id_tol |R_00| in the pivoted QR of its ID matrix.  In IEGPU_FP32
+ * with id_tol >= 5e-7 R comes from the matrix's FP64 Gram matrix, whose
+ * diagonal carries FP32's rounding (4e-14 of itself), and the cut is 0.9
+ * id_tol: ranks about 1 % above the FP32 QR's, which smaller tolerances
+ * use. */
 int iegpu_factor(iegpu_ctx* ctx, double id_tol, int precision);
 
 /* iegpu_factor followed by the solve x = A^{-1} b on device buffers (ndof

@@ -34,7 +34,7 @@ def test_gram_ids(pde, n, leaf):
     # the backward error bar of every form (ie_solver_test.cpp:84-95)
     assert np.linalg.norm(y - b) <= 50 * tol * np.linalg.norm(b)
     i32 = s.box_info()
-    # The cut lies at 0.8 tol of the diagonal, which the Gram matrix gives to
+    # The cut lies near 0.8 tol of the exact diagonal, which the Gram matrix gives to
     # 1e-8 of its norm (1 % of it): on the deepest level, where a leaf's ID
     # matrix is the same in every factorization, the rank lies between the
     # pivoted QR's at tolerances a little either side.
@@ -51,3 +51,25 @@ def test_gram_tolerance_limit(tol):
     b = np.random.default_rng(1).standard_normal(s.ndof)
     x, _, it, res = s.solve_refined(b, 1e-12, 10)
     assert res <= 1e-12 and it <= 5
+
+
+def test_unrefined_error_is_no_larger_than_the_qr_form():
+    """72 Stokes stars at 1e-6: the FP32 solve's backward error against the
+    FP64 one's at the same tolerance, in the mean.  23.7 is what the FP32
+    pivoted QR in the Gram form's place gave on these problems."""
+    ratio = []
+    for n in (900, 1300, 2000):
+        for k in range(3, 9):
+            for amp in (0.1, 0.14, 0.18, 0.22):
+                s = iesolver.RSSolver(0)
+                s.set_geometry(G.star(n, k=k, amp=amp), iesolver.PDE_STOKES)
+                s.build_tree(64)
+                b = np.random.default_rng(n + k).standard_normal(s.ndof)
+                err = []
+                for prec in (iesolver.FP32, iesolver.FP64):
+                    s.factor(1e-6, prec)
+                    err.append(np.linalg.norm(s.apply(s.solve(b)[0])[0] - b))
+                ratio.append(err[0] / err[1])
+    gm = float(np.exp(np.mean(np.log(ratio))))
+    print(f"FP32 / FP64 backward error: mean {gm:.1f}", flush=True)
+    assert gm <= 23.7

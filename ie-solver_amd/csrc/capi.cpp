@@ -623,10 +623,13 @@ void enqueue_factor(iegpu_ctx* c, double tol, const double* fb = nullptr,
     const int start = T.level_start[lv];
     const int count = T.level_start[lv + 1] - start;
     const int skip = c->plan_on ? c->plan_skip[lv] : 0;
+    int listed = count;  // boxes its lists can hold
+    if (c->inc_run)
+      listed = (int)std::count(c->h_dirty.begin() + start, c->h_dirty.begin() + start + count, 1);
     // the general QRCP's matrices after the sketches, for the boxes none took
     for (int stage : {kStageActive, kStageRows, kStageScan, kStageRid, kStageAssemble, kStageQrcp})
       c->prof.run(stage, lv, st, [&] {
-        launch_factor_stage<R>(stage, g, t, s, lv, start, count, tol, c->caps, st, skip);
+        launch_factor_stage<R>(stage, g, t, s, lv, start, count, listed, tol, c->caps, st, skip);
       });
     if (split) {
       HIP_TRY(hipEventRecord(c->evs[1 + lv], st));
@@ -638,8 +641,8 @@ void enqueue_factor(iegpu_ctx* c, double tol, const double* fb = nullptr,
       HIP_TRY(hipStreamWaitEvent(st, c->evs[T.n_levels + 2], 0));
     }
     c->prof.run(kStageDecouple, lv, st2, [&] {
-      launch_factor_stage<R>(kStageDecouple, g, t, s, lv, start, count, tol, c->caps, st2, skip,
-                             fork ? st : nullptr);
+      launch_factor_stage<R>(kStageDecouple, g, t, s, lv, start, count, listed, tol, c->caps, st2,
+                             skip, fork ? st : nullptr);
     });
     // After the fork the ID stream joins the decouple chain's last work and
     // runs level 1's upward sweep itself (no hop back and forth).

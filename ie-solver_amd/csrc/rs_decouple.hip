@@ -920,7 +920,7 @@ __global__ __launch_bounds__(kRootTR * kRootTC) void k_root_inv(DevState s) {
 
 template <typename R>
 void launch_decouple(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                     int count, const LaunchCaps& caps, hipStream_t st, int skip,
+                     int count, int listed, const LaunchCaps& caps, hipStream_t st, int skip,
                      hipStream_t st_big) {
   if (count >= caps.dsweep) {  // one wave per box with |active| <= 64
     launch_decouple_sweep<R>(g, t, s, level, start, count, st);
@@ -937,9 +937,9 @@ void launch_decouple(const DevGeom& g, const DevTree& t, const DevState& s, int 
   if (skip & kSkipDecBig) {
     // no such box on this level (launch plan)
   } else if (st_big) {
-    k_decouple<R, 1024><<<min(count, 512), 1024, 0, st_big>>>(g, t, s, start, level);
+    k_decouple<R, 1024><<<min(listed, 512), 1024, 0, st_big>>>(g, t, s, start, level);
   } else {
-    k_decouple<R, 256><<<min(count, 512), 256, 0, st>>>(g, t, s, start, level);
+    k_decouple<R, 256><<<min(listed, 512), 256, 0, st>>>(g, t, s, start, level);
   }
 }
 
@@ -968,7 +968,7 @@ void launch_root(const DevGeom& g, const DevTree& t, const DevState& s,
 
 #define IEGPU_INSTANTIATE_DEC(R)                                                            \
   template void launch_decouple<R>(const DevGeom&, const DevTree&, const DevState&, int, int, \
-                                   int, const LaunchCaps&, hipStream_t, int, hipStream_t);  \
+                                   int, int, const LaunchCaps&, hipStream_t, int, hipStream_t);  \
   template void launch_root<R>(const DevGeom&, const DevTree&, const DevState&, int, bool,  \
                                hipStream_t);
 

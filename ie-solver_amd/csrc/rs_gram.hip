@@ -493,13 +493,13 @@ __global__ __launch_bounds__(256) void k_gram_chol(DevGeom g, DevState s, int st
 
 template <typename R, int PDE>
 void launch_gram_pde(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                     int count, double tol, hipStream_t st, int skip) {
+                     int listed, double tol, hipStream_t st, int skip) {
   if (!(skip & kSkipRegQrcp)) {
-    k_gram_id<R, PDE, 32><<<count, 256, 0, st>>>(g, t, s, start, level, tol);
-    k_gram_id<R, PDE, 64><<<count, 256, 0, st>>>(g, t, s, start, level, tol);
+    k_gram_id<R, PDE, 32><<<listed, 256, 0, st>>>(g, t, s, start, level, tol);
+    k_gram_id<R, PDE, 64><<<listed, 256, 0, st>>>(g, t, s, start, level, tol);
   }
   if (!(skip & kSkipReg8Qrcp) || !(skip & kSkipAssemble)) {
-    const int nb = count < 256 ? count : 256, blocks = kGramCols / 32;
+    const int nb = listed < 256 ? listed : 256, blocks = kGramCols / 32;
     k_gram_blocks<R, PDE>
         <<<dim3(nb, blocks * (blocks + 1) / 2), 256, 0, st>>>(g, t, s, start, level);
     k_gram_chol<R><<<nb, 256, 0, st>>>(g, s, start, level, tol);
@@ -510,13 +510,13 @@ void launch_gram_pde(const DevGeom& g, const DevTree& t, const DevState& s, int 
 
 template <typename R>
 void launch_gram(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                 int count, double tol, hipStream_t st, int skip) {
+                 int listed, double tol, hipStream_t st, int skip) {
   if (g.pde == kPdeStokes)
-    launch_gram_pde<R, kPdeStokes>(g, t, s, level, start, count, tol, st, skip);
+    launch_gram_pde<R, kPdeStokes>(g, t, s, level, start, listed, tol, st, skip);
   else if (g.pde == kPdeLaplaceNeumann)
-    launch_gram_pde<R, kPdeLaplaceNeumann>(g, t, s, level, start, count, tol, st, skip);
+    launch_gram_pde<R, kPdeLaplaceNeumann>(g, t, s, level, start, listed, tol, st, skip);
   else
-    launch_gram_pde<R, kPdeLaplace>(g, t, s, level, start, count, tol, st, skip);
+    launch_gram_pde<R, kPdeLaplace>(g, t, s, level, start, listed, tol, st, skip);
 }
 
 template void launch_gram<float>(const DevGeom&, const DevTree&, const DevState&, int, int, int,

@@ -540,9 +540,9 @@ void launch_reset(const DevState& s, hipStream_t st) {
 template <typename R>
 void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
                          const DevState& s, int level, int start, int count,
-                         double tol, const LaunchCaps& caps, hipStream_t st, int skip,
+                         int listed, double tol, const LaunchCaps& caps, hipStream_t st, int skip,
                          hipStream_t st_big) {
-  if (count <= 0) return;
+  if (count <= 0 || listed <= 0) return;
   switch (stage) {
     case kStageActive:
       k_active<<<count, 64, 0, st>>>(t, s, start);
@@ -566,25 +566,25 @@ void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
       break;
     case kStageAssemble:
       if (!(skip & kSkipAssemble) && !s.gram)
-        k_assemble<R><<<min(count, caps.assemble), 256, 0, st>>>(g, t, s, start, level);
+        k_assemble<R><<<min(listed, caps.assemble), 256, 0, st>>>(g, t, s, start, level);
       break;
     case kStageRid:
-      if (s.rid_mode != 0) launch_rid<R>(g, t, s, level, start, count, tol, st, skip);
+      if (s.rid_mode != 0) launch_rid<R>(g, t, s, level, start, listed, tol, st, skip);
       break;
     case kStageQrcp:
       if constexpr (sizeof(R) == 4) {
         if (s.gram) {
-          launch_gram<R>(g, t, s, level, start, count, tol, st, skip);
+          launch_gram<R>(g, t, s, level, start, listed, tol, st, skip);
           if (skip & kSkipAssemble) break;
           // the boxes too large for it
-          k_assemble<R><<<min(count, caps.assemble), 256, 0, st>>>(g, t, s, start, level);
+          k_assemble<R><<<min(listed, caps.assemble), 256, 0, st>>>(g, t, s, start, level);
           skip |= kSkipRegQrcp | kSkipReg8Qrcp;
         }
       }
-      launch_qrcp<R>(g, t, s, level, start, count, tol, caps, st, skip);
+      launch_qrcp<R>(g, t, s, level, start, listed, tol, caps, st, skip);
       break;
     case kStageDecouple:
-      launch_decouple<R>(g, t, s, level, start, count, caps, st, skip, st_big);
+      launch_decouple<R>(g, t, s, level, start, count, listed, caps, st, skip, st_big);
       break;
     default:
       break;
@@ -593,8 +593,8 @@ void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
 
 #define IEGPU_INSTANTIATE(R)                                                   \
   template void launch_factor_stage<R>(int, const DevGeom&, const DevTree&,   \
-                                       const DevState&, int, int, int, double, \
-                                       const LaunchCaps&, hipStream_t, int,    \
+                                       const DevState&, int, int, int, int,    \
+                                       double, const LaunchCaps&, hipStream_t, int, \
                                        hipStream_t);
 
 IEGPU_INSTANTIATE(double)

@@ -57,13 +57,16 @@ struct LaunchCaps {
 };
 constexpr int kNumCaps = 8;
 
-// `skip`: kSkip* bits of kernels not to launch (their lists are empty by
-// the launch plan, which k_root verifies).  `st_big`: the decouple stage's
+// `listed`: the most boxes a list of the level can hold (its boxes, or in an
+// incremental run the marked ones; 0: nothing to do on it), which the grids
+// of the kernels that walk a list go by.  `skip`: kSkip* bits of kernels not
+// to launch (their lists are empty by the launch plan, which k_root
+// verifies).  `st_big`: the decouple stage's
 // boxes above 64 DOFs go on this stream when given (the caller orders it).
 template <typename R>
 void launch_factor_stage(int stage, const DevGeom& g, const DevTree& t,
                          const DevState& s, int level, int start, int count,
-                         double tol, const LaunchCaps& caps, hipStream_t st,
+                         int listed, double tol, const LaunchCaps& caps, hipStream_t st,
                          int skip = 0, hipStream_t st_big = nullptr);
 
 // Decouple of one level's compressed boxes with |active| <= 64, one wave
@@ -73,28 +76,28 @@ void launch_decouple_sweep(const DevGeom& g, const DevTree& t, const DevState& s
                            int start, int count, hipStream_t st);
 
 // One level's randomized ID (rs_rid.hip), pivoted-QR ID (rs_qrcp.hip) and
-// decouple of the workgroup forms (rs_decouple.hip); `skip`, `st_big` as in
-// launch_factor_stage.
+// decouple of the workgroup forms (rs_decouple.hip); `listed`, `skip`,
+// `st_big` as in launch_factor_stage.
 template <typename R>
 void launch_rid(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                int count, double tol, hipStream_t st, int skip);
+                int listed, double tol, hipStream_t st, int skip);
 template <typename R>
 void launch_qrcp(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                 int count, double tol, const LaunchCaps& caps, hipStream_t st, int skip);
+                 int listed, double tol, const LaunchCaps& caps, hipStream_t st, int skip);
 // The full IDs of an FP32 level from Gram matrices (rs_gram.hip), but for
 // boxes above 256 DOFs or 2,048 row DOFs.
 template <typename R>
 void launch_gram(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                 int count, double tol, hipStream_t st, int skip);
+                 int listed, double tol, hipStream_t st, int skip);
 template <typename R>
 void launch_decouple(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                     int count, const LaunchCaps& caps, hipStream_t st, int skip,
+                     int count, int listed, const LaunchCaps& caps, hipStream_t st, int skip,
                      hipStream_t st_big);
 
 // Randomized ID of a level's kLstRidBig boxes (rs_rid_big.hip).
 template <typename R>
 void launch_rid_big(const DevGeom& g, const DevTree& t, const DevState& s, int start, int level,
-                    int count, double tol, hipStream_t st);
+                    int listed, double tol, hipStream_t st);
 
 // Roots (slots 0 .. n_roots-1, one per problem): active list, dense
 // skeleton block, inverse.

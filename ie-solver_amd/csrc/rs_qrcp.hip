@@ -804,22 +804,22 @@ __global__ __launch_bounds__(NT) void k_qrcp(DevState s, int start, int level, d
 
 template <typename R>
 void launch_qrcp(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                 int count, double tol, const LaunchCaps& caps, hipStream_t st, int skip) {
+                 int listed, double tol, const LaunchCaps& caps, hipStream_t st, int skip) {
   // A register-QRCP kernel whose grid covers its whole list (known from
-  // the level's box count) runs one box per workgroup, without the
+  // the level's box listed) runs one box per workgroup, without the
   // grid-stride loop and the registers it keeps live (no spills).
-  const int jobs_max = count * kMaxChunks;
+  const int jobs_max = listed * kMaxChunks;
   if (skip & kSkipRegQrcp) {
     // no register-QRCP box on this level (launch plan)
   } else if (s.rid_mode != 0) {
     // Only the boxes without a successful sketch reach the full QRCP.
     k_rowcomp<R, 4><<<min(jobs_max, caps.rowcomp4), kXThreads, 0, st>>>(g, t, s, start,
                                                                         level);
-    if (count <= min(kQrcpPairBoxes, caps.qrcp_id)) {
-      k_qrcp_pair<R><<<count, kXThreads, 0, st>>>(g, t, s, start, level, tol);
-    } else if (count <= caps.qrcp_id) {
-      k_qrcp_id<R, 4, 8, 8, true, false><<<count, 512, 0, st>>>(g, t, s, start, level, tol);
-      k_qrcp_id<R, 4, 8, 16, true, false><<<count, kXThreads, 0, st>>>(g, t, s, start,
+    if (listed <= min(kQrcpPairBoxes, caps.qrcp_id)) {
+      k_qrcp_pair<R><<<listed, kXThreads, 0, st>>>(g, t, s, start, level, tol);
+    } else if (listed <= caps.qrcp_id) {
+      k_qrcp_id<R, 4, 8, 8, true, false><<<listed, 512, 0, st>>>(g, t, s, start, level, tol);
+      k_qrcp_id<R, 4, 8, 16, true, false><<<listed, kXThreads, 0, st>>>(g, t, s, start,
                                                                        level, tol);
     } else {
       const int grid = caps.qrcp_id;
@@ -827,27 +827,27 @@ void launch_qrcp(const DevGeom& g, const DevTree& t, const DevState& s, int leve
       k_qrcp_id<R, 4, 8, 16, true><<<grid, kXThreads, 0, st>>>(g, t, s, start, level, tol);
     }
   } else {
-    k_rowcomp<R, 4><<<min(2 * count, caps.rowcomp4), kXThreads, 0, st>>>(g, t, s, start,
+    k_rowcomp<R, 4><<<min(2 * listed, caps.rowcomp4), kXThreads, 0, st>>>(g, t, s, start,
                                                                         level);
-    if (count <= kQrcpPairBoxes) {
-      k_qrcp_pair<R><<<count, kXThreads, 0, st>>>(g, t, s, start, level, tol);
+    if (listed <= kQrcpPairBoxes) {
+      k_qrcp_pair<R><<<listed, kXThreads, 0, st>>>(g, t, s, start, level, tol);
     } else {
-      k_qrcp_id<R, 4, 8, 8, false><<<count, 512, 0, st>>>(g, t, s, start, level, tol);
-      k_qrcp_id<R, 4, 8, 16, false><<<count, kXThreads, 0, st>>>(g, t, s, start, level, tol);
+      k_qrcp_id<R, 4, 8, 8, false><<<listed, 512, 0, st>>>(g, t, s, start, level, tol);
+      k_qrcp_id<R, 4, 8, 16, false><<<listed, kXThreads, 0, st>>>(g, t, s, start, level, tol);
     }
   }
   if (!(skip & kSkipReg8Qrcp)) {
-    k_rowcomp<R, 8><<<min(2 * count, caps.rowcomp8), kXThreads, 0, st>>>(g, t, s, start,
+    k_rowcomp<R, 8><<<min(2 * listed, caps.rowcomp8), kXThreads, 0, st>>>(g, t, s, start,
                                                                         level);
-    if (count <= caps.qrcp_id8)
-      k_qrcp_id<R, 8, 4, 16, true, false><<<count, kXThreads, 0, st>>>(g, t, s, start,
+    if (listed <= caps.qrcp_id8)
+      k_qrcp_id<R, 8, 4, 16, true, false><<<listed, kXThreads, 0, st>>>(g, t, s, start,
                                                                        level, tol);
     else
       k_qrcp_id<R, 8, 4, 16, true><<<caps.qrcp_id8, kXThreads, 0, st>>>(g, t, s, start,
                                                                         level, tol);
   }
   if (!(skip & kSkipAssemble))
-    k_qrcp<R, 512><<<min(count, caps.qrcp), 512, 0, st>>>(s, start, level, tol);
+    k_qrcp<R, 512><<<min(listed, caps.qrcp), 512, 0, st>>>(s, start, level, tol);
 }
 
 template void launch_qrcp<double>(const DevGeom&, const DevTree&, const DevState&, int, int, int,

@@ -589,9 +589,9 @@ void launch_gaussian(double* out, int64_t n, uint64_t seed, hipStream_t st) {
 
 template <typename R, int PDE>
 void launch_rid_wide(const DevGeom& g, const DevTree& t, const DevState& s, int start,
-                     int level, int count, double tol, hipStream_t st) {
-  if (count <= kRidWideGrid)
-    k_rid_wide<R, PDE, false><<<count, 64 * kRidWideWaves, 0, st>>>(g, t, s, start, level, tol);
+                     int level, int listed, double tol, hipStream_t st) {
+  if (listed <= kRidWideGrid)
+    k_rid_wide<R, PDE, false><<<listed, 64 * kRidWideWaves, 0, st>>>(g, t, s, start, level, tol);
   else
     k_rid_wide<R, PDE, true>
         <<<kRidWideGrid, 64 * kRidWideWaves, 0, st>>>(g, t, s, start, level, tol);
@@ -599,27 +599,27 @@ void launch_rid_wide(const DevGeom& g, const DevTree& t, const DevState& s, int 
 
 template <typename R>
 void launch_rid(const DevGeom& g, const DevTree& t, const DevState& s, int level, int start,
-                int count, double tol, hipStream_t st, int skip) {
+                int listed, double tol, hipStream_t st, int skip) {
   if (skip & kSkipRid) {
     // no 16- or 32-row sketch on this level (launch plan)
   } else if (g.pde == kPdeStokes) {
-    k_rid<R, kPdeStokes><<<count, 256, 0, st>>>(g, t, s, start, level, tol);
+    k_rid<R, kPdeStokes><<<listed, 256, 0, st>>>(g, t, s, start, level, tol);
   } else if (g.pde == kPdeLaplaceNeumann) {
-    k_rid<R, kPdeLaplaceNeumann><<<count, 256, 0, st>>>(g, t, s, start, level, tol);
+    k_rid<R, kPdeLaplaceNeumann><<<listed, 256, 0, st>>>(g, t, s, start, level, tol);
   } else {
-    k_rid<R, kPdeLaplace><<<count, 256, 0, st>>>(g, t, s, start, level, tol);
+    k_rid<R, kPdeLaplace><<<listed, 256, 0, st>>>(g, t, s, start, level, tol);
   }
   if (!(skip & kSkipRidWide)) {
     if (g.pde == kPdeStokes)
-      launch_rid_wide<R, kPdeStokes>(g, t, s, start, level, count, tol, st);
+      launch_rid_wide<R, kPdeStokes>(g, t, s, start, level, listed, tol, st);
     else if (g.pde == kPdeLaplaceNeumann)
-      launch_rid_wide<R, kPdeLaplaceNeumann>(g, t, s, start, level, count, tol, st);
+      launch_rid_wide<R, kPdeLaplaceNeumann>(g, t, s, start, level, listed, tol, st);
     else
-      launch_rid_wide<R, kPdeLaplace>(g, t, s, start, level, count, tol, st);
+      launch_rid_wide<R, kPdeLaplace>(g, t, s, start, level, listed, tol, st);
   }
   // after the 64-row sketches, whose failures it takes
   if (level <= kRidBigTop && !(skip & kSkipRidBig))
-    launch_rid_big<R>(g, t, s, start, level, count, tol, st);
+    launch_rid_big<R>(g, t, s, start, level, listed, tol, st);
 }
 
 template void launch_rid<double>(const DevGeom&, const DevTree&, const DevState&, int, int, int,

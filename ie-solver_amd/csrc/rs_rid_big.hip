@@ -345,8 +345,8 @@ constexpr int kBigGrid = 256;  // boxes of the list in flight
 
 template <typename R>
 void launch_rid_big(const DevGeom& g, const DevTree& t, const DevState& s, int start, int level,
-                    int count, double tol, hipStream_t st) {
-  const int nb = count < kBigGrid ? count : kBigGrid;
+                    int listed, double tol, hipStream_t st) {
+  const int nb = listed < kBigGrid ? listed : kBigGrid;
   const dim3 grid(nb, kRidBigCols / 64, kRidBigParts);
   if (g.pde == kPdeStokes)
     k_rid_big_sketch<R, kPdeStokes><<<grid, 256, 0, st>>>(g, t, s, start, level);

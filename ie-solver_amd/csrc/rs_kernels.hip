@@ -211,12 +211,17 @@ __global__ __launch_bounds__(64) void k_rows(DevGeom g, DevTree t, DevState s,
       // past 26 below the top levels, where boxes are many and the register
       // QRCP takes them, and a box none is eligible for go straight to the
       // full QRCP.  The 64-row sketch is tried without the margin: a box it
-      // fails goes on to the 128-row one, which costs three times as much.
+      // fails goes on to the 128-row one, which costs more than as much
+      // again.  For Laplace, whose ranks of 48 to 54 on level 1 the model
+      // puts at 57 to 62, it is tried up to 14 past its limit (262,144 points:
+      // 2.79 ms per factorization with those boxes sent straight to the
+      // 128-row sketch, 2.62 so; an incremental one 2.36 and 2.14).
+      const float kw = kRidRowsW - kRidOver + (g.pde == kPdeLaplace ? 14 : 0);
       const float kp = mlp_rank(s.rank_model, f, hb) + (float)s.rid_margin;
       w = (elig && kp <= 16 - kRidOver) ? 16
           : (elig && kp <= kRidRows - kRidOver) ? kRidRows
           : (elig && level > kRidBigTop) ? 0
-          : (eligw && (kp - s.rid_margin <= kRidRowsW - kRidOver || !eligb)) ? kRidRowsW
+          : (eligw && (kp - s.rid_margin <= kw || !eligb)) ? kRidRowsW
           : eligb ? kRidRowsB
                   : 0;
     }

@@ -259,8 +259,9 @@ struct iegpu_ctx {
   bool have_model = false, record_features = false;
   int rid_margin = 0;
   DevBuf<float> d_model, d_feat, m_X, m_y, m_work;
-  DevBuf<double> d_work;  // solve vector for host-pointer solves
-  DevBuf<double> d_cols;  // its column-major form with several columns
+  DevBuf<double> d_work;  // solve vector for host-pointer solves (with several
+                          // columns the row-major form of up to 256 of them)
+  DevBuf<double> d_cols;  // right-hand sides of a multi-column solve
   // iterative refinement: b, x, residual / correction (ndof), border parts,
   // reduction partials
   DevBuf<double> r_b, r_x, r_r, r_a, r_ra, r_part;
@@ -1813,22 +1814,23 @@ int iegpu_solve_nrhs(iegpu_ctx* c, int nrhs, const double* b, double* mu, double
                                hipMemcpyDeviceToHost, st));
       }
     } else {
-      // every column through each sweep kernel in one pass, row-major there
-      // (a DOF's columns share its cache lines)
-      double* cols = nullptr;
-      c->d_work.alloc(nd * nrhs);
-      double* rows = c->d_work.p;
-      if (nrhs > 1) {
-        c->d_cols.alloc(nd * nrhs);
-        cols = c->d_cols.p;
-      } else {
-        cols = rows;
-      }
+      // up to kColumns columns through each sweep kernel in one pass,
+      // row-major there (a DOF's columns share its cache lines); the sweeps
+      // take 16 at a time, so more in a pass would only grow the copy
+      constexpr int kColumns = 256;
+      c->d_cols.alloc(nd * nrhs);
+      double* cols = c->d_cols.p;
       HIP_TRY(hipMemcpyAsync(cols, b, nd * nrhs * sizeof(double), hipMemcpyHostToDevice, st));
-      if (nrhs > 1) launch_transpose(rows, cols, nd, nrhs, true, st);
-      if (c->precision == IEGPU_FP32) enqueue_solve<float>(c, rows, nullptr, st, nullptr, nrhs);
-      else enqueue_solve<double>(c, rows, nullptr, st, nullptr, nrhs);
-      if (nrhs > 1) launch_transpose(cols, rows, nd, nrhs, false, st);
+      if (nrhs > 1) c->d_work.alloc(nd * std::min(nrhs, kColumns));
+      for (int q = 0; q < nrhs; q += kColumns) {
+        const int nq = std::min(kColumns, nrhs - q);
+        double* part = cols + nd * q;
+        double* rows = nrhs > 1 ? c->d_work.p : part;
+        if (nrhs > 1) launch_transpose(rows, part, nd, nq, true, st);
+        if (c->precision == IEGPU_FP32) enqueue_solve<float>(c, rows, nullptr, st, nullptr, nq);
+        else enqueue_solve<double>(c, rows, nullptr, st, nullptr, nq);
+        if (nrhs > 1) launch_transpose(part, rows, nd, nq, false, st);
+      }
       HIP_TRY(hipGetLastError());
       HIP_TRY(hipMemcpyAsync(mu, cols, nd * nrhs * sizeof(double), hipMemcpyDeviceToHost, st));
     }

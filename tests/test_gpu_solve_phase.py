@@ -182,3 +182,31 @@ def test_evaluate_far_sources():
     u, u0 = t.evaluate(tg, mu), s.evaluate(tg, mu0)
     assert np.all(np.isfinite(u))
     assert np.abs(u - u0).max() <= 600 * 8 * 2.3e-16 * g["weights"].max() * 25
+
+
+@pytest.mark.parametrize("nrhs", [1, 256, 257, 512, 530])
+def test_many_columns_in_pieces(nrhs):
+    """Columns are swept up to 256 at once: every one as solved alone."""
+    s = iesolver.RSSolver(0)
+    s.set_geometry(G.star(700))
+    s.build_tree(64)
+    s.factor(1e-10)
+    B = np.random.default_rng(4).standard_normal((s.ndof, nrhs))
+    MU, _ = s.solve_many(B)
+    for j in sorted({0, nrhs // 2, min(255, nrhs - 1), min(256, nrhs - 1), nrhs - 1}):
+        assert np.array_equal(MU[:, j], s.solve(B[:, j])[0]), j
+
+
+def test_multi_column_workspace():
+    """One copy of the right-hand sides on the device and a bounded piece of
+    them: a solve that fits the card with its columns does so still."""
+    import torch
+    s = iesolver.RSSolver(0)
+    s.set_geometry(G.star(2048))
+    s.build_tree(64)
+    s.factor(1e-10)
+    B = np.zeros((2048, 16384), order="F")
+    B[:, ::1000] = 1.0
+    free0 = torch.cuda.mem_get_info()[0]
+    s.solve_many(B)
+    assert free0 - torch.cuda.mem_get_info()[0] <= 1.25 * B.nbytes

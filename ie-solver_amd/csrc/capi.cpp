@@ -265,6 +265,9 @@ struct iegpu_ctx {
   // iterative refinement: b, x, residual / correction (ndof), border parts,
   // reduction partials
   DevBuf<double> r_b, r_x, r_r, r_a, r_ra, r_part;
+  // partial sums of the border products there: d_partial belongs to solves,
+  // which may run on a caller's stream at the same time
+  DevBuf<double> r_border;
   // FP64 operator form (iegpu_set_matvec) and the FMM's tree, translation
   // tables and expansions
   int mv_method = IEGPU_MATVEC_AUTO, fmm_order = 48, fmm_leaf = 64;
@@ -2168,6 +2171,7 @@ int iegpu_solve_refined(iegpu_ctx* c, const double* b, double* x, double* alpha,
     if (h > 0) {
       c->r_a.alloc(h);
       c->r_ra.alloc(h);
+      c->r_border.alloc((size_t)border_partials(nd, h));
     }
     std::vector<double> part(2 * nres);
     auto solve = [&](double* v, double* a, const double* g) {
@@ -2183,7 +2187,7 @@ int iegpu_solve_refined(iegpu_ctx* c, const double* b, double* x, double* alpha,
       // r = b - A x  (A bordered by [U; Psi, -I] with holes)
       enqueue_matvec(c, c->r_x.p, c->r_r.p, st);
       if (h > 0)
-        launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->d_partial.p,
+        launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->r_border.p,
                             c->r_r.p, c->r_ra.p, st);
       launch_residual(c->r_b.p, c->r_r.p, nd, c->r_part.p, st);
       HIP_TRY(hipMemcpyAsync(part.data(), c->r_part.p, sizeof(double) * 2 * nres,
@@ -2243,7 +2247,8 @@ int iegpu_apply(iegpu_ctx* c, const double* x, const double* alpha, double* y,
     if (h > 0 && alpha && z) {
       c->r_a.upload(alpha, h, st);
       c->r_ra.alloc(h);
-      launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->d_partial.p,
+      c->r_border.alloc((size_t)border_partials(nd, h));
+      launch_border_apply(c->d_U.p, c->d_PsiT.p, c->r_x.p, c->r_a.p, nd, h, c->r_border.p,
                           c->r_r.p, c->r_ra.p, st);
       HIP_TRY(hipMemcpyAsync(z, c->r_ra.p, sizeof(double) * h, hipMemcpyDeviceToHost, st));
     }

@@ -36,11 +36,10 @@ namespace {
 //
 // Bound by the chain of panels (wait, one update, 16 pivot steps, publish):
 // about 17 us per panel in FP64, mostly the steps' instructions.  A block of
-// 212 DOFs takes 235 us (224 with pivots picked on nine bits of the
-// mantissa, 250 with the panels handed over through agent-scope fences,
-// every wave in every step and the pivot rows stored step by step), one of
-// 393 504 us (495, 540), and k_inv_finish 21 and 42.  One workgroup streaming
-// the block from L2 took 986 us for 212 DOFs and 2,984 for 393, an LU in one
+// 212 DOFs takes 235 us and one of 393 504 us, k_inv_finish 21 and 42 (with
+// the panels handed over through agent-scope fences, every wave in every
+// step and the pivot rows stored step by step both kernels took 258 and 507
+// us where they took 228 and 463 without).  One workgroup streaming the block from L2 took 986 us for 212 DOFs and 2,984 for 393, an LU in one
 // workgroup 7,570 us for the 354-DOF bordered system of Stokes with 8 holes.
 // ---------------------------------------------------------------------------
 

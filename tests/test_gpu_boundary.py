@@ -12,6 +12,7 @@ and per-box factor read-back, on the GPU.
 """
 import numpy as np
 import pytest
+import torch
 
 import geometry as G
 import iesolver
@@ -132,3 +133,25 @@ def test_border_after_a_non_finite_one(pde):
         mf, af = t.solve(f)
         assert np.all(np.isfinite(mf)) and np.all(np.isfinite(af))
         assert np.array_equal(mu, mf) and np.array_equal(alpha, af)
+
+
+def test_apply_beside_a_solve_on_another_stream():
+    """A solve with holes on the caller's stream and the operator on the
+    context's, unordered: they share no scratch."""
+    g = G.circle_with_holes(30000, 8, 1)
+    s = _solver(g, iesolver.PDE_STOKES)
+    rng = np.random.default_rng(6)
+    b, x, a = (rng.standard_normal(k) for k in (s.ndof, s.ndof, 24))
+    mu, alpha = s.solve(b)
+    y, z = s.apply(x, a)
+    st = torch.cuda.Stream()
+    db = torch.from_numpy(b).cuda()
+    torch.cuda.synchronize()
+    for _ in range(20):
+        dm, da = torch.empty_like(db), torch.empty(24, dtype=torch.float64, device="cuda")
+        st.wait_stream(torch.cuda.current_stream())
+        s.solve_device(db.data_ptr(), dm.data_ptr(), da.data_ptr(), st.cuda_stream)
+        y2, z2 = s.apply(x, a)
+        st.synchronize()
+        assert np.array_equal(y2, y) and np.array_equal(z2, z)
+        assert np.array_equal(dm.cpu().numpy(), mu) and np.array_equal(da.cpu().numpy(), alpha)

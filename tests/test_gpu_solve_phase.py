@@ -5,6 +5,7 @@ import threading
 
 import numpy as np
 import pytest
+import torch
 
 import geometry as G
 import iesolver
@@ -200,7 +201,6 @@ def test_many_columns_in_pieces(nrhs):
 def test_multi_column_workspace():
     """One copy of the right-hand sides on the device and a bounded piece of
     them: a solve that fits the card with its columns does so still."""
-    import torch
     s = iesolver.RSSolver(0)
     s.set_geometry(G.star(2048))
     s.build_tree(64)

@@ -155,3 +155,44 @@ def test_apply_beside_a_solve_on_another_stream():
         st.synchronize()
         assert np.array_equal(y2, y) and np.array_equal(z2, z)
         assert np.array_equal(dm.cpu().numpy(), mu) and np.array_equal(da.cpu().numpy(), alpha)
+
+
+# Border widths of 5, 33, 64, 66 and 192 (the products' row lanes are 256 / h,
+# the Gram matrix takes 1,024 of its h^2 sums per pass, 4,096 rows of a block
+# at a time and past h = 48 4,096 per workgroup), DOF counts one and two past
+# a multiple of the chunks, bordered systems past the inverse's 512 rows.
+@pytest.mark.parametrize("pde,n,h,real", [
+    (iesolver.PDE_LAPLACE, 2049, 5, True), (iesolver.PDE_LAPLACE, 3000, 33, True),
+    (iesolver.PDE_LAPLACE, 4097, 64, False), (iesolver.PDE_STOKES, 3000, 11, True),
+    (iesolver.PDE_STOKES, 1537, 22, False), (iesolver.PDE_STOKES, 2049, 64, False)])
+def test_border_widths_against_the_dense_system(pde, n, h, real):
+    rng = np.random.default_rng(h)
+    if real:
+        g = G.circle_with_holes(n, h, 1)
+        c, r = g["holes"]["centers"], g["holes"]["radii"]
+    else:  # a simple boundary with a border of the caller's
+        g = G.star(n)
+        c, r = 0.5 + 0.01 * rng.standard_normal((h, 2)), np.full(h, 0.001)
+    s = iesolver.RSSolver(0)
+    s.set_geometry(g, pde)
+    s.build_tree(64)
+    s.set_holes(c, r)
+    hd = h * (3 if pde == iesolver.PDE_STOKES else 1)
+    if real:
+        U, Psi = oracle.OracleProblem(g, pde).U_Psi()
+    else:
+        U = rng.standard_normal((s.ndof, hd)) / np.sqrt(s.ndof)
+        Psi = rng.standard_normal((hd, s.ndof)) / np.sqrt(s.ndof)
+        s.set_border(U, Psi)
+    s.factor(TOL)
+    print("root", s.box_info()["n_active"][0], "border", hd, flush=True)
+    f = rng.standard_normal(s.ndof)
+    mu, alpha = s.solve(f)
+    K = oracle.dense_matrix(g, pde)
+    r1, r2 = K @ mu + U @ alpha - f, Psi @ mu - alpha
+    # the backward error bar of every form (ie_solver_test.cpp:84-95)
+    assert np.sqrt(np.sum(r1 ** 2) + np.sum(r2 ** 2)) <= 50 * TOL * np.linalg.norm(f)
+    y, z = s.apply(mu, alpha)  # the operator's own border products
+    bound = 1e-12 * (np.abs(K) @ np.abs(mu) + np.abs(U) @ np.abs(alpha)).max()
+    assert np.abs(y - (r1 + f)).max() <= bound
+    assert np.abs(z - r2).max() <= 1e-12 * (np.abs(Psi) @ np.abs(mu) + np.abs(alpha)).max()

@@ -73,3 +73,18 @@ def test_unrefined_error_is_no_larger_than_the_qr_form():
     gm = float(np.exp(np.mean(np.log(ratio))))
     print(f"FP32 / FP64 backward error: mean {gm:.1f}", flush=True)
     assert gm <= 23.7
+
+
+def test_gram_takes_over_at_its_limit():
+    """Below 5e-7 the FP32 QR's ranks, from there on the Gram form's: the two
+    tolerances lie 2 % apart, the forms' ranks on the deepest level about 3 %
+    of all of them."""
+    g = G.star(30000, k=5)
+    i = [_factored(g, iesolver.PDE_LAPLACE, 64, t, iesolver.FP32).box_info()
+         for t in (4.9e-7, 5e-7)]
+    deep = (i[0]["level"] >= i[0]["level"].max() - 1) & (i[0]["is_leaf"] == 1) & (i[0]["rank"] > 0)
+    assert deep.sum() > 100
+    a, b = (x["rank"][deep].sum() for x in i)
+    print(f"leaf ranks below the limit {a}, at it {b}", flush=True)
+    # a larger tolerance cannot add ranks within one form
+    assert b > a

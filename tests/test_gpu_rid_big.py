@@ -75,3 +75,40 @@ def test_learned_form_is_as_close_as_the_full_qr():
     gm = float(np.exp(np.mean(np.log(ratio))))
     print(f"learned / plain error: mean {gm:.2f}, largest {max(ratio):.2f}", flush=True)
     assert gm <= 1
+
+
+def _eligible(i, pde):
+    proxy = np.where(i["level"] >= 3, 512 if pde == iesolver.PDE_STOKES else 256, 0)
+    return ((i["level"] > 0) & (i["m_rows"] > 0) & (i["n_active"] <= 256) &
+            ((i["m_rows"] - proxy) // 2 <= 1280))
+
+
+@pytest.mark.parametrize("n,leaf,pde", [
+    (700, 128, iesolver.PDE_STOKES), (1100, 150, iesolver.PDE_STOKES),
+    (1500, 256, iesolver.PDE_STOKES), (3000, 300, iesolver.PDE_LAPLACE_NEUMANN)])
+def test_large_boxes_are_sketched(n, leaf, pde):
+    """Trees whose compressed boxes all lie on levels 1 to 4: every one up to
+    256 columns and 1,280 near DOFs ends with a sketch's ID, those of more
+    than 128 columns or ranks past 58, which only the 128-row sketch gives,
+    among them."""
+    s = _solver(G.star(n, k=5), pde, leaf, True)
+    i = s.box_info()
+    el = _eligible(i, pde)
+    assert i["level"][el].max() <= 4
+    sketched, fallback = s.id_stats()
+    assert fallback == 0 and sketched == el.sum()
+    assert (el & ((i["n_active"] > 128) | (i["rank"] > 58))).sum() >= 4
+    assert (el & (i["n_active"] > 64) & (i["is_leaf"] == 1)).any()
+
+
+@pytest.mark.parametrize("n,leaf,pde", [
+    (1500, 256, iesolver.PDE_STOKES), (3000, 300, iesolver.PDE_LAPLACE_NEUMANN)])
+def test_large_boxes_are_sketched_fp32(n, leaf, pde):
+    """At 1e-6 a few narrow sketches fail; fewer than there are boxes of more
+    than 128 columns, so the 128-row sketch gave some of those their IDs."""
+    s = _solver(G.star(n, k=5), pde, leaf, True, iesolver.FP32, 1e-6)
+    i = s.box_info()
+    el = _eligible(i, pde)
+    sketched, fallback = s.id_stats()
+    assert sketched + fallback == el.sum()
+    assert fallback < (el & (i["n_active"] > 128)).sum()

@@ -551,7 +551,7 @@ void alloc_state(iegpu_ctx* c) {
   }
   c->s_rid_done.alloc(nb);
   c->s_lists.alloc((size_t)kNumLists * nb);
-  c->s_lcnt.alloc((size_t)2 * kMaxLevels * kNumLists);
+  c->s_lcnt.alloc((size_t)kMaxLevels * kNumLists);
   c->s_jobs.alloc((size_t)2 * kMaxChunks * nb);
   c->s_njobs.alloc(kMaxLevels);
   c->s_halt.alloc(kMaxLevels);
@@ -1675,11 +1675,11 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
     }
     if (plan_ok && !c->plan_on && !(errbits & kErrSingular)) {
       // Record the plan from this factorization's per-level list counts.
-      std::vector<int> lc((size_t)2 * kMaxLevels * kNumLists);
+      std::vector<int> lc((size_t)kMaxLevels * kNumLists);
       HIP_TRY(hipMemcpy(lc.data(), c->s_lcnt.p, sizeof(int) * lc.size(), hipMemcpyDeviceToHost));
       c->plan_skip.assign(kMaxLevels, 0);
       for (int lv = 1; lv < c->tree.n_levels; lv++) {
-        auto cnt = [&](int L) { return lc[(size_t)2 * (lv * kNumLists + L)]; };
+        auto cnt = [&](int L) { return lc[(size_t)lv * kNumLists + L]; };
         const int reg = c->rid_mode != 0 ? cnt(kLstFallback) : cnt(kLstReg) + cnt(kLstRegHalf);
         int m = 0;
         if (cnt(kLstLds) == 0) m |= kSkipAssemble;

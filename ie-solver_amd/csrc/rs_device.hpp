@@ -195,7 +195,7 @@ struct DevState {
   int* qkind;          // ID route of the box (QrcpKind)
   int nbox;            // box slots
   int* lists;          // kNumLists x nbox: a level's list L starts at its first slot
-  int* lcnt;           // kMaxLevels x kNumLists x 2: list lengths (second word spare)
+  int* lcnt;           // kMaxLevels x kNumLists: list lengths
   int* jobs;           // (box, chunk) row-compression jobs, kMaxChunks per box slot
   int* njobs;          // per level: number of row-compression jobs
   int64_t* id_sz;      // scratch doubles/floats needed (per box, level-local)
@@ -274,7 +274,7 @@ __device__ inline bool box_clean(const DevState& s, int b) {
 }
 
 __device__ inline int* list_slot(const DevState& s, int level, int L) {
-  return s.lcnt + 2 * (level * kNumLists + L);
+  return s.lcnt + (level * kNumLists + L);
 }
 // Row-compression jobs (chunks) of box b.
 __device__ inline int row_jobs(const DevState& s, int b) {

@@ -1,5 +1,6 @@
 // Device helpers shared by the interpolative-decomposition kernels
-// (rs_kernels.hip, rs_rid_big.hip): ID rows, Householder scalars, MFMA tiles.
+// (rs_kernels.hip, rs_qrcp.hip, rs_rid.hip, rs_rid_big.hip, rs_gram.hip): ID
+// rows, Householder scalars, MFMA tiles, sketches.
 #pragma once
 
 #include <hip/hip_runtime.h>

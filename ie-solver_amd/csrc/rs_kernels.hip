@@ -42,7 +42,7 @@ __global__ void k_reset(DevState s) {
     if (!s.dirty) *s.fac_top = 0;
   }
   if (threadIdx.x < kMaxLevels) s.njobs[threadIdx.x] = 0;
-  for (int i = threadIdx.x; i < 2 * kMaxLevels * kNumLists; i += blockDim.x) s.lcnt[i] = 0;
+  for (int i = threadIdx.x; i < kMaxLevels * kNumLists; i += blockDim.x) s.lcnt[i] = 0;
 }
 
 // active(box) = concatenation of the children's outgoing lists (skeleton if

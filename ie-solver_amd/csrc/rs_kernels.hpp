@@ -1,4 +1,4 @@
-// Launch wrappers for the RS factor + solve kernels (rs_kernels.hip).
+// Launch wrappers for the RS factor + solve kernels.
 #pragma once
 
 #include <hip/hip_runtime.h>

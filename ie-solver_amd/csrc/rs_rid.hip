@@ -32,8 +32,8 @@ namespace {
 
 // One workgroup (4 waves) per box.  The box's row geometry (near DOFs,
 // then the proxy circle) is staged in LDS; wave w sketches the 16-column
-// tile w (n <= 64) segment by segment (near target rows, near source rows,
-// proxy target rows, proxy source rows).  The tiles of Y go to LDS, and
+// tile w (n <= 64) over the near DOFs, then the proxy circle, both directions
+// of an entry at once (sketch_pairs).  The tiles of Y go to LDS, and
 // wave 0 alone runs the pivoted QR of Y, the other waves ending there.
 // QR layout: lane c holds column c's active rows, shifted so that the
 // step's row is always register 0; row j of R leaves the registers for
@@ -230,22 +230,22 @@ __global__ __launch_bounds__(256, 5) void k_rid(DevGeom g, DevTree t, DevState s
   }
 }
 
-// Wide randomized ID (a box below the top levels takes it only past 64
-// columns: k_qrcp took 2.0 to 3.4 ms for a level of 70 to 100 such boxes of
-// 65 to 87 Stokes DOFs, whose stacked triangles do not fit the register
-// QRCP; this form 230 us): the boxes too large for k_rid (up
-// to kRidMaxNearW row DOFs and kRidWideCols columns, ranks up to kRidRowsW
-// - kRidOver).  Same sketch, rank rule and outputs as k_rid with a sketch
-// of kRidRowsW rows from its own table, on 8 waves: wave w sketches the
-// 16-column tile w % (4 QW) over every (8 / 4 QW)-th 16-row block, the
-// row parts added in a fixed order.  QW waves then run the pivoted QR,
-// wave q holding columns 64 q + lane: QW = 1 for n <= 64 (one wave, no
-// barrier), QW = 2 for n <= 128 (each step's pivot found from both waves'
-// maxima through LDS, the pivot column's Householder vector published by
-// its wave; two barriers per step).  A box whose sketch shows no cut keeps
-// rid_done = 0: a register-QRCP box joins the fallback list, any other is
-// still on its full-QRCP list (whose kernels skip the boxes the sketch
-// took).
+// Wide randomized ID: the boxes too large for k_rid, by columns or by near
+// DOFs, and on the top levels those whose predicted rank passes its widest
+// sketch (up to kRidMaxNearW near DOFs and kRidWideCols columns, ranks up to
+// kRidRowsW - kRidOver).  With the rank model on every level: k_qrcp took 2.0
+// to 3.4 ms for a level of 70 to 100 boxes of 65 to 87 Stokes DOFs, whose
+// stacked triangles do not fit the register QRCP, this form 230 us.  Same
+// sketch and outputs as k_rid with kRidRowsW rows from its own table, on 8
+// waves: wave w sketches the 16-column tile w % (4 QW) over every (8 / 4
+// QW)-th 16-row block, the row parts added in a fixed order.  QW waves then
+// run the pivoted QR, wave q holding columns 64 q + lane: QW = 1 for n <= 64
+// (one wave, no barrier), QW = 2 for n <= 128 (each wave publishes its best
+// column's Householder vector and key, both read the winner's; one barrier
+// per step).  A box whose sketch shows no cut goes on to the 128-row sketch
+// on the top levels; below them a register-QRCP box joins the fallback list
+// and any other is still on its full-QRCP list (whose kernels skip the boxes
+// a sketch took).
 constexpr int kRidWideWaves = 8;
 
 // LDS of the wide sketch: the row table, then Y, then the rows of R (a

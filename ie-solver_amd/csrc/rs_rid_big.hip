@@ -1,7 +1,7 @@
 // Randomized interpolative decomposition with a 128-row sketch: the large
 // boxes of the top tree levels (up to kRidBigCols columns, ranks up to
-// kRidRowsB - kRidOver), which the 16- to 64-row sketches of rs_kernels.hip
-// cannot take.  Same sketch, rank rule and outputs as there.
+// kRidRowsB - kRidOver), which the 16- to 64-row sketches of rs_rid.hip
+// cannot take.  Same sketch and outputs as there.
 
 #include <hip/hip_runtime.h>
 

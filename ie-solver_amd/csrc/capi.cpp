@@ -26,6 +26,10 @@ using namespace iegpu;
 static_assert(IEGPU_RANK_FEATURES == kFeat && IEGPU_RANK_MODEL_LEN == kMlpLen &&
                   IEGPU_RANK_PARAMS == kMlpParams,
               "rank model layout of iegpu.h");
+// Entries of the 32-, 64- and 128-row sketches' Gaussian tables.
+constexpr int64_t kOmega = (int64_t)kRidTableRows * kRidRows;
+constexpr int64_t kOmegaW = (int64_t)kRidTableRowsW * kRidRowsW;
+constexpr int64_t kOmegaB = (int64_t)kRidTableRowsW * kRidRowsB;
 static_assert(kRootPiv == kInvFlags, "panel flags behind a root's pivot rows");
 static_assert(IEGPU_NUM_LAUNCH_CAPS == kNumCaps, "launch caps of iegpu.h");
 
@@ -244,7 +248,7 @@ struct iegpu_ctx {
   // randomized ID
   int rid_mode = 0, rid_width = 0;
   int gram = 0;  // of the factorization being enqueued
-  DevBuf<double> d_omega, d_omega_w, d_omega_b;
+  DevBuf<double> d_omega;  // the sketches' three Gaussian tables (kOmega*)
   // factorization replayed as a captured HIP graph (iegpu_set_graphs)
   bool use_graphs = false;
   hipGraphExec_t fgraph = nullptr;
@@ -417,8 +421,8 @@ struct iegpu_ctx {
     s.sk_w = s_sk_w.p;
     s.rid_done = s_rid_done.p;
     s.omega = d_omega.p;
-    s.omega_w = d_omega_w.p;
-    s.omega_b = d_omega_b.p;
+    s.omega_w = d_omega.p ? d_omega.p + kOmega : nullptr;
+    s.omega_b = d_omega.p ? d_omega.p + kOmega + kOmegaW : nullptr;
     s.rank_model = d_model.p;
     s.rid_margin = rid_margin;
     s.feat = record_features ? d_feat.p : nullptr;
@@ -1521,15 +1525,11 @@ int factor_impl(iegpu_ctx* c, double id_tol, int precision, const double* fb, do
     if (c->fac_cap == 0) c->fac_cap = std::max<int64_t>(nd * 160, 1 << 22);
     if (c->dec_cap == 0) c->dec_cap = std::max<int64_t>(nd * 8, 1 << 20);
     if (c->rid_mode != 0 && !c->d_omega.p) {
-      const int64_t no = (int64_t)kRidTableRows * kRidRows;
-      c->d_omega.alloc(no);
-      launch_gaussian(c->d_omega.p, no, 0x5EEDull, c->stream);
-      const int64_t nw = (int64_t)kRidTableRowsW * kRidRowsW;
-      c->d_omega_w.alloc(nw);
-      launch_gaussian(c->d_omega_w.p, nw, 0x5EEDull, c->stream);
-      const int64_t nb = (int64_t)kRidTableRowsW * kRidRowsB;
-      c->d_omega_b.alloc(nb);
-      launch_gaussian(c->d_omega_b.p, nb, 0x5EEDull, c->stream);
+      // one allocation (65 us for the largest table alone)
+      c->d_omega.alloc(kOmega + kOmegaW + kOmegaB);
+      launch_gaussian(c->d_omega.p, kOmega, 0x5EEDull, c->stream);
+      launch_gaussian(c->d_omega.p + kOmega, kOmegaW, 0x5EEDull, c->stream);
+      launch_gaussian(c->d_omega.p + kOmega + kOmegaW, kOmegaB, 0x5EEDull, c->stream);
     }
     // After iegpu_update_geometry on the same tree, only the marked boxes
     // are re-factored (same tolerance and precision as the kept factors).

@@ -33,8 +33,8 @@ namespace {
 // k_gram_blocks / k_gram_chol: 65 to 256 columns, a workgroup per 32 x 32
 // block of G, then one per box.
 // Entry evaluation and its MFMAs bound k_gram_id, the latency of the steps
-// k_gram_chol.  Stokes with 8 holes, 131,072 points, plain FP32 at 1e-6: 4.2
-// ms per factorization (k_gram_id 2.5, k_gram_blocks 0.15, k_gram_chol 1.5)
+// k_gram_chol.  Stokes with 8 holes, 131,072 points, plain FP32 at 1e-6: 4.3
+// ms per factorization (k_gram_id 2.5, k_gram_blocks 0.14, k_gram_chol 1.6)
 // against 25.1 for row compression, register and general QR and assembly.
 // ---------------------------------------------------------------------------
 
